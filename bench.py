@@ -320,7 +320,8 @@ def bench_single(args, w, wname):
                                                    evals)
     fp64_ms = rel = rel_exact = kt_cmp = None
     if args.fp64_steps > 0:
-        fp64_ms = timed(lambda: E.voigt(st, grid, 0.0, E.HK_VOIGT_FP64, K=K, workspace=ws),
+        fp64_ms = timed(lambda: E.voigt(st, grid, 0.0, E.HK_VOIGT_FP64, K=K, workspace=ws,
+                                        exact_pairs=True),
                         args.fp64_steps)
         log("bench: %s FP64 Voigt %.3f ms" % (wname, fp64_ms))
         tau = 1e-12 * float(K.max())
@@ -562,7 +563,8 @@ def bench_batched(args, w, wname):
     res = {"fp64": None}
     rel = rel_exact = kt_cmp = None
     if args.fp64_steps > 0:
-        b64 = E.VoigtBatch(items, mode=E.HK_VOIGT_FP64, tile_points=tile, stage_lines=stage)
+        b64 = E.VoigtBatch(items, mode=E.HK_VOIGT_FP64, tile_points=tile, stage_lines=stage,
+                           exact_pairs=True)      # plain FP64: every pair evaluated
         g_64, _ = capture(b64.launch)
         res["fp64"] = replay_ms(g_64, args.fp64_steps)
         log("bench: FP64 batched Voigt %.1f ms per replay" % res["fp64"])

@@ -8,9 +8,9 @@
 //     centres, the lines whose cut window can reach the tile, and (FP32
 //     form) a power-of-two strength scale for the tile;
 //   * each workgroup stages 256 lines at a time through LDS; every thread
-//     owns W/256 grid points and keeps their sums in registers (the FP64
-//     form adds the lines in index order, the FP32 form path by path within
-//     a stage) -- no atomics, bit-identical reruns;
+//     owns W/256 grid points and keeps their sums in registers, added in a
+//     fixed order -- no atomics, bit-identical reruns (the FP64 form's tiles
+//     are described in hk_voigt64.h);
 //   * a line contributes to point j iff |x_j - nu| < hw in FP64 (the
 //     integer window is computed once per line and tile, cut_window).
 //
@@ -28,7 +28,8 @@
 // Forms:
 //   HK_VOIGT_FP64  x = (x_j - nu)/alpha_D in FP64, FP64 profile (Algorithm
 //                  916 core, 8- and 4-node Gauss-Hermite, 3-term asymptotic)
-//                  and FP64 accumulation.
+//                  and FP64 accumulation; lines far from a tile through 20
+//                  Chebyshev nodes, exact to FP64 rounding (hk_voigt64.h).
 //   HK_VOIGT_FP32C the line offset is formed in FP64 once per line and tile
 //                  (nearest grid point jc, remainder r), then
 //                  x = (j - jc) vb + r in FP32 with vb split hi+lo; FP32
@@ -52,10 +53,10 @@
 #include "hk_device.h"
 #include "hk_internal.h"
 #include "hk_tiles.h"
+#include "hk_voigt64.h"
 
 namespace hk {
 
-constexpr int kThreads = 256;
 constexpr int kStage = 256;          // lines per LDS stage (one per thread)
 
 struct VArgs {
@@ -74,11 +75,6 @@ struct VArgs {
 // LDS record of one line for one tile.  lo/hi: the line's cut window
 // (tile-relative); code: 4 bits per wave, the evaluation path that wave takes
 // for this line (wave_code), decided once when the record is built.
-struct Rec64 {
-    double nu, ia, y2, B, G, p2, p3, p4;
-    int32_t lo, hi, code, pad;
-};
-
 // FP32 record, grouped by the path that reads it: x and r2; the asymptotic
 // series of the wings with the strength folded into the coefficients
 // (far: B, 1.5 B, BC; mid: q2..q6, see far4_32); the 8-node rule and the
@@ -222,133 +218,6 @@ __device__ __forceinline__ float core_q1_32(float y) {
     return s;
 }
 
-
-// ---------------------------------------------------------------------------
-// FP64 form.  Wave w owns the contiguous points [w*64*PPT, (w+1)*64*PPT) of
-// the tile; lane l holds points w*64*PPT + 64k + l.  FULL: the line's cut
-// window covers the wave's points, so no per-point mask.
-// ---------------------------------------------------------------------------
-template <int PATH, bool FULL, int PPT>
-__device__ __forceinline__ void eval64(const Rec64 &qr, const double *xj, double *acc, int jr0) {
-    const double nu = qr.nu, ia = qr.ia, y2 = qr.y2, B = qr.B, G = qr.G;
-    const double p2 = qr.p2, p3 = qr.p3, p4 = qr.p4;
-    const int32_t lo = qr.lo, hi = qr.hi;
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        const double x = (xj[k] - nu) * ia;
-        const double r2 = fma(x, x, y2);
-        double v;
-        if (PATH == kPathFar) {
-            const double inv = rcp64(r2);
-            v = B * inv * fma(fma(fma(fma(p4, inv, p3), inv, p2), inv, 1.5), inv, 1.0);
-        } else if (PATH == kPathMid) {
-            v = G * gh4_sum64(x * x, r2);
-        } else if (PATH == kPathMid2) {
-            v = G * gh8_sum64(x * x, r2);
-        } else {
-            if (r2 >= kRF64) {
-                const double inv = rcp64(r2);
-                v = B * inv * fma(fma(fma(fma(p4, inv, p3), inv, p2), inv, 1.5), inv, 1.0);
-            } else if (r2 >= kRM64) {
-                v = G * gh4_sum64(x * x, r2);
-            } else if (r2 >= kRB64) {
-                v = G * gh8_sum64(x * x, r2);
-            } else {
-                v = 0.0;            // line core: added by the line-core pass
-            }
-        }
-        if (!FULL) {
-            const int jr = jr0 + 64 * k;
-            v = (jr >= lo && jr < hi) ? v : 0.0;
-        }
-        acc[k] += v;
-    }
-}
-
-template <int PPT>
-__device__ __forceinline__ void dispatch64(const Rec64 &q, int code, const double *xj, double *acc,
-                                           int jr0) {
-    switch (code) {
-        case 1: eval64<kPathFar, true, PPT>(q, xj, acc, jr0); break;
-        case 2: eval64<kPathFar, false, PPT>(q, xj, acc, jr0); break;
-        case 3: eval64<kPathMid, true, PPT>(q, xj, acc, jr0); break;
-        case 4: eval64<kPathMid, false, PPT>(q, xj, acc, jr0); break;
-        case 5: eval64<kPathMid2, true, PPT>(q, xj, acc, jr0); break;
-        case 6: eval64<kPathMid2, false, PPT>(q, xj, acc, jr0); break;
-        case 7: eval64<kPathAny, true, PPT>(q, xj, acc, jr0); break;
-        default: eval64<kPathAny, false, PPT>(q, xj, acc, jr0); break;
-    }
-}
-
-// LM: stages of kThreads * LM lines (each thread stages LM lines per stage);
-// results do not depend on it (lines are added in index order either way).
-template <int PPT, int LM>
-__device__ __forceinline__ void tile_f64(const VArgs &a, int64_t tile, Rec64 *rec) {
-    constexpr int W = kThreads * PPT;
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wlo = wave * 64 * PPT;
-    const int jr0 = wlo + lane;
-    const TileInfo ti = a.tiles[tile];
-    const int64_t j0 = tile * W;
-    double xj[PPT], acc[PPT];
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        xj[k] = fma((double)(j0 + jr0 + 64 * k), a.dnu, a.numin);
-        acc[k] = 0.0;
-    }
-    for (int64_t base = ti.lo; base < ti.hi; base += kThreads * LM) {
-#pragma unroll 1
-        for (int q = 0; q < LM; ++q) {
-            const int64_t i = base + q * kThreads + t;
-            Rec64 r;
-            r.lo = 0; r.hi = 0; r.code = 0;
-            if (i < ti.hi) {
-                const double nu = a.nu[i];
-                int64_t wl, wh;
-                cut_window(nu, a.hw[i], a.numin, a.dnu, a.nx, wl, wh);
-                const int64_t clo = max(wl, j0), chi = min(wh, j0 + W);
-                if (clo < chi) {
-                    const double ia = a.ia[i], y = a.y[i], y2 = y * y;
-                    const double A = a.S[i] * kISqrtPi;
-                    r.nu = nu; r.ia = ia; r.y2 = y2;
-                    r.B = A * y * kISqrtPi; r.G = A * y * (2.0 / kPi);
-                    r.p2 = 3.75 - 2.0 * y2; r.p3 = -15.0 * y2; r.p4 = 12.0 * y2 * y2;
-                    r.lo = (int32_t)(clo - j0); r.hi = (int32_t)(chi - j0);
-                    const double jcd = rint((nu - a.numin) / a.dnu);
-                    const double rr = (fma(jcd, a.dnu, a.numin) - nu) * ia;
-                    const double vb = a.dnu * ia, d0 = (double)j0 - jcd;
-                    int32_t ri[6];
-                    region_interval(kRF64, y2, rr, vb, d0, W, ri[0], ri[1]);
-                    region_interval(kRM64, y2, rr, vb, d0, W, ri[2], ri[3]);
-                    region_interval(kRB64, y2, rr, vb, d0, W, ri[4], ri[5]);
-                    r.code = wave_codes<64 * PPT>(r.lo, r.hi, ri, [](int) { return 0.0; }, 1.0, 1.0);
-                }
-            }
-            // the previous stage's readers of rec[] must be done before it is
-            // written (the first record is built while they finish)
-            if (q == 0) __syncthreads();
-            rec[q * kThreads + t] = r;
-        }
-        __syncthreads();
-        const int nst = (int)min((int64_t)kThreads * LM, ti.hi - base);
-        for (int c0 = 0; c0 < nst; c0 += 64) {
-            const int nib = c0 + lane < nst ? (rec[c0 + lane].code >> (4 * wave)) & 15 : 0;
-            unsigned long long m = __ballot(nib != 0);       // 0: window misses this wave
-            while (m) {
-                const int b = lowest_bit(m);
-                const int code = __builtin_amdgcn_readlane(nib, b);
-                dispatch64<PPT>(rec[c0 + b], code, xj, acc, jr0);
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        const int64_t j = j0 + jr0 + 64 * k;
-        if (j < a.nx) a.K[j] = a.accumulate ? a.K[j] + acc[k] : a.kmin + acc[k];
-    }
-}
 
 // ---------------------------------------------------------------------------
 // FP32 compensated form (same point ownership as the FP64 form)
@@ -552,7 +421,6 @@ __device__ __forceinline__ double far_u(int k) {
 // to the targets (the waves whose points it covers) in the target columns
 // (xhi, xlo).  Totals and coefficients are per target wave: each wave
 // interpolates its own sums at its own points.
-constexpr int kWaves = kThreads / 64;
 template <int N>
 struct FarBand {
     float hi[N][kWaves];              // common node sums, one column per wave
@@ -1556,8 +1424,8 @@ template <int MODE, int PPT, int LM>
 __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_kernel(VArgs a) {
     const int64_t tile = blockIdx.x;
     if (MODE == HK_VOIGT_FP64) {
-        __shared__ Rec64 rec[kThreads * LM];
-        tile_f64<PPT, LM>(a, tile, rec);
+        __shared__ Far64LDS sh;
+        tile_f64<PPT>(a, tile, &sh);
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
@@ -1601,13 +1469,13 @@ __global__ __launch_bounds__(256, PPT == 0 ? (MODE == HK_VOIGT_FP32C ? 5 : 1) : 
 void voigt_persistent_kernel(const VArgs *__restrict__ specs,
                                                                const int64_t *__restrict__ item_start,
                                                                int nspec, unsigned long long *counter) {
-    constexpr size_t kRecBytes =
-        PPT == 0 ? (MODE == HK_VOIGT_FP64 ? sizeof(Core64) : sizeof(Core32))
-                 : (MODE == HK_VOIGT_FP64 ? sizeof(Rec64) : sizeof(Rec32));
+    constexpr size_t kBytes =
+        MODE == HK_VOIGT_FP64 ? (PPT == 0 ? sizeof(Core64) * kThreads : sizeof(Far64LDS))
+                              : (PPT == 0 ? sizeof(Core32) : sizeof(Rec32)) * kThreads * LM;
     __shared__ int64_t s_item;
     __shared__ int cnt[kThreads / 64];
     __shared__ float dtab[(PPT == 0 && MODE == HK_VOIGT_FP32C) ? kStage * kDT : 1];
-    __shared__ __attribute__((aligned(16))) char smem[kRecBytes * kThreads * LM];
+    __shared__ __attribute__((aligned(16))) char smem[kBytes];
     __shared__ FarLDS fl[1];
     const int64_t total = item_start[nspec];
     for (;;) {
@@ -1628,7 +1496,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
             if constexpr (MODE == HK_VOIGT_FP64) core_f64(a, tile, (Core64 *)smem, cnt);
             else core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
-            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LM>(a, tile, (Rec64 *)smem);
+            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
         }
     }
@@ -1834,7 +1702,7 @@ void launch_tiles_lm(int ppt, int64_t ntiles, hipStream_t s, const VArgs &a) {
 
 template <int MODE>
 void launch_tiles(int ppt, int lm, int64_t ntiles, hipStream_t s, const VArgs &a) {
-    if (lm == 2) launch_tiles_lm<MODE, 2>(ppt, ntiles, s, a);
+    if (MODE == HK_VOIGT_FP32C && lm == 2) launch_tiles_lm<HK_VOIGT_FP32C, 2>(ppt, ntiles, s, a);
     else launch_tiles_lm<MODE, 1>(ppt, ntiles, s, a);
 }
 
@@ -1857,8 +1725,8 @@ void launch_persistent(int ppt, int lm, unsigned grid, hipStream_t s, const VArg
     if (ppt == 0)
         hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 0, 1>), dim3(grid), dim3(kThreads), 0, s,
                            specs, item_start, nspec, counter);
-    else if (lm == 2)
-        launch_persistent_lm<MODE, 2>(ppt, grid, s, specs, item_start, nspec, counter);
+    else if (MODE == HK_VOIGT_FP32C && lm == 2)
+        launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, grid, s, specs, item_start, nspec, counter);
     else
         launch_persistent_lm<MODE, 1>(ppt, grid, s, specs, item_start, nspec, counter);
 }
@@ -1914,10 +1782,12 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     TileInfo *ctiles = (TileInfo *)((char *)tiles + align_up((size_t)ncore * sizeof(TileInfo), 256));
     const int scale = mode == HK_VOIGT_FP32C ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s,
-                       st->key, st->nlines, st->radius, st->blk_max, grid->numin, grid->dnu,
-                       grid->nx, W, ntiles, scale, tiles);
-    HK_LAUNCH_CHECK();
+    if (mode == HK_VOIGT_FP32C) {           // (the FP64 tiles search their ranges themselves)
+        hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s,
+                           st->key, st->nlines, st->radius, st->blk_max, grid->numin, grid->dnu,
+                           grid->nx, W, ntiles, scale, tiles);
+        HK_LAUNCH_CHECK();
+    }
     hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ncore + 3) / 4)), dim3(256), 0, s,
                        st->key, st->nlines, st->radius + 1, st->blk_max, grid->numin, grid->dnu,
                        grid->nx, kCoreW, ncore, scale, ctiles);
@@ -1927,7 +1797,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     a.key = st->key; a.blk_max = st->blk_max; a.radius = st->radius; a.nl = st->nlines;
     a.tiles = tiles; a.numin = grid->numin; a.dnu = grid->dnu; a.nx = grid->nx;
     a.kmin = kmin; a.accumulate = accumulate; a.K = K;
-    a.far = (mode == HK_VOIGT_FP32C && !(tune && tune->exact_pairs)) ? 1 : 0;
+    a.far = tune && tune->exact_pairs ? 0 : 1;
     if (mode == HK_VOIGT_FP64) launch_tiles<HK_VOIGT_FP64>(ppt, lm, ntiles, s, a);
     else launch_tiles<HK_VOIGT_FP32C>(ppt, lm, ntiles, s, a);
     HK_LAUNCH_CHECK();
@@ -2086,7 +1956,7 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
         a.tiles = (TileInfo *)(base + L.tile_off[i]);
         a.numin = sp.grid.numin; a.dnu = sp.grid.dnu; a.nx = sp.grid.nx;
         a.kmin = sp.kmin; a.accumulate = sp.accumulate; a.K = sp.K;
-        a.far = (mode == HK_VOIGT_FP32C && !(tune && tune->exact_pairs)) ? 1 : 0;
+        a.far = tune && tune->exact_pairs ? 0 : 1;
         cargs[q] = a;
         cargs[q].radius = sp.st.radius + 1;
         cargs[q].tiles = (TileInfo *)(base + L.ctile_off[i]);
@@ -2137,9 +2007,11 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counter);
     HK_LAUNCH_CHECK();
     if (batch->items_main > 0) {
-        hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_main + 3) / 4)),
-                           dim3(256), 0, s, args, items, nspec, batch->tile_points, scale);
-        HK_LAUNCH_CHECK();
+        if (batch->mode == HK_VOIGT_FP32C) {
+            hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_main + 3) / 4)),
+                               dim3(256), 0, s, args, items, nspec, batch->tile_points, scale);
+            HK_LAUNCH_CHECK();
+        }
         hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_core + 3) / 4)),
                            dim3(256), 0, s, cargs, citems, nspec, kCoreW, scale);
         HK_LAUNCH_CHECK();

@@ -55,7 +55,8 @@ enum {
 
 /* Voigt evaluation forms. */
 enum {
-    HK_VOIGT_FP64 = 0,          /* plain FP64 profile, FP64 accumulation */
+    HK_VOIGT_FP64 = 0,          /* FP64 profile and sums; lines far from a
+                                   tile interpolated to FP64 rounding */
     HK_VOIGT_FP32C = 1,         /* FP32 profile, compensated FP32 tile sums */
     HK_VOIGT_COMPAT = 2         /* the reference's own FP32 region formulas
                                    (Line6fA/B/C_kernel, voigt.h:1177-1706:
@@ -143,10 +144,10 @@ typedef struct {
 typedef struct {
     int tile_points;    /* grid points per workgroup tile: 512, 1024
                            (default), 2048 or 4096 */
-    int exact_pairs;    /* HK_VOIGT_FP32C: 1 evaluates every (line, point)
-                           pair; 0 (default) sums lines far from a tile,
-                           or from a wave's quarter of it, through
-                           Chebyshev far fields */
+    int exact_pairs;    /* 1 evaluates every (line, point) pair; 0
+                           (default) sums lines far from a tile, or from a
+                           wave's quarter of it, through Chebyshev far
+                           fields (HK_VOIGT_FP64: to FP64 rounding) */
     int stage_lines;    /* lines staged through LDS per step of the main
                            pass: 256 (default) or 512 (the reference's fixed
                            line blocks def_nlA/B/C, define.h:56-58); FP64
@@ -185,7 +186,7 @@ int hk_line_params(const hk_lines *lines, const hk_tp *tp, const hk_cut *cut,
 /* Voigt sum onto the grid: K_j = kmin + sum_i S_i Re w(x_ij, y_i)/sqrt(pi)
  * (accumulate == 0) or K_j += sum (accumulate != 0), over the lines whose
  * cut window holds j: |x_j - nu_i| < hw_i in FP64.  Deterministic: each
- * point is owned by one thread that adds the lines in index order.
+ * point is owned by one thread, and every sum is taken in a fixed order.
  * HK_VOIGT_COMPAT instead evaluates each pair as the reference's FP32
  * kernels do (x = va + j vb in float, kept when x^2 < vcut2, region formulas
  * of Line6fA/B/C_kernel, S3_kernel's FP32 line constants) and adds the
@@ -221,8 +222,9 @@ int hk_voigt_accumulate_noalloc(const hk_line_state *st, const hk_grid *grid,
 int hk_voigt_pair_count(const hk_line_state *st, const hk_grid *grid,
                         unsigned long long *counts, hk_stream_t stream);
 
-/* Work actually done by one hk_voigt_accumulate call with this mode and
- * tuning (tile width set by tile_points): counts (12 device uint64) =
+/* Work actually done by one HK_VOIGT_FP32C hk_voigt_accumulate call with
+ * this tuning (tile width set by tile_points; for HK_VOIGT_FP64 the pairs of
+ * the windows, however they are summed): counts (12 device uint64) =
  * [direct pairs in regions A, B, C (as hk_voigt_pair_count), pairs summed
  * through the FP32 far fields, far (line, tile) pairs of band 1 -- each 9
  * node evaluations --, of band 2 -- 15 each --, of band 3 -- 19 each --,
