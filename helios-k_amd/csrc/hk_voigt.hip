@@ -14,7 +14,8 @@
 //   * a line contributes to point j iff |x_j - nu| < hw in FP64 (the
 //     integer window is computed once per line and tile, cut_window).
 //
-// Two passes per spectrum, in stream order:
+// The FP64 form takes one pass (hk_voigt64.h).  The FP32C form takes two, in
+// stream order:
 //   * the main pass above evaluates every (line, point) pair of the cut
 //     windows except the line cores, x^2 + y^2 < R_core, which it skips;
 //   * the line-core pass (voigt_core_kernel) adds the core pairs: tiles of
@@ -26,9 +27,9 @@
 //   footprint, and so its occupancy, set by the wing formulas.
 //
 // Forms:
-//   HK_VOIGT_FP64  x = (x_j - nu)/alpha_D in FP64, FP64 profile (Algorithm
-//                  916 core, 8- and 4-node Gauss-Hermite, 3-term asymptotic)
-//                  and FP64 accumulation; lines far from a tile through 20
+//   HK_VOIGT_FP64  x = (x_j - nu)/alpha_D in FP64, FP64 profile (midpoint
+//                  rule with the pole's residue in the core, 8- and 4-node
+//                  Gauss-Hermite, 3-term asymptotic) and FP64 accumulation; lines far from a tile through 20
 //                  Chebyshev nodes, exact to FP64 rounding (hk_voigt64.h).
 //   HK_VOIGT_FP32C the line offset is formed in FP64 once per line and tile
 //                  (nearest grid point jc, remainder r), then
@@ -92,11 +93,6 @@ struct Rec32 {
 
 // Line-core pass records: lo/hi bound the points of the tile that lie both
 // in the line's cut window and in its (conservative) core interval.
-struct Core64 {
-    double nu, ia, y, y2, A, ey, q1;
-    int32_t lo, hi;
-};
-
 struct Core32 {
     float r, vbh, vbl, y, y2, A, ey, q1;
     int32_t lo, hi, d0, pad;
@@ -181,26 +177,6 @@ __device__ __forceinline__ int32_t wave_codes(int32_t lo, int32_t hi, const int3
         code |= (1 + 2 * path + full) << (4 * w);
     }
     return code;
-}
-
-// FP64 per-line core constant q1 = sum_{n=1..13} e^{-a^2n^2} / (a^2 n^2 +
-// y^2), a = kA64, with e^{-a^2 n^2} and a^2 n^2 as literals.
-__device__ __forceinline__ double core_q1_64(double y) {
-    constexpr double c[13] = {0.755683658862919, 0.32610700211508303, 0.08036376573837029,
-                              0.011309424249254312, 0.0009088679210029174, 4.171008895272509e-05,
-                              1.0931040894428156e-06, 1.6359197067600175e-08, 1.3981137635663895e-10,
-                              6.823435648847615e-13, 1.9017076395301824e-15, 3.0266657632272252e-18,
-                              2.7508394197950315e-21};
-    constexpr double an2[13] = {0.2801324310308401, 1.1205297241233605, 2.5211918792775614,
-                                4.482118896493442, 7.003310775771004, 10.084767517110246,
-                                13.726489120511166, 17.928475585973768, 22.690726913498057,
-                                28.013243103084015, 33.89602415473165, 40.33907006844098,
-                                47.34238084421199};
-    const double yy = y * y;
-    double s = 0.0;
-#pragma unroll
-    for (int n = 0; n < 13; ++n) s = fma(c[n], rcp64(an2[n] + yy), s);
-    return s;
 }
 
 // FP32 per-line core constant q1 = sum_{n=1..6} e^{-a^2n^2} / (a^2 n^2 + y^2),
@@ -1207,64 +1183,6 @@ __device__ __forceinline__ void tile_f32c(const VArgs &a, int64_t tile, Rec32 *r
 // ---------------------------------------------------------------------------
 constexpr int kCoreW = 256;
 
-__device__ __forceinline__ void core_f64(const VArgs &a, int64_t tile, Core64 *rec, int *cnt) {
-    constexpr int W = kCoreW;
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wlo = wave * 64, whi = wlo + 64;
-    const int jr = wlo + lane;
-    const TileInfo ti = a.tiles[tile];
-    const int64_t j0 = tile * W;
-    const double xj = fma((double)(j0 + jr), a.dnu, a.numin);
-    double acc = 0.0;
-    bool touched = false;
-    for (int64_t base = ti.lo; base < ti.hi; base += kStage) {
-        const int64_t i = base + t;
-        Core64 r;
-        bool valid = false;
-        if (i < ti.hi) {
-            const double nu = a.nu[i];
-            int64_t wl, wh;
-            cut_window(nu, a.hw[i], a.numin, a.dnu, a.nx, wl, wh);
-            const int64_t clo = max(wl, j0), chi = min(wh, j0 + W);
-            const double y = a.y[i], y2 = y * y;
-            if (clo < chi && y2 < kRB64) {
-                const double ia = a.ia[i];
-                const double jcd = rint((nu - a.numin) / a.dnu);
-                const double rr = (fma(jcd, a.dnu, a.numin) - nu) * ia;
-                int32_t clo3, chi3;
-                region_interval(kRB64, y2, rr, a.dnu * ia, (double)j0 - jcd, W, clo3, chi3);
-                r.lo = max((int32_t)(clo - j0), max(clo3, 0));
-                r.hi = min((int32_t)(chi - j0), min(chi3, W));
-                valid = r.lo < r.hi;
-                if (valid) {
-                    r.nu = nu; r.ia = ia; r.y = y; r.y2 = y2;
-                    r.A = a.S[i] * kISqrtPi;
-                    r.ey = a.ey[i];
-                    r.q1 = core_q1_64(y);
-                }
-            }
-        }
-        // the previous stage's readers of rec[] and cnt[] are done after this
-        __syncthreads();
-        int n;
-        const int slot = compact_slot(valid, cnt, n);
-        if (valid) rec[slot] = r;
-        __syncthreads();
-        for (int l = 0; l < n; ++l) {
-            const Core64 &q = rec[l];
-            if ((q.hi <= wlo) | (q.lo >= whi)) continue;      // one LDS read for both
-            touched = true;
-            const double x = (xj - q.nu) * q.ia;
-            const double r2 = fma(x, x, q.y2);
-            if (jr >= q.lo && jr < q.hi && r2 < kRB64) acc += q.A * rew_core64(x, q.y, q.ey, q.q1);
-        }
-    }
-    const int64_t j = j0 + jr;
-    if (touched && j < a.nx) a.K[j] += acc;
-}
-
 __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *rec, float *dtab,
                                           int *cnt) {
     constexpr int W = kCoreW;
@@ -1433,18 +1351,11 @@ __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_ke
     }
 }
 
-template <int MODE>
 __global__ __launch_bounds__(256) void voigt_core_kernel(VArgs a) {
     __shared__ int cnt[kThreads / 64];
-    const int64_t tile = blockIdx.x;
-    if (MODE == HK_VOIGT_FP64) {
-        __shared__ Core64 rec[kStage];
-        core_f64(a, tile, rec, cnt);
-    } else {
-        __shared__ Core32 rec[kStage];
-        __shared__ float dtab[kStage * kDT];
-        core_f32c(a, tile, rec, dtab, cnt);
-    }
+    __shared__ Core32 rec[kStage];
+    __shared__ float dtab[kStage * kDT];
+    core_f32c(a, blockIdx.x, rec, dtab, cnt);
 }
 
 // Persistent form: workgroups take (spectrum, tile) items from a queue.
@@ -1470,7 +1381,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
                                                                const int64_t *__restrict__ item_start,
                                                                int nspec, unsigned long long *counter) {
     constexpr size_t kBytes =
-        MODE == HK_VOIGT_FP64 ? (PPT == 0 ? sizeof(Core64) * kThreads : sizeof(Far64LDS))
+        MODE == HK_VOIGT_FP64 ? sizeof(Far64LDS)
                               : (PPT == 0 ? sizeof(Core32) : sizeof(Rec32)) * kThreads * LM;
     __shared__ int64_t s_item;
     __shared__ int cnt[kThreads / 64];
@@ -1493,8 +1404,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
         const VArgs a = specs[s];
         const int64_t tile = item - item_start[s];
         if constexpr (PPT == 0) {
-            if constexpr (MODE == HK_VOIGT_FP64) core_f64(a, tile, (Core64 *)smem, cnt);
-            else core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
+            core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
             if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
@@ -1722,8 +1632,8 @@ void launch_persistent_lm(int ppt, unsigned grid, hipStream_t s, const VArgs *sp
 template <int MODE>
 void launch_persistent(int ppt, int lm, unsigned grid, hipStream_t s, const VArgs *specs,
                        const int64_t *item_start, int nspec, unsigned long long *counter) {
-    if (ppt == 0)
-        hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 0, 1>), dim3(grid), dim3(kThreads), 0, s,
+    if (MODE == HK_VOIGT_FP32C && ppt == 0)
+        hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP32C, 0, 1>), dim3(grid), dim3(kThreads), 0, s,
                            specs, item_start, nspec, counter);
     else if (MODE == HK_VOIGT_FP32C && lm == 2)
         launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, grid, s, specs, item_start, nspec, counter);
@@ -1780,34 +1690,30 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     const int64_t ncore = (grid->nx + kCoreW - 1) / kCoreW;
     TileInfo *tiles = (TileInfo *)align_up((size_t)ws, 256);
     TileInfo *ctiles = (TileInfo *)((char *)tiles + align_up((size_t)ncore * sizeof(TileInfo), 256));
-    const int scale = mode == HK_VOIGT_FP32C ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
-    if (mode == HK_VOIGT_FP32C) {           // (the FP64 tiles search their ranges themselves)
-        hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s,
-                           st->key, st->nlines, st->radius, st->blk_max, grid->numin, grid->dnu,
-                           grid->nx, W, ntiles, scale, tiles);
-        HK_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ncore + 3) / 4)), dim3(256), 0, s,
-                       st->key, st->nlines, st->radius + 1, st->blk_max, grid->numin, grid->dnu,
-                       grid->nx, kCoreW, ncore, scale, ctiles);
-    HK_LAUNCH_CHECK();
     VArgs a;
     a.nu = st->nu; a.S = st->S; a.ia = st->ialphaD; a.y = st->y; a.hw = st->hw; a.ey = st->ey;
     a.key = st->key; a.blk_max = st->blk_max; a.radius = st->radius; a.nl = st->nlines;
     a.tiles = tiles; a.numin = grid->numin; a.dnu = grid->dnu; a.nx = grid->nx;
     a.kmin = kmin; a.accumulate = accumulate; a.K = K;
     a.far = tune && tune->exact_pairs ? 0 : 1;
-    if (mode == HK_VOIGT_FP64) launch_tiles<HK_VOIGT_FP64>(ppt, lm, ntiles, s, a);
-    else launch_tiles<HK_VOIGT_FP32C>(ppt, lm, ntiles, s, a);
+    if (mode == HK_VOIGT_FP64) {            // one pass; its tiles search their own line ranges
+        launch_tiles<HK_VOIGT_FP64>(ppt, lm, ntiles, s, a);
+        HK_LAUNCH_CHECK();
+        return HK_OK;
+    }
+    hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s,
+                       st->key, st->nlines, st->radius, st->blk_max, grid->numin, grid->dnu,
+                       grid->nx, W, ntiles, 1, tiles);
+    HK_LAUNCH_CHECK();
+    hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ncore + 3) / 4)), dim3(256), 0, s,
+                       st->key, st->nlines, st->radius + 1, st->blk_max, grid->numin, grid->dnu,
+                       grid->nx, kCoreW, ncore, 1, ctiles);
+    HK_LAUNCH_CHECK();
+    launch_tiles<HK_VOIGT_FP32C>(ppt, lm, ntiles, s, a);
     HK_LAUNCH_CHECK();
     a.tiles = ctiles;
-    if (mode == HK_VOIGT_FP64)
-        hipLaunchKernelGGL(voigt_core_kernel<HK_VOIGT_FP64>, dim3((unsigned)ncore), dim3(kThreads),
-                           0, s, a);
-    else
-        hipLaunchKernelGGL(voigt_core_kernel<HK_VOIGT_FP32C>, dim3((unsigned)ncore), dim3(kThreads),
-                           0, s, a);
+    hipLaunchKernelGGL(voigt_core_kernel, dim3((unsigned)ncore), dim3(kThreads), 0, s, a);
     HK_LAUNCH_CHECK();
     return HK_OK;
 }
@@ -2002,32 +1908,27 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
     const int64_t *citems = (const int64_t *)(base + batch->off_citems);
     unsigned long long *counter = (unsigned long long *)(base + batch->off_counter);
     const int nspec = batch->nspec;
-    const int scale = batch->mode == HK_VOIGT_FP32C ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counter);
     HK_LAUNCH_CHECK();
-    if (batch->items_main > 0) {
-        if (batch->mode == HK_VOIGT_FP32C) {
-            hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_main + 3) / 4)),
-                               dim3(256), 0, s, args, items, nspec, batch->tile_points, scale);
-            HK_LAUNCH_CHECK();
-        }
-        hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_core + 3) / 4)),
-                           dim3(256), 0, s, cargs, citems, nspec, kCoreW, scale);
+    if (batch->items_main <= 0) return HK_OK;
+    const unsigned gm = persistent_grid(batch->items_main);
+    if (batch->mode == HK_VOIGT_FP64) {
+        launch_persistent<HK_VOIGT_FP64>(ppt, lm, gm, s, args, items, nspec, counter);
         HK_LAUNCH_CHECK();
-        const unsigned gm = persistent_grid(batch->items_main);
-        const unsigned gc = persistent_grid(batch->items_core);
-        if (batch->mode == HK_VOIGT_FP64) {
-            launch_persistent<HK_VOIGT_FP64>(ppt, lm, gm, s, args, items, nspec, counter);
-            HK_LAUNCH_CHECK();
-            launch_persistent<HK_VOIGT_FP64>(0, 1, gc, s, cargs, citems, nspec, counter + 1);
-        } else {
-            launch_persistent<HK_VOIGT_FP32C>(ppt, lm, gm, s, args, items, nspec, counter);
-            HK_LAUNCH_CHECK();
-            launch_persistent<HK_VOIGT_FP32C>(0, 1, gc, s, cargs, citems, nspec, counter + 1);
-        }
-        HK_LAUNCH_CHECK();
+        return HK_OK;
     }
+    hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_main + 3) / 4)),
+                       dim3(256), 0, s, args, items, nspec, batch->tile_points, 1);
+    HK_LAUNCH_CHECK();
+    hipLaunchKernelGGL(batched_ranges_kernel, dim3((unsigned)((batch->items_core + 3) / 4)),
+                       dim3(256), 0, s, cargs, citems, nspec, kCoreW, 1);
+    HK_LAUNCH_CHECK();
+    const unsigned gc = persistent_grid(batch->items_core);
+    launch_persistent<HK_VOIGT_FP32C>(ppt, lm, gm, s, args, items, nspec, counter);
+    HK_LAUNCH_CHECK();
+    launch_persistent<HK_VOIGT_FP32C>(0, 1, gc, s, cargs, citems, nspec, counter + 1);
+    HK_LAUNCH_CHECK();
     return HK_OK;
 }
 

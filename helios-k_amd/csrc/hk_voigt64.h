@@ -24,8 +24,10 @@
 //
 // What bounds it: FP64 vector instructions.  At 1e5 lines, 3e6 points, cut
 // 100 cm^-1 a line has 2e4 pairs in its window; it takes 20 node values in
-// each of ~17 tiles, 20 in ~9 waves and ~13 instructions' worth of 64
-// points -- 30 times fewer evaluations than pairs.
+// each of ~17 tiles, 20 in ~9 waves and ~13 segments of 64 points -- 30 times
+// fewer evaluations than pairs.  Pair by pair (with a separate line-core
+// pass) that spectrum took 2217 us, now 533; 2.35e6 lines on 7e6 points at
+// 10 bar, cut 25: 132 ms, now 15.3.
 #pragma once
 #include "hk_device.h"
 #include "hk_tiles.h"
@@ -56,10 +58,19 @@ struct Far64LDS {
     double F[kWaves][kFN64];                    // tile node sums, one row per wave
     double wF[kWaves][kFN64];                   // wave node sums, then its series
     double c[kWaves][kFN64];                    // tile series (a copy per wave)
+    double tab[kWaves][64];                     // core table of the wave's line
     double cosv[4 * kFN64];                     // cos(j pi / 40)
+    uint64_t taken[kWaves][kRound64 / 64];      // lines of a chunk the wave's nodes took
     int cnt[kWaves];
     int64_t range[2];
 };
+
+// Orders a wave's own LDS writes before its later reads of them.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // A uniform constant the compiler cannot hoist: the unrolled node loops use
 // dozens of FP64 literals, and kept in scalar registers across the tile loop
@@ -276,13 +287,6 @@ __device__ __forceinline__ double cheb_coef64(const double *F, const double *cos
     return (m == 0 ? 1.0 : 2.0) / (double)kFN64 * c;
 }
 
-// Orders a wave's own LDS writes before its later reads of them.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ double cheb_sum64(const double *c, double u) {
     double b1 = 0.0, b2 = 0.0;
     const double u2 = 2.0 * u;
@@ -302,38 +306,148 @@ __device__ __forceinline__ double lane_f64(double v, int b) {
     return __longlong_as_double(((long long)hi << 32) | lo);
 }
 
+// ---------------------------------------------------------------------------
+// Line core, x^2 + y^2 < 100: the midpoint rule for
+//   w(x + iy) = (i/pi) int e^{-(x+s)^2} / (iy - s) ds
+// on s = (k + 1/2) h (nodes that move with x, so the pole at s = iy is never
+// near one), plus that pole's residue (Chiarella & Reichel 1968, Hunter &
+// Regan 1972):
+//   Re w = (h y/pi) sum_s e^{-(x+s)^2} / (s^2 + y^2)
+//          + 2 e^{y^2-x^2} cos(2xy) / (1 + e^{2 pi y/h})     (y < pi/h)
+// With x = (n0 + 1/2) h + d, |d| <= h/2, the 24 nodes that count have
+// exponents -(d + m h)^2, m = -11..12: e^{-d^2} times a polynomial in
+// e^{-2hd} whose coefficients are the constants e^{-h^2 m^2} and the line's
+// table 1/(s^2 + y^2) at s = (n0 - m + 1/2) h.  h = 0.5178 leaves
+// e^{-pi^2/h^2} = 1e-16 of the integral; relative error of Re w <= 5e-15
+// against 50-digit values for 0 <= y < 10, tiny y and the far Doppler wing
+// included (every term of the sum is positive).
+// One exponential, one cosine and 24 table reads replace the 40 reciprocals
+// and 4 exponentials of the Algorithm 916 series that a separate pass took
+// (2.35e6 lines, 7e6 points at 10 bar: that pass 31 ms, the whole sum 39.9 ms,
+// now 15.3; 1e5 lines, 3e6 points: 900 -> 533 us).
+// ---------------------------------------------------------------------------
+constexpr double kHC = 0.5178;
+constexpr int kCLo = 11, kCHi = 12;               // m = -kCLo .. kCHi
+constexpr int kCTab = 19 + kCLo + kCHi + 1;       // n0 <= 19
+constexpr double kPiHC = 6.0671932282537524;      // pi / h
+// e^{-h^2 m^2}
+constexpr double kCE[kCHi + 1] = {
+    1, 0.76481841449861865, 0.34216323515981589, 0.089541635567738392, 0.013706714729223335,
+    0.0012273216551150678, 6.428358545165617e-05, 1.9695112154195025e-06, 3.5296650648060179e-08,
+    3.7002000654827686e-10, 2.2689952580918315e-12, 8.1387674929739835e-15, 1.7076559162725319e-17};
+
+// e^v for |v| <= 0.35 by its Taylor series (first term left out < 3e-18).
+__device__ __forceinline__ double exp_small(double v) {
+    constexpr double c[14] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
+                              1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800,
+                              1.0 / 479001600, 1.0 / 6227020800};
+    double s = local_const(c[13]);
+#pragma unroll
+    for (int k = 12; k >= 2; --k) s = fma(s, v, local_const(c[k]));
+    return fma(fma(s, v, 1.0), v, 1.0);
+}
+
+// e^-t, 0 <= t <= 100 (t = n ln 2 - v in two parts).
+__device__ __forceinline__ double exp_neg(double t) {
+    const double n = rint(t * local_const(1.4426950408889634));
+    double v = fma(n, local_const(0.69314718055994531), -t);
+    v = fma(n, local_const(2.3190468138462996e-17), v);
+    return ldexp(exp_small(v), -(int)n);
+}
+
+// cos(t), 0 <= t <= 130, to ~1e-16 absolute: t = n pi + v in two parts, the
+// Taylor series in v^2 (|v| <= pi/2; first term left out < 2e-17).
+__device__ __forceinline__ double cos_bounded(double t) {
+    constexpr double c[12] = {1.0, -1.0 / 2, 1.0 / 24, -1.0 / 720, 1.0 / 40320, -1.0 / 3628800,
+                              1.0 / 479001600, -1.0 / 87178291200.0, 1.0 / 20922789888000.0,
+                              -1.0 / 6402373705728000.0, 1.0 / 2432902008176640000.0,
+                              -1.0 / 1124000727777607680000.0};
+    const double n = rint(t * local_const(0.31830988618379067));
+    double v = fma(-n, local_const(3.1415926535897931), t);
+    v = fma(-n, local_const(1.2246467991473532e-16), v);
+    const double w = v * v;
+    double s = local_const(c[11]);
+#pragma unroll
+    for (int k = 10; k >= 1; --k) s = fma(s, w, local_const(c[k]));
+    s = fma(s, w, 1.0);
+    return ((int)n & 1) ? -s : s;
+}
+
+// Factor of e^{-x^2} cos(2xy) in sqrt(pi) Re w's pole term, per line.
+__device__ __forceinline__ double core_pole(double y) {
+    if (!(y < kPiHC)) return 0.0;
+    const double b = y * (2.0 * kPiHC - y);          // 2 pi y/h - y^2 >= 0
+    return 2.0 * exp_neg(b) / (1.0 + exp_neg(2.0 * kPiHC * y));
+}
+
+// The line's table, lane l < kCTab: 1/(s^2 + y^2), s = (l - kCHi + 1/2) h.
+__device__ __forceinline__ void core_table(double *tab, double y2) {
+    const int lane = threadIdx.x & 63;
+    const double s = ((double)(lane - kCHi) + 0.5) * kHC;
+    wave_lds_sync();
+    if (lane < kCTab) tab[lane] = rcp64(fma(s, s, y2));
+    wave_lds_sync();
+}
+
+// sqrt(pi) times the profile, times S: G h/2 e^{-d^2} (polynomial) + Apf
+// e^{-x^2} cos(2xy), for |x| <= 10.
+__device__ __forceinline__ double core_value(double x, double y, double G, double Apf,
+                                             const double *tab) {
+    const double ax = fmin(fabs(x), 10.0);
+    const int n0 = (int)(ax * (1.0 / kHC));
+    const double d = fma(-((double)n0 + 0.5), kHC, ax);
+    const double *tb = tab + n0;
+    const double r = exp_small(-2.0 * kHC * d), ri = rcp64(r);
+    double P = 0.0, Q = 0.0;
+#pragma unroll
+    for (int m = kCHi; m >= 0; --m) {
+        const double ce = local_const(kCE[m]);
+        P = fma(P, r, ce * tb[kCHi - m]);
+        if (m > 0 && m <= kCLo) Q = fma(Q, ri, ce * tb[kCHi + m]);
+    }
+    double v = (0.5 * kHC) * G * exp_small(-d * d) * fma(Q, ri, P);
+    if (Apf != 0.0) v = fma(Apf * exp_neg(ax * ax), cos_bounded(2.0 * ax * y), v);
+    return v;
+}
+
 // Point-by-point part of one line on the wave's points: per 64-point segment
 // 2 bits of code, 1: x^2 + y^2 >= 1e4 at all its points (4 nodes), 2: >= 100
-// (8 nodes), 3: some points lie in the line core (skipped here; the line-core
-// pass adds them).
+// (8 nodes), 3: some points lie in the line core.
 template <int PPT>
-__device__ __forceinline__ void add_points(uint32_t code, double nu, double ia, double y2, double G,
-                                           int lo, int hi, bool full, const double (&xj)[PPT],
-                                           double (&acc)[PPT]) {
+__device__ __forceinline__ void add_points(uint32_t code, double nu, double ia, double y, double G,
+                                           double Apf, int lo, int hi, bool full, double jd,
+                                           double numin, double dnu, double (&acc)[PPT],
+                                           double *tab) {
     const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        const int c = (code >> (2 * k)) & 3;
+    const double y2 = y * y;
+    if (code & (code >> 1) & 0x55555555u) core_table(tab, y2);
+    for (int k = 0; code != 0; ++k, code >>= 2) {
+        const int c = code & 3;
         if (c == 0) continue;
-        const double x = (xj[k] - nu) * ia;
+        const double x = (fma(jd + (double)(64 * k), dnu, numin) - nu) * ia;
         const double x2 = x * x;
-        double v;
+        const double r2 = fma(x, x, y2);
+        double v = 0.0, num, den;
         if (c == 1) {
-            double num, den;
-            gh_frac(GH<2>(), x2, x2 + y2, num, den);
+            gh_frac(GH<2>(), x2, r2, num, den);
             v = G * (num * rcp64(den));
-        } else {
-            const double r2 = fma(x, x, y2);
-            double num, den;
+        } else if (c == 2 || __ballot(r2 >= kRB64) != 0ull) {
             gh_frac(GH<4>(), x2, r2, num, den);
             v = G * (num * rcp64(den));
-            if (c == 3) v = r2 >= kRB64 ? v : 0.0;
+        }
+        if (c == 3) {
+            const double w = core_value(x, y, G, Apf, tab);
+            v = r2 < kRB64 ? w : v;
         }
         if (!full) {
             const int j = lane + 64 * k;
             v = (j >= lo && j < hi) ? v : 0.0;
         }
-        acc[k] += v;
+        // one copy of the code above for all segments: acc is a register
+        // array, so the segment's sum is picked by uniform branches
+#pragma unroll
+        for (int q = 0; q < PPT; ++q)
+            if (q == k) acc[q] += v;
     }
 }
 
@@ -355,12 +469,10 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     const double xwf = fma((double)jw, a.dnu, a.numin);
     const double hw_w = fmax(0.5 * (double)(nw - 1), 0.5) * a.dnu;
     const double xcw = fma((double)jw + 0.5 * (double)max(nw - 1, 0), a.dnu, a.numin);
-    double xj[PPT], acc[PPT];
+    const double jd = (double)(jw + lane);        // this lane's first point
+    double acc[PPT];
 #pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        xj[k] = fma((double)(jw + lane + 64 * k), a.dnu, a.numin);
-        acc[k] = 0.0;
-    }
+    for (int k = 0; k < PPT; ++k) acc[k] = 0.0;
     // line range of the tile: waves 0 and 1 search one end each
     if (t < 4 * kFN64) sh->cosv[t] = cospi((double)t / (2.0 * kFN64));
     if (lane < kFN64) { sh->F[wave][lane] = 0.0; sh->wF[wave][lane] = 0.0; }
@@ -416,37 +528,71 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         }
         if (lane == 0) sh->cnt[wave] = cnt;
         __syncthreads();
-        // near lines of all waves, 64 at a time, one per lane
+        // near lines of all waves, in chunks of 64, one line per lane
         int cum[kWaves + 1];
         cum[0] = 0;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) cum[w + 1] = cum[w] + sh->cnt[w];
         const int total = nw > 0 ? cum[kWaves] : 0;
-        double f[kFN64];
+        auto line_at = [&](int e) {
+            int w = 0, c = 0;
 #pragma unroll
-        for (int k = 0; k < kFN64; ++k) f[k] = 0.0;
-        bool used = false;
+            for (int q = 1; q < kWaves; ++q)
+                if (e >= cum[q]) { w = q; c = cum[q]; }
+            return r0 + sh->list[w][e - c];
+        };
+        // wave level (a loop of its own: its node sums and the point loop's
+        // values do not fit the registers together)
+        {
+            double f[kFN64];
+#pragma unroll
+            for (int k = 0; k < kFN64; ++k) f[k] = 0.0;
+            bool used = false;
+            const double xwl = fma((double)(jw + nw - 1), a.dnu, a.numin);
+            for (int c0 = 0; c0 < total; c0 += 64) {
+                int cls = 0;
+                double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0;
+                if (a.far && c0 + lane < total) {
+                    const int64_t i = line_at(c0 + lane);
+                    const double nu = a.nu[i], hw = a.hw[i];
+                    const double dl = xwf - nu, dh = xwl - nu;
+                    D = xcw - nu;
+                    if (dl > -hw && dl < hw && dh > -hw && dh < hw &&
+                        fabs(D) >= kFarRatio64 * hw_w) {
+                        const double y = a.y[i];
+                        ia = a.ia[i];
+                        y2 = y * y;
+                        G = a.S[i] * y * (kISqrtPi * 2.0 / kPi);
+                        cls = far_class64(D, hw_w, ia, y2, G);
+                    }
+                }
+                unsigned long long wm = __ballot(cls != 0);
+                if (__popcll(wm) >= wave_min_lines(PPT)) {
+                    add_far_lines(cls, D, hw_w, ia, y2, G, f);
+                    used = true;
+                } else wm = 0ull;
+                if (lane == 0) sh->taken[wave][c0 >> 6] = wm;
+            }
+            if (used) { add_node_totals(f, sh->wF[wave]); any_wave = true; }
+        }
+        wave_lds_sync();
+        // the rest point by point
         for (int c0 = 0; c0 < total; c0 += 64) {
             const int e = c0 + lane;
             uint32_t code = 0;
-            int lo = 0, hi = 0, cls = 0;
-            double nu = 0.0, ia = 1.0, y2 = 1.0, G = 0.0, D = 1.0;
-            if (e < total) {
-                int w = 0;
-#pragma unroll
-                for (int q = 1; q < kWaves; ++q) w += e >= cum[q];
-                const int64_t i = r0 + sh->list[w][e - (w == 0 ? 0 : w == 1 ? cum[1] : w == 2 ? cum[2] : cum[3])];
+            int lo = 0, hi = 0;
+            double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0;
+            if (e < total && !((sh->taken[wave][c0 >> 6] >> lane) & 1ull)) {
+                const int64_t i = line_at(e);
                 nu = a.nu[i];
-                const double hw = a.hw[i], y = a.y[i];
-                ia = a.ia[i];
-                y2 = y * y;
-                G = a.S[i] * y * (kISqrtPi * 2.0 / kPi);
-                clip_window(nu, hw, a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
+                clip_window(nu, a.hw[i], a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
                 if (lo < hi) {
-                    D = xcw - nu;
-                    if (a.far && lo == 0 && hi == nw) cls = far_class64(D, hw_w, ia, y2, G);
+                    const double A = a.S[i] * kISqrtPi;
+                    y = a.y[i];
+                    ia = a.ia[i];
+                    G = A * y * (2.0 / kPi);
                     // conservative point intervals with x^2 + y^2 < 100, 1e4
-                    const float vb = (float)(a.dnu * ia), fy2 = (float)y2;
+                    const float vb = (float)(a.dnu * ia), fy2 = (float)(y * y);
                     const float cen = (float)((nu - xwf) * inv_dnu);
                     const float r1 = sqrtf(fmaxf(1.0002e2f - fy2, 0.0f)) / vb;
                     const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
@@ -460,13 +606,8 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         const bool c2 = in2 && cen - r2 - mg <= (float)s1 && cen + r2 + mg >= (float)s0;
                         code |= (c3 ? 3u : c2 ? 2u : 1u) << (2 * k);
                     }
+                    if (code & (code >> 1) & 0x55555555u) Apf = A * core_pole(y);
                 }
-            }
-            const unsigned long long wm = __ballot(cls != 0);
-            if (__popcll(wm) >= wave_min_lines(PPT)) {
-                add_far_lines(cls, D, hw_w, ia, y2, G, f);
-                used = true;
-                if (cls) code = 0;
             }
             unsigned long long m = __ballot(code != 0);
             while (m) {
@@ -474,11 +615,11 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 m &= m - 1ull;
                 const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
                 add_points<PPT>((uint32_t)__builtin_amdgcn_readlane((int)code, b), lane_f64(nu, b),
-                                lane_f64(ia, b), lane_f64(y2, b), lane_f64(G, b), slo, shi,
-                                slo == 0 && shi == nw, xj, acc);
+                                lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b), lane_f64(Apf, b),
+                                slo, shi, slo == 0 && shi == nw, jd, a.numin, a.dnu, acc,
+                                sh->tab[wave]);
             }
         }
-        if (used) { add_node_totals(f, sh->wF[wave]); any_wave = true; }
         __syncthreads();      // the lists are free for the next round
     }
     // node sums -> one series per wave.  any_far differs between waves: the
@@ -510,7 +651,8 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         if (lane < kFN64) c[lane] = cm;
         wave_lds_sync();
 #pragma unroll
-        for (int k = 0; k < PPT; ++k) acc[k] += cheb_sum64(c, (xj[k] - xcw) / hw_w);
+        for (int k = 0; k < PPT; ++k)
+            acc[k] += cheb_sum64(c, (fma(jd + (double)(64 * k), a.dnu, a.numin) - xcw) / hw_w);
     }
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
