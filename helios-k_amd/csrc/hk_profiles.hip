@@ -22,61 +22,33 @@
 // factor on, every profile -- Voigt included, through the FP64 Faddeeva
 // function -- runs in this file's FP64 gather.
 //
-// Kernels: one workgroup of 256 threads per tile of 1024 points (4 per
-// thread, coalesced); the tile's line range comes from the shared
-// binary-search kernel; lines are staged 256 at a time in LDS with their
-// cut window clipped to the tile; sums stay in registers in line order, so
-// results are deterministic.  All arithmetic is FP64.
+// Kernel: the FP64 tile sum of hk_voigt64.h with the profile as its parameter --
+// Voigt and Lorentz wings far from a tile or a wave through Chebyshev nodes
+// (with the sub-Lorentzian factor where it is one analytic piece there),
+// Doppler and binned-Gaussian lines only where they do not underflow to zero,
+// plinths of lines that cover a tile or a wave as one constant -- so a line
+// costs a few hundred evaluations, not one per point of its window.  What bounds
+// it: FP64 vector instructions.  All arithmetic is FP64, in a fixed order.
+// Pair by pair, Voigt with chi over 2e4 lines, 1e5 points, cut 120 took 7.0 ms,
+// this 1.05; Voigt with plinth over 3e5 lines, 3e6 points, cut 25 in two passes
+// 1.57 ms, in one 1.29.
 #include <math.h>
 
 #include "hk_device.h"
 #include "hk_internal.h"
-#include "hk_tiles.h"
+#include "hk_voigt64.h"
 
 namespace {
 
 using namespace hk;
 
-constexpr int kPT = 256;             // threads per workgroup
 constexpr int kPPT = 4;              // points per thread
-constexpr int kPW = kPT * kPPT;      // points per tile
-
-struct PRec {
-    double nu, ia, S1, y, pl, vb;
-    int32_t lo, hi;                  // tile-relative window [lo, hi)
-};
-
-// Binned Gaussian cell average of exp(-t^2)/sqrt(pi) times vb:
-// (erf(x + h) - erf(x - h)) / 2 with h = vb/2.
-__device__ __forceinline__ double binned_gauss(double x, double h) {
-    return x >= 0.0 ? 0.5 * (erfc(x - h) - erfc(x + h)) : 0.5 * (erfc(-x - h) - erfc(-x + h));
-}
-
-// Profile value of one pair; S1 is the per-line prefactor formed at staging.
-template <int PROFILE>
-__device__ __forceinline__ double profile_value(double S1, double x, double y, double vb) {
-    if (PROFILE == 1) return S1 * rew64(x, y);
-    if (PROFILE == 2) return S1 / (x * x + y * y);
-    if (PROFILE == 3) return S1 * exp(-x * x);
-    return S1 / vb * binned_gauss(x, 0.5 * vb);
-}
+constexpr int kPW = kThreads * kPPT; // points per tile
 
 __device__ __forceinline__ double prefactor(int profile, double S, double y) {
     if (profile == 2) return S * y / kPi;
     if (profile == 3 || profile == 1) return S * kISqrtPi;
     return S;
-}
-
-struct Chi {
-    double s1, s2, s3, B1, B2, B3, lo, hi;
-};
-
-// Perrin & Hartmann (1989) chi of the distance d = |x - nu| [cm^-1].
-__device__ __forceinline__ double chi_of(const Chi &c, double d) {
-    if (d < c.s1) return 1.0;
-    if (d < c.s2) return exp(-c.B1 * (d - c.s1));
-    if (d < c.s3) return exp(-c.B1 * (c.s2 - c.s1) - c.B2 * (d - c.s2));
-    return exp(-c.B1 * (c.s2 - c.s1) - c.B2 * (c.s3 - c.s2) - c.B3 * (d - c.s3));
 }
 
 // Plinth of each line: its profile at the cut (0 for empty lines).
@@ -97,81 +69,52 @@ __global__ __launch_bounds__(256) void plinth_kernel(
 }
 
 struct PArgs {
-    const double *nu, *S, *ia, *y, *hw, *pl;
+    const double *nu, *S, *ia, *y, *hw, *pl, *key, *radius;
     int64_t nl;
-    const TileInfo *tiles;
     double numin, dnu;
     int64_t nx;
     double kmin;
-    int accumulate;
+    int accumulate, far;
     double *K;
     Chi chi;
+    // sub-Lorentzian range and the points a pass writes: 0 all, 1 those inside
+    // the range, -1 those outside
+    double lo, hi;
+    int side;
 };
 
 // PROFILE 1..4: profile sums (minus plinths when PLINTH); PROFILE 0: the
-// plinth subtraction alone (after a Voigt sum), always accumulating.
+// plinth subtraction alone (after an FP32C or compat Voigt sum).
 template <int PROFILE, bool PLINTH, bool CHI>
-__global__ __launch_bounds__(kPT) void profile_tiles_kernel(PArgs a) {
-    __shared__ PRec rec[kPT];
-    const int tid = threadIdx.x;
-    const int64_t j0 = (int64_t)blockIdx.x * kPW;
-    const TileInfo ti = a.tiles[blockIdx.x];
-    double acc[kPPT];
-#pragma unroll
-    for (int k = 0; k < kPPT; ++k) acc[k] = 0.0;
-    for (int64_t base = ti.lo; base < ti.hi; base += kPT) {
-        const int64_t i = base + tid;
-        PRec r;
-        r.lo = 0; r.hi = 0;
-        r.nu = 0.0; r.ia = 0.0; r.S1 = 0.0; r.y = 0.0; r.pl = 0.0; r.vb = 0.0;
-        if (i < ti.hi) {
-            int64_t lo, hi;
-            cut_window(a.nu[i], a.hw[i], a.numin, a.dnu, a.nx, lo, hi);
-            lo = max(lo, j0) - j0;
-            hi = min(hi, j0 + kPW) - j0;
-            if (lo < hi) {
-                r.lo = (int32_t)lo; r.hi = (int32_t)hi;
-                r.nu = a.nu[i]; r.ia = a.ia[i]; r.y = a.y[i];
-                r.S1 = PROFILE ? prefactor(PROFILE, a.S[i], r.y) : 0.0;
-                r.pl = PLINTH ? a.pl[i] : 0.0;
-                r.vb = a.dnu * r.ia;
+__global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
+    __shared__ Far64LDS sh;
+    if constexpr (CHI) {
+        // a tile that an end of the range cuts is summed twice, as if all of it
+        // lay inside and then outside: the factor is smooth over each.  (Summed
+        // point by point instead, the two such tiles of a 1e5-point grid took
+        // 8.1 ms, the other 96 together 1.1.)
+        const int64_t j0 = (int64_t)blockIdx.x * kPW;
+        const double x0 = fma((double)j0, a.dnu, a.numin);
+        const double x1 = fma((double)min(j0 + kPW, a.nx) - 1.0, a.dnu, a.numin);
+        const bool cut = (x0 <= a.lo && x1 > a.lo) || (x0 < a.hi && x1 >= a.hi);
+        for (int pass = 0; pass < (cut ? 2 : 1); ++pass) {
+            if (cut) {
+                a.side = pass == 0 ? 1 : -1;
+                a.chi.lo = pass == 0 ? -INFINITY : INFINITY;
+                a.chi.hi = -a.chi.lo;
+                __syncthreads();
             }
+            tile_f64<kPPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
         }
-        rec[tid] = r;
-        __syncthreads();
-        const int nr = (int)min((int64_t)kPT, ti.hi - base);
-        for (int q = 0; q < nr; ++q) {
-            const PRec &L = rec[q];
-            if (L.lo >= L.hi) continue;
-#pragma unroll
-            for (int k = 0; k < kPPT; ++k) {
-                const int jj = tid + k * kPT;
-                if (jj >= L.lo && jj < L.hi) {
-                    double v = 0.0;
-                    if (PROFILE) {
-                        const double xj = fma((double)(j0 + jj), a.dnu, a.numin);
-                        const double d = xj - L.nu;
-                        v = profile_value<PROFILE>(L.S1, d * L.ia, L.y, L.vb);
-                        if (CHI && xj > a.chi.lo && xj < a.chi.hi)
-                            v *= chi_of(a.chi, fabs(d)) * xj / L.nu;
-                    }
-                    acc[k] += v - L.pl;
-                }
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < kPPT; ++k) {
-        const int64_t j = j0 + tid + k * kPT;
-        if (j < a.nx) a.K[j] = (a.accumulate || PROFILE == 0) ? a.K[j] + acc[k] : a.kmin + acc[k];
+    } else {
+        tile_f64<kPPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
     }
 }
 
 template <int PROFILE, bool PLINTH, bool CHI = false>
 void launch_profile(int64_t ntiles, hipStream_t s, const PArgs &a) {
     hipLaunchKernelGGL((profile_tiles_kernel<PROFILE, PLINTH, CHI>), dim3((unsigned)ntiles),
-                       dim3(kPT), 0, s, a);
+                       dim3(kThreads), 0, s, a);
 }
 
 template <int PROFILE>
@@ -180,16 +123,9 @@ void launch_chi(bool plinth, int64_t ntiles, hipStream_t s, const PArgs &a) {
     else launch_profile<PROFILE, false, true>(ntiles, s, a);
 }
 
-size_t tiles_bytes(const hk_grid *g) {
-    const int64_t nt = (g->nx + kPW - 1) / kPW;
-    return align_up((size_t)nt * sizeof(TileInfo), 256);
-}
-
 size_t region_bytes(const hk_grid *g) {
     hk_tune t = {0, 0};
-    const size_t v = hk_voigt_workspace_bytes(g, &t);
-    const size_t p = tiles_bytes(g);
-    return align_up(v > p ? v : p, 256);
+    return align_up(hk_voigt_workspace_bytes(g, &t), 256);
 }
 
 }  // namespace
@@ -228,7 +164,11 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
         HK_CHECK_ARG(chi->sigma[0] <= chi->sigma[1] && chi->sigma[1] <= chi->sigma[2],
                      "hk_profile_accumulate: chi breaks must be ascending");
     }
-    if (profile == HK_PROFILE_VOIGT && !chi) {
+    // Voigt without the plinth, or in another form than FP64: the Voigt sum
+    // (then the plinths alone)
+    const bool voigt_sum = profile == HK_PROFILE_VOIGT && !chi &&
+                           !(remove_plinth && voigt_mode == HK_VOIGT_FP64);
+    if (voigt_sum) {
         hk_tune t = {0, 0};
         int rc = hk_voigt_accumulate(st, grid, kmin, accumulate, voigt_mode, &t, K, w, rb, stream);
         if (rc != HK_OK || !remove_plinth) return rc;
@@ -240,20 +180,20 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
         HK_LAUNCH_CHECK();
     }
     const int64_t ntiles = (grid->nx + kPW - 1) / kPW;
-    TileInfo *tiles = (TileInfo *)w;
-    hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((ntiles + 3) / 4)), dim3(256), 0, s,
-                       st->key, n, st->radius, st->blk_max, grid->numin, grid->dnu, grid->nx,
-                       kPW, ntiles, 0, tiles);
-    HK_LAUNCH_CHECK();
     PArgs a;
     a.nu = st->nu; a.S = st->S; a.ia = st->ialphaD; a.y = st->y; a.hw = st->hw; a.pl = pl;
-    a.nl = n; a.tiles = tiles; a.numin = grid->numin; a.dnu = grid->dnu; a.nx = grid->nx;
-    a.kmin = kmin; a.accumulate = accumulate; a.K = K;
+    a.key = st->key; a.radius = st->radius;
+    a.nl = n; a.numin = grid->numin; a.dnu = grid->dnu; a.nx = grid->nx;
+    a.kmin = kmin; a.accumulate = accumulate || voigt_sum; a.far = 1; a.K = K;
     a.chi = Chi{0, 0, 0, 0, 0, 0, 0, 0};
+    a.lo = a.hi = 0.0;
+    a.side = 0;
     const bool P = remove_plinth != 0;
     if (chi) {
         a.chi = Chi{chi->sigma[0], chi->sigma[1], chi->sigma[2], chi->B[0], chi->B[1], chi->B[2],
                     chi->range[0], chi->range[1]};
+        a.lo = a.chi.lo;
+        a.hi = a.chi.hi;
         switch (profile) {
         case HK_PROFILE_VOIGT: launch_chi<1>(P, ntiles, s, a); break;
         case HK_PROFILE_LORENTZ: launch_chi<2>(P, ntiles, s, a); break;
@@ -264,7 +204,9 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
         return HK_OK;
     }
     switch (profile) {
-    case HK_PROFILE_VOIGT: launch_profile<0, true>(ntiles, s, a); break;
+    case HK_PROFILE_VOIGT:
+        voigt_sum ? launch_profile<0, true>(ntiles, s, a) : launch_profile<1, true>(ntiles, s, a);
+        break;
     case HK_PROFILE_LORENTZ:
         P ? launch_profile<2, true>(ntiles, s, a) : launch_profile<2, false>(ntiles, s, a);
         break;

@@ -1343,7 +1343,7 @@ __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_ke
     const int64_t tile = blockIdx.x;
     if (MODE == HK_VOIGT_FP64) {
         __shared__ Far64LDS sh;
-        tile_f64<PPT>(a, tile, &sh);
+        tile_f64<PPT, LineSum<1, false, false>>(a, tile, &sh);
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
@@ -1406,7 +1406,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
         if constexpr (PPT == 0) {
             core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
-            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT>(a, tile, (Far64LDS *)smem);
+            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false>>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
         }
     }

@@ -61,6 +61,7 @@ struct Far64LDS {
     double tab[kWaves][64];                     // core table of the wave's line
     double cosv[4 * kFN64];                     // cos(j pi / 40)
     uint64_t taken[kWaves][kRound64 / 64];      // lines of a chunk the wave's nodes took
+    double cst[kWaves];                         // plinths of lines that cover the tile
     int cnt[kWaves];
     int64_t range[2];
 };
@@ -78,6 +79,25 @@ __device__ __forceinline__ void wave_lds_sync() {
 __device__ __forceinline__ double local_const(double v) {
     asm volatile("" : "+s"(v));
     return v;
+}
+
+// e^v for |v| <= 0.35 by its Taylor series (first term left out < 3e-18).
+__device__ __forceinline__ double exp_small(double v) {
+    constexpr double c[14] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
+                              1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800,
+                              1.0 / 479001600, 1.0 / 6227020800};
+    double s = local_const(c[13]);
+#pragma unroll
+    for (int k = 12; k >= 2; --k) s = fma(s, v, local_const(c[k]));
+    return fma(fma(s, v, 1.0), v, 1.0);
+}
+
+// e^-t, |t| <= 800 (t = n ln 2 - v in two parts).
+__device__ __forceinline__ double exp_neg(double t) {
+    const double n = rint(t * local_const(1.4426950408889634));
+    double v = fma(n, local_const(0.69314718055994531), -t);
+    v = fma(n, local_const(2.3190468138462996e-17), v);
+    return ldexp(exp_small(v), -(int)n);
 }
 
 __device__ __forceinline__ double swap_add32(double a, double b) {
@@ -133,16 +153,100 @@ __device__ __forceinline__ void add_node_totals(const double (&f)[kFN64], double
     if (p < kFN64 / 4) row[4 * p + (r == 1 ? 2 : r == 2 ? 1 : r)] += mine;
 }
 
+// Sub-Lorentzian factor of the wings (hk_chi): for lo < x < hi a line's value is
+// multiplied by chi(|x - nu|) x / nu.
+struct Chi {
+    double s1, s2, s3, B1, B2, B3, lo, hi;
+};
+
+// -ln chi at distance d (Perrin & Hartmann 1989).
+__device__ __forceinline__ double chi_exponent(const Chi &c, double d) {
+    if (d < c.s1) return 0.0;
+    if (d < c.s2) return c.B1 * (d - c.s1);
+    if (d < c.s3) return fma(c.B1, c.s2 - c.s1, c.B2 * (d - c.s2));
+    return fma(c.B1, c.s2 - c.s1, fma(c.B2, c.s3 - c.s2, c.B3 * (d - c.s3)));
+}
+
+// The factor over an interval on which it is one analytic piece:
+// exp(-(B (x - nu) + t0)) (1 + (x - nu) inv_nu); all 0 outside the range.
+struct ChiPiece {
+    double B = 0.0, t0 = 0.0, inv_nu = 0.0;
+};
+
+// Finds the piece for the points xa..xb (D: the interval's centre from the
+// line's); false when they straddle a break or an end of the range, or when the
+// exponential varies too much for the nodes (|B| half <= 2 leaves 1e-18).
+__device__ __forceinline__ bool chi_piece(const Chi &c, double xa, double xb, double nu, double D,
+                                          double half, ChiPiece &p) {
+    p = ChiPiece();
+    if (xb <= c.lo || xa >= c.hi) return true;
+    if (!(xa > c.lo && xb < c.hi)) return false;
+    const double d0 = fabs(D) - half, d1 = fabs(D) + half;
+    double B, t0;
+    if (d1 <= c.s1) { B = 0.0; t0 = 0.0; }
+    else if (d0 >= c.s1 && d1 <= c.s2) { B = c.B1; t0 = -c.B1 * c.s1; }
+    else if (d0 >= c.s2 && d1 <= c.s3) { B = c.B2; t0 = fma(c.B1, c.s2 - c.s1, -c.B2 * c.s2); }
+    else if (d0 >= c.s3) {
+        B = c.B3;
+        t0 = fma(c.B1, c.s2 - c.s1, fma(c.B2, c.s3 - c.s2, -c.B3 * c.s3));
+    } else return false;
+    p.B = D < 0.0 ? -B : B;
+    p.t0 = t0;
+    p.inv_nu = 1.0 / nu;
+    return fabs(B) * half <= 2.0;
+}
+
+// What a line contributes to a point: PROFILE 1 Voigt, 2 Lorentz, 3 Doppler,
+// 4 binned Gaussian, 0 nothing but the plinth; PLINTH subtracts the line's
+// value at its cut (args.pl) over its whole window; CHI applies args.chi.
+template <int PROFILE_, bool PLINTH_, bool CHI_>
+struct LineSum {
+    static constexpr int PROFILE = PROFILE_;
+    static constexpr bool PLINTH = PLINTH_, CHI = CHI_;
+    // wings that the nodes can take, or a value that underflows to zero beyond
+    // x = kDopplerEnd (e^-x^2 does at 27.3)
+    static constexpr bool WINGS = PROFILE == 1 || PROFILE == 2;
+    static constexpr bool COMPACT = PROFILE == 3 || PROFILE == 4;
+};
+constexpr double kDopplerEnd = 27.5;
+
+// The factor G of a line's profile value.
+template <class P>
+__device__ __forceinline__ double line_factor(double S, double y) {
+    if (P::PROFILE == 1) return S * kISqrtPi * y * (2.0 / kPi);
+    if (P::PROFILE == 2) return S * y / kPi;
+    return P::PROFILE == 3 ? S * kISqrtPi : P::PROFILE == 4 ? S : 0.0;
+}
+
+__device__ __forceinline__ double lane_f64(double v, int b) {
+    const long long x = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)x, b);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(x >> 32), b);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
+// Sum of v over the wave (fixed order), in every lane.
+__device__ __forceinline__ double wave_total64(double v) {
+    v += row_dpp64<0xb1>(v);
+    v += row_dpp64<0x4e>(v);
+    v += row_dpp64<0x141>(v);
+    v += row_dpp64<0x140>(v);
+    return ((lane_f64(v, 0) + lane_f64(v, 16)) + lane_f64(v, 32)) + lane_f64(v, 48);
+}
+
 // Far class of a line for an interval of half width `half` whose centre lies
 // D from the line centre [cm^-1]: 0 = not far, else the wing formula its
-// nearest point allows (1 series, 2 four nodes, 3 eight nodes).
+// nearest point allows (1 series, 2 four nodes, 3 eight nodes; Lorentz has one
+// formula).
+template <class P>
 __device__ __forceinline__ int far_class64(double D, double half, double ia, double y2, double G) {
+    if (!P::WINGS) return 0;
     const double d = fabs(D);
     const double xn = (d - half) * ia, xf = (d + half) * ia;
     const double rn = fma(xn, xn, y2), rf = fma(xf, xf, y2);
-    const bool ok = d >= kFarRatio64 * half && rn >= kRB64 && rf < kFarMaxR2 &&
-                    fabs(G) < 1.0e300;
-    return !ok ? 0 : rn >= kRF64 ? 1 : rn >= kRM64 ? 2 : 3;
+    const bool ok = d >= kFarRatio64 * half && fabs(G) < 1.0e300;
+    if (P::PROFILE == 2) return ok && rn > 0.0 && rf < 1.0e150 ? 1 : 0;
+    return !(ok && rn >= kRB64 && rf < kFarMaxR2) ? 0 : rn >= kRF64 ? 1 : rn >= kRM64 ? 2 : 3;
 }
 
 // Constants of the two Gauss-Hermite rules (gh4_sum64, gh8_sum64): squared
@@ -190,13 +294,13 @@ __device__ __forceinline__ void gh_frac(const GH<4> &q, double x2, double r2, do
 
 // One line's values at the 20 nodes of an interval (centre D from the line
 // centre, half width half), added to f.  The nodes +-u_k share one
-// reciprocal.  g = 2 S y / pi^1.5 (0 for a lane without a line).
-template <int CLASS>
+// reciprocal.  g: line_factor (0 for a lane without a line).
+template <class P, int CLASS>
 __device__ __forceinline__ void add_nodes(double D, double half, double ia, double y2, double g,
-                                          double (&f)[kFN64]) {
+                                          const ChiPiece &chi, double (&f)[kFN64]) {
     const double xc = D * ia, h = half * ia;
     double p2 = 0.0, p3 = 0.0, p4 = 0.0;
-    if (CLASS == 1) {
+    if (P::PROFILE == 1 && CLASS == 1) {
         p2 = fma(-2.0, y2, 3.75); p3 = -15.0 * y2; p4 = 12.0 * y2 * y2;
         g *= 0.5 * kPi * kISqrtPi;      // S y / pi
     }
@@ -208,33 +312,45 @@ __device__ __forceinline__ void add_nodes(double D, double half, double ia, doub
         const double xa = fma(u, h, xc), xb = fma(-u, h, xc);
         const double a2 = xa * xa, b2 = xb * xb;
         const double ra = a2 + y2, rb = b2 + y2;
-        if (CLASS == 1) {
+        double va, vb;
+        if (P::PROFILE == 2) {
+            const double q = rcp64(ra * rb);
+            va = q * rb;
+            vb = q * ra;
+        } else if (CLASS == 1) {
             const double q = rcp64(ra * rb), ia1 = q * rb, ib1 = q * ra;
-            const double va = fma(fma(fma(fma(p4, ia1, p3), ia1, p2), ia1, 1.5), ia1, 1.0);
-            const double vb = fma(fma(fma(fma(p4, ib1, p3), ib1, p2), ib1, 1.5), ib1, 1.0);
-            f[k] = fma(g * ia1, va, f[k]);
-            f[kFN64 - 1 - k] = fma(g * ib1, vb, f[kFN64 - 1 - k]);
+            va = ia1 * fma(fma(fma(fma(p4, ia1, p3), ia1, p2), ia1, 1.5), ia1, 1.0);
+            vb = ib1 * fma(fma(fma(fma(p4, ib1, p3), ib1, p2), ib1, 1.5), ib1, 1.0);
         } else {
             double na, da, nb, db;
             gh_frac(gh, a2, ra, na, da);
             gh_frac(gh, b2, rb, nb, db);
-            // (g last: strengths far below 1e-100 must not meet the products)
             const double q = rcp64(da * db);
-            f[k] = fma(g, na * db * q, f[k]);
-            f[kFN64 - 1 - k] = fma(g, nb * da * q, f[kFN64 - 1 - k]);
+            va = na * db * q;
+            vb = nb * da * q;
         }
+        if (P::CHI) {
+            const double ea = fma(u, half, D), eb = fma(-u, half, D);
+            va *= exp_neg(fma(chi.B, ea, chi.t0)) * fma(ea, chi.inv_nu, 1.0);
+            vb *= exp_neg(fma(chi.B, eb, chi.t0)) * fma(eb, chi.inv_nu, 1.0);
+        }
+        // (g last: strengths far below 1e-100 must not meet the products)
+        f[k] = fma(g, va, f[k]);
+        f[kFN64 - 1 - k] = fma(g, vb, f[kFN64 - 1 - k]);
     }
 }
 
 // The lanes with cls != 0 add their lines' node values; the whole wave takes
 // the formula of the line nearest its interval (valid farther out too).
+template <class P>
 __device__ __forceinline__ void add_far_lines(int cls, double D, double half, double ia, double y2,
-                                              double G, double (&f)[kFN64]) {
-    if (__ballot(cls != 0) == 0ull) return;
+                                              double G, const ChiPiece &chi,
+                                              double (&f)[kFN64]) {
+    if (!P::WINGS || __ballot(cls != 0) == 0ull) return;
     if (cls == 0) { D = 1.0; half = 0.0; ia = 1.0e4; y2 = 0.0; G = 0.0; }
-    if (__ballot(cls == 3)) add_nodes<3>(D, half, ia, y2, G, f);
-    else if (__ballot(cls == 2)) add_nodes<2>(D, half, ia, y2, G, f);
-    else add_nodes<1>(D, half, ia, y2, G, f);
+    if (P::PROFILE == 1 && __ballot(cls == 3)) add_nodes<P, 3>(D, half, ia, y2, G, chi, f);
+    else if (P::PROFILE == 1 && __ballot(cls == 2)) add_nodes<P, 2>(D, half, ia, y2, G, chi, f);
+    else add_nodes<P, 1>(D, half, ia, y2, G, chi, f);
 }
 
 // First index p of [0, n) with !(v[p] < key) (LOWER) or v[p] > key, by one
@@ -299,13 +415,6 @@ __device__ __forceinline__ double cheb_sum64(const double *c, double u) {
     return fma(u, b1, c[0] - b2);
 }
 
-__device__ __forceinline__ double lane_f64(double v, int b) {
-    const long long x = __double_as_longlong(v);
-    const unsigned lo = __builtin_amdgcn_readlane((int)x, b);
-    const unsigned hi = __builtin_amdgcn_readlane((int)(x >> 32), b);
-    return __longlong_as_double(((long long)hi << 32) | lo);
-}
-
 // ---------------------------------------------------------------------------
 // Line core, x^2 + y^2 < 100: the midpoint rule for
 //   w(x + iy) = (i/pi) int e^{-(x+s)^2} / (iy - s) ds
@@ -335,25 +444,6 @@ constexpr double kCE[kCHi + 1] = {
     1, 0.76481841449861865, 0.34216323515981589, 0.089541635567738392, 0.013706714729223335,
     0.0012273216551150678, 6.428358545165617e-05, 1.9695112154195025e-06, 3.5296650648060179e-08,
     3.7002000654827686e-10, 2.2689952580918315e-12, 8.1387674929739835e-15, 1.7076559162725319e-17};
-
-// e^v for |v| <= 0.35 by its Taylor series (first term left out < 3e-18).
-__device__ __forceinline__ double exp_small(double v) {
-    constexpr double c[14] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
-                              1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800,
-                              1.0 / 479001600, 1.0 / 6227020800};
-    double s = local_const(c[13]);
-#pragma unroll
-    for (int k = 12; k >= 2; --k) s = fma(s, v, local_const(c[k]));
-    return fma(fma(s, v, 1.0), v, 1.0);
-}
-
-// e^-t, 0 <= t <= 100 (t = n ln 2 - v in two parts).
-__device__ __forceinline__ double exp_neg(double t) {
-    const double n = rint(t * local_const(1.4426950408889634));
-    double v = fma(n, local_const(0.69314718055994531), -t);
-    v = fma(n, local_const(2.3190468138462996e-17), v);
-    return ldexp(exp_small(v), -(int)n);
-}
 
 // cos(t), 0 <= t <= 130, to ~1e-16 absolute: t = n pi + v in two parts, the
 // Taylor series in v^2 (|v| <= pi/2; first term left out < 2e-17).
@@ -413,34 +503,57 @@ __device__ __forceinline__ double core_value(double x, double y, double G, doubl
 // Point-by-point part of one line on the wave's points: per 64-point segment
 // 2 bits of code, 1: x^2 + y^2 >= 1e4 at all its points (4 nodes), 2: >= 100
 // (8 nodes), 3: some points lie in the line core.
-template <int PPT>
-__device__ __forceinline__ void add_points(uint32_t code, double nu, double ia, double y, double G,
-                                           double Apf, int lo, int hi, bool full, double jd,
-                                           double numin, double dnu, double (&acc)[PPT],
+// Binned Gaussian cell average of exp(-t^2)/sqrt(pi) times vb:
+// (erf(x + h) - erf(x - h)) / 2 with h = vb/2, from the side away from the
+// centre.
+__device__ __forceinline__ double binned_gauss(double x, double h) {
+    return x >= 0.0 ? 0.5 * (erfc(x - h) - erfc(x + h)) : 0.5 * (erfc(-x - h) - erfc(-x + h));
+}
+
+template <class P, int PPT, class Args>
+__device__ __forceinline__ void add_points(const Args &a, uint32_t code, double nu, double ia,
+                                           double y, double G, double Apf, double pl, int lo,
+                                           int hi, bool full, double jd, double (&acc)[PPT],
                                            double *tab) {
     const int lane = threadIdx.x & 63;
-    const double y2 = y * y;
-    if (code & (code >> 1) & 0x55555555u) core_table(tab, y2);
+    const double y2 = y * y, numin = a.numin, dnu = a.dnu;
+    if (P::PROFILE == 1 && code & (code >> 1) & 0x55555555u) core_table(tab, y2);
     for (int k = 0; code != 0; ++k, code >>= 2) {
         const int c = code & 3;
         if (c == 0) continue;
-        const double x = (fma(jd + (double)(64 * k), dnu, numin) - nu) * ia;
+        const double xj = fma(jd + (double)(64 * k), dnu, numin);
+        const double dd = xj - nu;
+        const double x = dd * ia;
         const double x2 = x * x;
         const double r2 = fma(x, x, y2);
         double v = 0.0, num, den;
-        if (c == 1) {
+        if (P::PROFILE == 0) {
+        } else if (P::PROFILE == 2) {
+            v = G / r2;
+        } else if (P::PROFILE == 3) {
+            v = G * exp_neg(fmin(x2, 800.0));
+        } else if (P::PROFILE == 4) {
+            const double vb = dnu * ia;
+            v = G / vb * binned_gauss(x, 0.5 * vb);
+        } else if (c == 1) {
             gh_frac(GH<2>(), x2, r2, num, den);
             v = G * (num * rcp64(den));
         } else if (c == 2 || __ballot(r2 >= kRB64) != 0ull) {
             gh_frac(GH<4>(), x2, r2, num, den);
             v = G * (num * rcp64(den));
         }
-        if (c == 3) {
+        if (P::PROFILE == 1 && c == 3) {
             const double w = core_value(x, y, G, Apf, tab);
             v = r2 < kRB64 ? w : v;
         }
+        if constexpr (P::CHI) {
+            if (xj > a.chi.lo && xj < a.chi.hi)
+                v *= exp_neg(fmin(chi_exponent(a.chi, fabs(dd)), 800.0)) * (xj / nu);
+        }
         if (!full) {
+            // (a line that covers the wave has its plinth in the constants)
             const int j = lane + 64 * k;
+            if (P::PLINTH) v -= pl;
             v = (j >= lo && j < hi) ? v : 0.0;
         }
         // one copy of the code above for all segments: acc is a register
@@ -451,7 +564,7 @@ __device__ __forceinline__ void add_points(uint32_t code, double nu, double ia, 
     }
 }
 
-template <int PPT, class Args>
+template <int PPT, class P, class Args>
 __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *sh) {
     constexpr int W = kThreads * PPT, WP = 64 * PPT;
     const int t = threadIdx.x;
@@ -487,6 +600,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     __syncthreads();
     const int64_t first = sh->range[0], last = sh->range[1];
     bool any_far = false, any_wave = false;
+    double cst = 0.0, wcst = 0.0;          // plinths of lines that cover the tile, the wave
     for (int64_t r0 = first; r0 < last; r0 += kRound64) {
         const int nr = (int)min((int64_t)kRound64, last - r0);
         // tile level: one line per lane; near lines listed per wave
@@ -501,6 +615,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 bool near = false;
                 int cls = 0;
                 double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0;
+                ChiPiece chi;
                 if (e < nr) {
                     const int64_t i = r0 + e;
                     const double nu = a.nu[i], hw = a.hw[i];
@@ -508,17 +623,29 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                     near = hw > 0.0 && dl < hw && dh > -hw;
                     const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
                     D = xc - nu;
-                    if (a.far && near && full && fabs(D) >= kFarRatio64 * hW) {
+                    if constexpr (P::PLINTH) {
+                        if (near && full) cst -= a.pl[i];
+                    }
+                    if (P::PROFILE == 0) {
+                        near = near && !full;
+                    } else if (P::COMPACT) {
+                        ia = a.ia[i];
+                        if (near && !(P::PLINTH && !full) && fabs(a.S[i]) < 1.0e300)
+                            near = (fabs(D) - hW - a.dnu) * ia <= kDopplerEnd;
+                    } else if (a.far && near && full && fabs(D) >= kFarRatio64 * hW) {
                         const double y = a.y[i];
                         ia = a.ia[i];
                         y2 = y * y;
-                        G = a.S[i] * y * (kISqrtPi * 2.0 / kPi);
-                        cls = far_class64(D, hW, ia, y2, G);
+                        G = line_factor<P>(a.S[i], y);
+                        cls = far_class64<P>(D, hW, ia, y2, G);
+                        if constexpr (P::CHI) {
+                            if (cls && !chi_piece(a.chi, xfirst, xlast, nu, D, hW, chi)) cls = 0;
+                        }
                         near = cls == 0;
                     }
                 }
                 used |= __ballot(cls != 0) != 0ull;
-                add_far_lines(cls, D, hW, ia, y2, G, f);
+                add_far_lines<P>(cls, D, hW, ia, y2, G, chi, f);
                 const unsigned long long m = __ballot(near);
                 if (near)
                     sh->list[wave][cnt + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)e;
@@ -552,23 +679,31 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
             for (int c0 = 0; c0 < total; c0 += 64) {
                 int cls = 0;
                 double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0;
-                if (a.far && c0 + lane < total) {
+                ChiPiece chi;
+                if ((a.far || P::PLINTH) && c0 + lane < total) {
                     const int64_t i = line_at(c0 + lane);
                     const double nu = a.nu[i], hw = a.hw[i];
                     const double dl = xwf - nu, dh = xwl - nu;
                     D = xcw - nu;
-                    if (dl > -hw && dl < hw && dh > -hw && dh < hw &&
-                        fabs(D) >= kFarRatio64 * hw_w) {
+                    const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
+                    if constexpr (P::PLINTH) {
+                        const double el = xfirst - nu, eh = xlast - nu;
+                        if (full && !(el > -hw && el < hw && eh > -hw && eh < hw)) wcst -= a.pl[i];
+                    }
+                    if (P::WINGS && a.far && full && fabs(D) >= kFarRatio64 * hw_w) {
                         const double y = a.y[i];
                         ia = a.ia[i];
                         y2 = y * y;
-                        G = a.S[i] * y * (kISqrtPi * 2.0 / kPi);
-                        cls = far_class64(D, hw_w, ia, y2, G);
+                        G = line_factor<P>(a.S[i], y);
+                        cls = far_class64<P>(D, hw_w, ia, y2, G);
+                        if constexpr (P::CHI) {
+                            if (cls && !chi_piece(a.chi, xwf, xwl, nu, D, hw_w, chi)) cls = 0;
+                        }
                     }
                 }
                 unsigned long long wm = __ballot(cls != 0);
                 if (__popcll(wm) >= wave_min_lines(PPT)) {
-                    add_far_lines(cls, D, hw_w, ia, y2, G, f);
+                    add_far_lines<P>(cls, D, hw_w, ia, y2, G, chi, f);
                     used = true;
                 } else wm = 0ull;
                 if (lane == 0) sh->taken[wave][c0 >> 6] = wm;
@@ -581,32 +716,50 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
             const int e = c0 + lane;
             uint32_t code = 0;
             int lo = 0, hi = 0;
-            double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0;
+            double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0, pl = 0.0;
             if (e < total && !((sh->taken[wave][c0 >> 6] >> lane) & 1ull)) {
                 const int64_t i = line_at(e);
                 nu = a.nu[i];
                 clip_window(nu, a.hw[i], a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
                 if (lo < hi) {
-                    const double A = a.S[i] * kISqrtPi;
+                    const double S = a.S[i];
                     y = a.y[i];
                     ia = a.ia[i];
-                    G = A * y * (2.0 / kPi);
-                    // conservative point intervals with x^2 + y^2 < 100, 1e4
-                    const float vb = (float)(a.dnu * ia), fy2 = (float)(y * y);
-                    const float cen = (float)((nu - xwf) * inv_dnu);
-                    const float r1 = sqrtf(fmaxf(1.0002e2f - fy2, 0.0f)) / vb;
-                    const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
-                    const float mg = 2.0f + 1.0e-5f * fabsf(cen);
-                    const bool in1 = fy2 < 1.0002e2f, in2 = fy2 < 1.0002e4f;
+                    G = line_factor<P>(S, y);
+                    if constexpr (P::PLINTH) pl = a.pl[i];
+                    if constexpr (P::PROFILE == 1) {
+                        // conservative point intervals with x^2 + y^2 < 100, 1e4
+                        const float vb = (float)(a.dnu * ia), fy2 = (float)(y * y);
+                        const float cen = (float)((nu - xwf) * inv_dnu);
+                        const float r1 = sqrtf(fmaxf(1.0002e2f - fy2, 0.0f)) / vb;
+                        const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
+                        const float mg = 2.0f + 1.0e-5f * fabsf(cen);
+                        const bool in1 = fy2 < 1.0002e2f, in2 = fy2 < 1.0002e4f;
 #pragma unroll
-                    for (int k = 0; k < PPT; ++k) {
-                        const int s0 = 64 * k, s1 = s0 + 63;
-                        if (lo > s1 || hi <= s0) continue;
-                        const bool c3 = in1 && cen - r1 - mg <= (float)s1 && cen + r1 + mg >= (float)s0;
-                        const bool c2 = in2 && cen - r2 - mg <= (float)s1 && cen + r2 + mg >= (float)s0;
-                        code |= (c3 ? 3u : c2 ? 2u : 1u) << (2 * k);
+                        for (int k = 0; k < PPT; ++k) {
+                            const int s0 = 64 * k, s1 = s0 + 63;
+                            if (lo > s1 || hi <= s0) continue;
+                            const bool c3 = in1 && cen - r1 - mg <= (float)s1 && cen + r1 + mg >= (float)s0;
+                            const bool c2 = in2 && cen - r2 - mg <= (float)s1 && cen + r2 + mg >= (float)s0;
+                            code |= (c3 ? 3u : c2 ? 2u : 1u) << (2 * k);
+                        }
+                        if (code & (code >> 1) & 0x55555555u) Apf = S * kISqrtPi * core_pole(y);
+                    } else {
+                        // segments that the window touches; a compact profile's
+                        // only where it is not zero, unless a plinth is there
+                        int l = lo, h = hi;
+                        const bool part = P::PROFILE == 0 || (P::PLINTH && (lo > 0 || hi < nw));
+                        if (P::COMPACT && !part && fabs(S) < 1.0e300) {
+                            const double off = (nu - xwf) * inv_dnu;
+                            const double w = kDopplerEnd / ia * inv_dnu + 2.0;
+                            l = max(lo, (int)fmin(fmax(off - w, 0.0), (double)nw));
+                            h = min(hi, (int)fmin(fmax(off + w, 0.0), (double)nw));
+                        }
+                        if (P::PROFILE != 0 || part)
+#pragma unroll
+                            for (int k = 0; k < PPT; ++k)
+                                if (l < 64 * k + 64 && h > 64 * k && l < h) code |= 1u << (2 * k);
                     }
-                    if (code & (code >> 1) & 0x55555555u) Apf = A * core_pole(y);
                 }
             }
             unsigned long long m = __ballot(code != 0);
@@ -614,18 +767,30 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 const int b = __builtin_ctzll(m);
                 m &= m - 1ull;
                 const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
-                add_points<PPT>((uint32_t)__builtin_amdgcn_readlane((int)code, b), lane_f64(nu, b),
-                                lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b), lane_f64(Apf, b),
-                                slo, shi, slo == 0 && shi == nw, jd, a.numin, a.dnu, acc,
-                                sh->tab[wave]);
+                add_points<P, PPT>(a, (uint32_t)__builtin_amdgcn_readlane((int)code, b),
+                                   lane_f64(nu, b), lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b),
+                                   P::PROFILE == 1 ? lane_f64(Apf, b) : 0.0,
+                                   P::PLINTH ? lane_f64(pl, b) : 0.0, slo, shi,
+                                   slo == 0 && shi == nw, jd, acc, sh->tab[wave]);
             }
         }
         __syncthreads();      // the lists are free for the next round
     }
     // node sums -> one series per wave.  any_far differs between waves: the
     // tile's totals are taken whenever any wave has some.
+    if (P::PLINTH) {
+        const double c = wave_total64(cst);
+        if (lane == 0) sh->cst[wave] = c;
+    }
     const bool tile_far = __syncthreads_or(any_far) != 0;
     if (nw == 0) return;
+    if (P::PLINTH) {
+        double c = wave_total64(wcst);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) c += sh->cst[w];
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) acc[k] += c;
+    }
     if (tile_far || any_wave) {
         double *c = sh->c[wave], *wF = sh->wF[wave];
         if (tile_far) {
@@ -657,6 +822,10 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
         const int64_t j = jw + lane + 64 * k;
+        if constexpr (P::CHI) {
+            const double x = fma(jd + (double)(64 * k), a.dnu, a.numin);
+            if (a.side != 0 && (x > a.lo && x < a.hi) != (a.side > 0)) continue;
+        }
         if (j < a.nx) a.K[j] = a.accumulate ? a.K[j] + acc[k] : a.kmin + acc[k];
     }
 }
