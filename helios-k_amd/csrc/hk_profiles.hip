@@ -42,9 +42,6 @@ namespace {
 
 using namespace hk;
 
-constexpr int kPPT = 4;              // points per thread
-constexpr int kPW = kThreads * kPPT; // points per tile
-
 __device__ __forceinline__ double prefactor(int profile, double S, double y) {
     if (profile == 2) return S * y / kPi;
     if (profile == 3 || profile == 1) return S * kISqrtPi;
@@ -85,7 +82,7 @@ struct PArgs {
 
 // PROFILE 1..4: profile sums (minus plinths when PLINTH); PROFILE 0: the
 // plinth subtraction alone (after an FP32C or compat Voigt sum).
-template <int PROFILE, bool PLINTH, bool CHI>
+template <int PPT, int PROFILE, bool PLINTH, bool CHI>
 __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
     __shared__ Far64LDS sh;
     if constexpr (CHI) {
@@ -93,9 +90,9 @@ __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
         // lay inside and then outside: the factor is smooth over each.  (Summed
         // point by point instead, the two such tiles of a 1e5-point grid took
         // 8.1 ms, the other 96 together 1.1.)
-        const int64_t j0 = (int64_t)blockIdx.x * kPW;
+        const int64_t j0 = (int64_t)blockIdx.x * kThreads * PPT;
         const double x0 = fma((double)j0, a.dnu, a.numin);
-        const double x1 = fma((double)min(j0 + kPW, a.nx) - 1.0, a.dnu, a.numin);
+        const double x1 = fma((double)min(j0 + kThreads * PPT, a.nx) - 1.0, a.dnu, a.numin);
         const bool cut = (x0 <= a.lo && x1 > a.lo) || (x0 < a.hi && x1 >= a.hi);
         for (int pass = 0; pass < (cut ? 2 : 1); ++pass) {
             if (cut) {
@@ -104,23 +101,25 @@ __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
                 a.chi.hi = -a.chi.lo;
                 __syncthreads();
             }
-            tile_f64<kPPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
+            tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
         }
     } else {
-        tile_f64<kPPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
+        tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
     }
 }
 
 template <int PROFILE, bool PLINTH, bool CHI = false>
-void launch_profile(int64_t ntiles, hipStream_t s, const PArgs &a) {
-    hipLaunchKernelGGL((profile_tiles_kernel<PROFILE, PLINTH, CHI>), dim3((unsigned)ntiles),
-                       dim3(kThreads), 0, s, a);
+void launch_profile(hipStream_t s, const PArgs &a) {
+    const int ppt = default_ppt64(a.nx);
+    const dim3 g((unsigned)((a.nx + kThreads * ppt - 1) / (kThreads * ppt))), b(kThreads);
+    if (ppt == 1) hipLaunchKernelGGL((profile_tiles_kernel<1, PROFILE, PLINTH, CHI>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((profile_tiles_kernel<2, PROFILE, PLINTH, CHI>), g, b, 0, s, a);
 }
 
 template <int PROFILE>
-void launch_chi(bool plinth, int64_t ntiles, hipStream_t s, const PArgs &a) {
-    if (plinth) launch_profile<PROFILE, true, true>(ntiles, s, a);
-    else launch_profile<PROFILE, false, true>(ntiles, s, a);
+void launch_chi(bool plinth, hipStream_t s, const PArgs &a) {
+    if (plinth) launch_profile<PROFILE, true, true>(s, a);
+    else launch_profile<PROFILE, false, true>(s, a);
 }
 
 size_t region_bytes(const hk_grid *g) {
@@ -179,7 +178,6 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
                            st->S, st->ialphaD, st->y, st->hw, n, profile, pl);
         HK_LAUNCH_CHECK();
     }
-    const int64_t ntiles = (grid->nx + kPW - 1) / kPW;
     PArgs a;
     a.nu = st->nu; a.S = st->S; a.ia = st->ialphaD; a.y = st->y; a.hw = st->hw; a.pl = pl;
     a.key = st->key; a.radius = st->radius;
@@ -195,25 +193,25 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
         a.lo = a.chi.lo;
         a.hi = a.chi.hi;
         switch (profile) {
-        case HK_PROFILE_VOIGT: launch_chi<1>(P, ntiles, s, a); break;
-        case HK_PROFILE_LORENTZ: launch_chi<2>(P, ntiles, s, a); break;
-        case HK_PROFILE_DOPPLER: launch_chi<3>(P, ntiles, s, a); break;
-        default: launch_profile<4, false, true>(ntiles, s, a); break;
+        case HK_PROFILE_VOIGT: launch_chi<1>(P, s, a); break;
+        case HK_PROFILE_LORENTZ: launch_chi<2>(P, s, a); break;
+        case HK_PROFILE_DOPPLER: launch_chi<3>(P, s, a); break;
+        default: launch_profile<4, false, true>(s, a); break;
         }
         HK_LAUNCH_CHECK();
         return HK_OK;
     }
     switch (profile) {
     case HK_PROFILE_VOIGT:
-        voigt_sum ? launch_profile<0, true>(ntiles, s, a) : launch_profile<1, true>(ntiles, s, a);
+        voigt_sum ? launch_profile<0, true>(s, a) : launch_profile<1, true>(s, a);
         break;
     case HK_PROFILE_LORENTZ:
-        P ? launch_profile<2, true>(ntiles, s, a) : launch_profile<2, false>(ntiles, s, a);
+        P ? launch_profile<2, true>(s, a) : launch_profile<2, false>(s, a);
         break;
     case HK_PROFILE_DOPPLER:
-        P ? launch_profile<3, true>(ntiles, s, a) : launch_profile<3, false>(ntiles, s, a);
+        P ? launch_profile<3, true>(s, a) : launch_profile<3, false>(s, a);
         break;
-    default: launch_profile<4, false>(ntiles, s, a); break;
+    default: launch_profile<4, false>(s, a); break;
     }
     HK_LAUNCH_CHECK();
     return HK_OK;

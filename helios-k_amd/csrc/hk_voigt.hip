@@ -1582,15 +1582,21 @@ using namespace hk;
 
 namespace {
 
-int pick_ppt(int mode, const hk_tune *tune) {
-    // defaults: 1024-point tiles for both forms (with the FP32 far field,
-    // smaller tiles trade direct pairs for node evaluations; 1024 was
-    // fastest at 1e7 lines x 3e7 points)
-    int tp = tune && tune->tile_points > 0 ? tune->tile_points : 1024;
-    return tp / kThreads;
+// Points per thread of the main pass's tiles: the caller's choice, or
+//  FP32C  1024-point tiles (smaller ones trade direct pairs for node
+//         evaluations; 1024 was fastest at 1e7 lines x 3e7 points);
+//  FP64   default_ppt64.
+int pick_ppt(int mode, const hk_tune *tune, int64_t nx) {
+    if (tune && tune->tile_points > 0) return tune->tile_points / kThreads;
+    return mode == HK_VOIGT_FP64 ? default_ppt64(nx) : 4;
 }
 
-bool ppt_ok(int ppt) { return ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16; }
+// tile_points a caller may ask for: 512, 1024, 2048 or 4096 (256-point tiles
+// are FP64's own choice for short grids).
+bool tile_points_ok(int mode, const hk_tune *tune, int ppt) {
+    if (!(tune && tune->tile_points > 0)) return true;
+    return (ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16);
+}
 
 // Lines per LDS stage of the main pass: 256 (default) or 512; returns the
 // multiple of kThreads, 0 when the request is not one of those.
@@ -1603,6 +1609,7 @@ template <int MODE, int LM>
 void launch_tiles_lm(int ppt, int64_t ntiles, hipStream_t s, const VArgs &a) {
     dim3 g((unsigned)ntiles), b(kThreads);
     switch (ppt) {
+        case 1: hipLaunchKernelGGL((voigt_tiles_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, a); break;
         case 2: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 2, LM>), g, b, 0, s, a); break;
         case 4: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 4, LM>), g, b, 0, s, a); break;
         case 8: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 8, LM>), g, b, 0, s, a); break;
@@ -1621,6 +1628,7 @@ void launch_persistent_lm(int ppt, unsigned grid, hipStream_t s, const VArgs *sp
                           const int64_t *item_start, int nspec, unsigned long long *counter) {
     dim3 g(grid), b(kThreads);
     switch (ppt) {
+        case 1: hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, specs, item_start, nspec, counter); break;
         case 2: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 2, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
         case 4: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 4, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
         case 8: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 8, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
@@ -1674,8 +1682,8 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
                  "hk_voigt_accumulate: mode %d", mode);
     if (int e = check_state(st, "hk_voigt_accumulate")) return e;
     if (int e = check_grid(grid, "hk_voigt_accumulate")) return e;
-    const int ppt = pick_ppt(mode, tune);
-    HK_CHECK_ARG(ppt_ok(ppt), "hk_voigt_accumulate: tile_points must be 512, 1024, 2048 or 4096");
+    const int ppt = pick_ppt(mode, tune, grid->nx);
+    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_accumulate: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_accumulate: stage_lines must be 256 or 512");
     if (ws_bytes < hk_voigt_workspace_bytes(grid, tune)) {
@@ -1778,10 +1786,11 @@ namespace {
 struct BatchLayout {
     size_t off_args, off_cargs, off_items, off_citems, off_counter, total;
     std::vector<size_t> tile_off, ctile_off;
-    std::vector<int64_t> ntiles, ncore;
+    std::vector<int64_t> ncore;
 };
 
 BatchLayout batch_layout(int nspec, const hk_spectrum *spec, int W) {
+    W = std::max(W, 512);       // (FP64 tiles, 256 points the smallest, have no table)
     BatchLayout L;
     size_t o = 0;
     L.off_args = o; o = align_up(o + sizeof(VArgs) * nspec, 256);
@@ -1792,7 +1801,6 @@ BatchLayout batch_layout(int nspec, const hk_spectrum *spec, int W) {
     for (int i = 0; i < nspec; ++i) {
         const int64_t nt = (spec[i].grid.nx + W - 1) / W;
         const int64_t nc = (spec[i].grid.nx + kCoreW - 1) / kCoreW;
-        L.ntiles.push_back(nt);
         L.ncore.push_back(nc);
         L.tile_off.push_back(o);
         o = align_up(o + sizeof(TileInfo) * nt, 256);
@@ -1825,8 +1833,11 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
     HK_CHECK_ARG(nspec > 0 && spec && ws && batch, "hk_voigt_batched_prepare: bad arguments");
     HK_CHECK_ARG(mode == HK_VOIGT_FP64 || mode == HK_VOIGT_FP32C,
                  "hk_voigt_batched_prepare: mode %d", mode);
-    const int ppt = pick_ppt(mode, tune);
-    HK_CHECK_ARG(ppt_ok(ppt), "hk_voigt_batched_prepare: tile_points must be 512, 1024, 2048 or 4096");
+    // one tile width for the batch: that of its longest grid
+    int64_t longest = 0;
+    for (int i = 0; i < nspec; ++i) longest = std::max(longest, spec[i].grid.nx);
+    const int ppt = pick_ppt(mode, tune, longest);
+    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_batched_prepare: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_batched_prepare: stage_lines must be 256 or 512");
     for (int i = 0; i < nspec; ++i) {
@@ -1866,7 +1877,7 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
         cargs[q] = a;
         cargs[q].radius = sp.st.radius + 1;
         cargs[q].tiles = (TileInfo *)(base + L.ctile_off[i]);
-        items[q + 1] = items[q] + L.ntiles[i];
+        items[q + 1] = items[q] + (sp.grid.nx + W - 1) / W;
         citems[q + 1] = citems[q] + L.ncore[i];
     }
     hipStream_t s = (hipStream_t)stream;
@@ -1898,7 +1909,8 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
                  "hk_voigt_batched_launch: batch not prepared");
     const int ppt = batch->tile_points / kThreads;
     const int lm = batch->stage_lines / kThreads;
-    HK_CHECK_ARG(ppt_ok(ppt) && (lm == 1 || lm == 2) &&
+    HK_CHECK_ARG((ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16 ||
+                  (ppt == 1 && batch->mode == HK_VOIGT_FP64)) && (lm == 1 || lm == 2) &&
                      (batch->mode == HK_VOIGT_FP64 || batch->mode == HK_VOIGT_FP32C),
                  "hk_voigt_batched_launch: batch not prepared");
     char *base = (char *)batch->workspace;
@@ -2054,8 +2066,8 @@ extern "C" int hk_voigt_work_count(const hk_line_state *st, const hk_grid *grid,
                  mode);
     if (int e = check_state(st, "hk_voigt_work_count")) return e;
     if (int e = check_grid(grid, "hk_voigt_work_count")) return e;
-    const int ppt = pick_ppt(mode, tune);
-    HK_CHECK_ARG(ppt_ok(ppt), "hk_voigt_work_count: tile_points must be 512, 1024, 2048 or 4096");
+    const int ppt = pick_ppt(HK_VOIGT_FP32C, tune, grid->nx);
+    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_work_count: tile_points must be 512, 1024, 2048 or 4096");
     const int far = (mode == HK_VOIGT_FP32C && !(tune && tune->exact_pairs)) ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(zero12_kernel, dim3(1), dim3(64), 0, s, counts);

@@ -47,6 +47,16 @@ constexpr double kU64[kFN64 / 2] = {0.99691733373312796, 0.97236992039767667, 0.
                                     0.85264016435409218, 0.76040596560003093, 0.64944804833018377,
                                     0.52249856471594880, 0.38268343236508984, 0.23344536385590542,
                                     0.078459095727844999};
+// Points per thread of a tile (256 threads) when the caller leaves it open.
+// Halving the tile doubles the tile-level node evaluations and halves the point
+// sums; 512 points win over 1024 at 1e5 lines, 3e6 points, cut 100 (491 against
+// 520 us), 5e6 lines (15.2 / 20.4 ms) and 3.3e5 lines, 1e6 points (0.98 / 1.34
+// ms), and cost 3 % at 2.35e6 lines, 7e6 points, cut 25 on a 0.001 cm^-1 grid.
+// Grids of fewer than four 512-point tiles per CU take 256-point tiles: 1e4
+// points 73 against 106 us, 3e4 points under 1e5 lines 1.12 / 1.97 ms, 3e5
+// points 665 / 805 us; at 1e6 points the two are equal.
+inline int default_ppt64(int64_t nx) { return (nx + 511) / 512 < 1024 ? 1 : 2; }
+
 // lines taken per round of the tile loop (each wave lists its own quarter)
 constexpr int kRound64 = 4096;
 // a chunk of 64 lines goes through the wave's nodes when at least this many

@@ -88,3 +88,24 @@ def test_fp64_non_finite_strength_stays_in_its_window():
         assert not torch.isfinite(K2[inside]).any()
         a, b = K2[~inside], K[~inside]
         assert torch.isfinite(a).all() and float(((a - b).abs() / b.clamp(min=1e-40)).max()) <= 1e-13
+
+
+@pytest.mark.gpu
+def test_fp64_batch_takes_one_tile_width():
+    """A batch of a short and a long grid (one tile width for both) against
+    the single sums (each grid's own), and a batch of short grids bit for bit."""
+    import torch
+    from heliosk import engine as E
+    d = random_lines(400, seed=8, numin=1000.0, numax=1060.0)
+    st = E.line_params(species_from(d), 900.0, 0.5, Q=d["iso_Q"], cut_mode=0, cut=5.0)
+    grids = [E.make_grid(1001.0, 1004.0, 0.001), E.make_grid(1000.0, 1060.0, 1e-4)]
+    assert grids[1].nx > 1024 * 512 > grids[0].nx
+    K = [torch.empty(g.nx, dtype=torch.float64, device="cuda") for g in grids]
+    E.voigt_batched([(st, g, 0.0, k) for g, k in zip(grids, K)], mode=E.HK_VOIGT_FP64)
+    for g, k in zip(grids, K):
+        assert rel_err(k.cpu().numpy(), E.voigt(st, g, 0.0, E.HK_VOIGT_FP64).cpu().numpy()) <= 1e-13
+    short = torch.empty_like(K[0])
+    E.voigt_batched([(st, grids[0], 0.0, short)], mode=E.HK_VOIGT_FP64)
+    assert torch.equal(short, E.voigt(st, grids[0], 0.0, E.HK_VOIGT_FP64))
+    with pytest.raises(Exception, match="tile_points"):
+        E.voigt(st, grids[0], 0.0, E.HK_VOIGT_FP64, tile_points=256)
