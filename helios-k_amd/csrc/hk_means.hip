@@ -25,6 +25,7 @@
 
 #include "hk_device.h"
 #include "hk_internal.h"
+#include "hk_voigt64.h"
 
 namespace {
 
@@ -116,53 +117,244 @@ __global__ __launch_bounds__(kMeanThreads) void means_final_kernel(
     if (t < 4) sums[t] = s[t][0];
 }
 
-constexpr int kTrThreads = 256;
-constexpr int kTrM = 8;               // m values per workgroup
+constexpr int kTrThreads = 512;
+constexpr int kTrWaves = kTrThreads / 64;
+constexpr int kTrGroups = 1;                 // groups of 16 m values per wave
+constexpr int kTrPer = kTrWaves * kTrGroups * 16;   // m values per workgroup
+constexpr int kTrC = 128;                    // points per cluster
+constexpr int kTrBatch = 128;                // clusters in LDS at a time
+constexpr int kTrSuper = 16;                 // clusters per super-cluster
+// Largest half width of a cluster times m that its nodes may stand for: 20
+// Chebyshev nodes leave 2 I_20(3) = 2e-15 of e^{-K m} at the cluster's least K.
+constexpr double kTrNodes = 3.0;
+// e^-t is 0 from t = 745.2 on.
+constexpr double kTrZero = 746.0;
+// A cluster whose terms are all below e^-50 of the bin's largest adds less than
+// a rounding (1e-18 of the sum for 1e4 points).
+constexpr double kTrNone = 50.0;
 
-// grid (ceil(nTr / kTrM), nbins): one workgroup sums kTrM transmission
-// points of one bin; K of the bin is read once per workgroup (coalesced).
-__global__ __launch_bounds__(kTrThreads) void transmission_kernel(
+// e^-t (t clamped where the result is 0 or infinite).
+__device__ __forceinline__ double tr_exp(double t) {
+    t = t > 800.0 ? 800.0 : t;
+    return hk::exp_neg(t < -800.0 ? -800.0 : t);
+}
+
+// Minimum of v over the wave, in every lane.
+__device__ __forceinline__ double wave_min64(double v) {
+    v = fmin(v, hk::row_dpp64<0xb1>(v));
+    v = fmin(v, hk::row_dpp64<0x4e>(v));
+    v = fmin(v, hk::row_dpp64<0x141>(v));
+    v = fmin(v, hk::row_dpp64<0x140>(v));
+    return fmin(fmin(hk::lane_f64(v, 0), hk::lane_f64(v, 16)),
+                fmin(hk::lane_f64(v, 32), hk::lane_f64(v, 48)));
+}
+
+struct TrCluster {
+    double lo, half;
+    int n, nodes;            // points; whether the nodes may stand for them
+};
+
+// One workgroup sums up to kTrPer transmission points of one bin.  The bin is
+// taken in clusters of kTrC consecutive values: e^{-K m} is entire in K, so over
+// a cluster whose half width h has h m <= 3 the sum over its values is that over
+// 20 Chebyshev nodes with the values' Lagrange weights, whatever m; a cluster
+// too wide for an m is summed value by value, and one with nothing left to add
+// is skipped.  Sixteen clusters make a super-cluster, whose nodes stand for them
+// where they are narrow enough for the m.  The waves make the clusters of a batch together, then each takes
+// its m values, 16 at a time and four lanes each, without waiting for the
+// others.  A cluster's range is its values' own, so bins that are not sorted
+// are summed too, more slowly.
+// Bound by FP64 vector instructions (300 bins of 1e4 points, 300 m: one
+// exponential per point and m took 724 us, this 273).
+__global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     const double *__restrict__ Ks, int Nxb, const int32_t *__restrict__ nxmin, double kmin,
     int nTr, double dTr, double *__restrict__ Tr) {
-    __shared__ double s[kTrM][kTrThreads];
+    using namespace hk;
+    __shared__ double Gp[kFN64 / 4][kTrBatch][4];     // node weights, node 4k + part
+    __shared__ double Mw[kTrWaves][3 * kFN64];
+    __shared__ TrCluster cl[kTrBatch], sc[kTrBatch / kTrSuper];
+    __shared__ double Gs[kTrBatch / kTrSuper][kFN64];
+    __shared__ double cosv[4 * kFN64];
+    __shared__ double red[kTrWaves];
     const int b = blockIdx.y;
-    const int t0 = blockIdx.x * kTrM;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, part = tid & 3;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const double *Kb = Ks + (size_t)b * Nxb;
-    double m[kTrM], a[kTrM];
+    // this lane's m of group g: t0 + 16 (wave + 8 g) + lane / 4
+    const int t0 = blockIdx.x * kTrPer + 16 * wave + (lane >> 2);
+    auto m_of = [&](int g) { return exp((double)(t0 + 16 * kTrWaves * g - nTr / 2) * dTr); };
+    if (tid < 4 * kFN64) cosv[tid] = cospi((double)tid / (2.0 * kFN64));
+    double least = INFINITY;
+    for (int k = tid; k < Nxb; k += kTrThreads) least = fmin(least, Kb[k]);
+    least = wave_min64(least);
+    if (lane == 0) red[wave] = least;
+    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < kTrM; ++q) {
-        m[q] = exp((double)(t0 + q - nTr / 2) * dTr);
-        a[q] = 0.0;
-    }
-    for (int k = tid; k < Nxb; k += kTrThreads) {
-        const double kv = Kb[k];
+    for (int w = 0; w < kTrWaves; ++w) least = fmin(least, red[w]);
+    double acc[kTrGroups];
 #pragma unroll
-        for (int q = 0; q < kTrM; ++q) a[q] += exp(-kv * m[q]);
-    }
-    if (tid < 3) {
-        const double w[3] = {-5.0 / 8.0, 1.0 / 6.0, -1.0 / 24.0};
-        const double klo = Kb[tid], khi = Kb[Nxb - 1 - tid];
+    for (int g = 0; g < kTrGroups; ++g) acc[g] = 0.0;
+    double un[kFN64 / 4];                  // (K - lo) / half at this lane's nodes
 #pragma unroll
-        for (int q = 0; q < kTrM; ++q) {
-            a[q] += w[tid] * exp(-klo * m[q]);
-            a[q] += w[2 - tid] * exp(-khi * m[q]);
+    for (int k = 0; k < kFN64 / 4; ++k)
+        un[k] = 1.0 + cospi((2.0 * (4 * k + part) + 1.0) / (2.0 * kFN64));
+    for (int k0 = 0; k0 < Nxb; k0 += kTrC * kTrBatch) {
+        const int ncl = min(kTrBatch, (Nxb - k0 + kTrC - 1) / kTrC);
+        __syncthreads();                    // the previous batch's readers are done
+        // three at a time: their node weights come from 60 lanes together
+        for (int c3 = wave * 3; c3 < ncl; c3 += kTrWaves * 3) {
+            double *M = Mw[wave];
+            wave_lds_sync();
+            if (lane < 3 * kFN64) M[lane] = 0.0;
+            wave_lds_sync();
+            for (int c = c3; c < min(c3 + 3, ncl); ++c) {
+                // range and moments
+                const int first = k0 + c * kTrC, n = min(kTrC, Nxb - first);
+                double v[kTrC / 64];
+                double lo = INFINITY, hi = -INFINITY;
+                bool fin = true;
+#pragma unroll
+                for (int q = 0; q < kTrC / 64; ++q) {
+                    const int k = lane + 64 * q;
+                    v[q] = k < n ? Kb[first + k] : 0.0;
+                    if (k < n) {
+                        lo = fmin(lo, v[q]);
+                        hi = fmax(hi, v[q]);
+                        fin &= fabs(v[q]) < 1.0e300;
+                    }
+                }
+                lo = wave_min64(lo);
+                hi = -wave_min64(-hi);
+                const bool nodes = __ballot(!fin) == 0ull;
+                const double half = 0.5 * (hi - lo), mid = 0.5 * (hi + lo);
+                if (nodes) {
+                    double f[kFN64];
+#pragma unroll
+                    for (int q = 0; q < kFN64; ++q) f[q] = 0.0;
+                    const double ih = half > 0.0 ? 1.0 / half : 0.0;
+#pragma unroll
+                    for (int q = 0; q < kTrC / 64; ++q)
+                        add_moments20(lane + 64 * q < n ? 1.0 : 0.0, (v[q] - mid) * ih, f);
+                    add_node_totals(f, M + (c - c3) * kFN64);
+                }
+                // (a cluster with undefined or infinite values is never skipped)
+                if (lane == 0) cl[c] = TrCluster{nodes ? lo : -INFINITY, half, n, nodes ? 1 : 0};
+            }
+            wave_lds_sync();
+            const int c = c3 + lane / kFN64, k = lane % kFN64;
+            if (lane < 3 * kFN64 && c < ncl)
+                Gp[k >> 2][c][k & 3] = node_weight(M + lane / kFN64 * kFN64, cosv, k);
+        }
+        __syncthreads();
+        // super-clusters, from the nodes of their clusters
+        const int nsc = (ncl + kTrSuper - 1) / kTrSuper;
+        for (int h = wave; h < nsc; h += kTrWaves) {
+            const int c0 = h * kTrSuper, nc = min(kTrSuper, ncl - c0);
+            double lo = INFINITY, hi = -INFINITY;
+            int ok = 1;
+            for (int c = c0; c < c0 + nc; ++c) {
+                lo = fmin(lo, cl[c].lo);
+                hi = fmax(hi, fma(2.0, cl[c].half, cl[c].lo));
+                ok &= cl[c].nodes;
+            }
+            const double half = 0.5 * (hi - lo), mid = 0.5 * (hi + lo);
+            if (ok) {
+                double f[kFN64];
+#pragma unroll
+                for (int q = 0; q < kFN64; ++q) f[q] = 0.0;
+                const double ih = half > 0.0 ? 1.0 / half : 0.0;
+                for (int q = lane; q < kTrSuper * kFN64; q += 64) {
+                    const int c = c0 + min(q / kFN64, nc - 1), k = q % kFN64;
+                    const double K = fma(cl[c].half, 1.0 + cosv[2 * k + 1], cl[c].lo);
+                    add_moments20(q / kFN64 < nc ? Gp[k >> 2][c][k & 3] : 0.0, (K - mid) * ih, f);
+                }
+                double *M = Mw[wave];
+                wave_lds_sync();
+                if (lane < kFN64) M[lane] = 0.0;
+                wave_lds_sync();
+                add_node_totals(f, M);
+                wave_lds_sync();
+                if (lane < kFN64) Gs[h][lane] = node_weight(M, cosv, lane);
+            }
+            if (lane == 0) sc[h] = TrCluster{lo, half, 0, ok};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < kTrGroups; ++g) {
+            if (blockIdx.x * kTrPer + 16 * (wave + kTrWaves * g) >= nTr) break;
+            const double m = m_of(g);
+            double a = acc[g];
+            // e^{-lo m} (the product's rounding, eps lo m of the value, put
+            // back) times the nodes' e^{-(K - lo) m}, argument <= 6
+            auto by_nodes = [&](const TrCluster &q, const double (&w)[kFN64 / 4]) {
+                const double hm = fmin(q.half * m, kTrNodes);
+                double v = 0.0;
+#pragma unroll
+                for (int k = 0; k < kFN64 / 4; ++k) v = fma(w[k], exp_neg(un[k] * hm), v);
+                const double p = q.lo * m, e = fma(q.lo, m, -p);
+                return v * (tr_exp(p) * (1.0 - e));
+            };
+            auto none = [&](const TrCluster &q) {
+                return (q.lo - least) * m > kTrNone || q.lo * m > kTrZero;
+            };
+            double w[kFN64 / 4];
+            for (int h = 0; h < nsc; ++h) {
+                const TrCluster s = sc[h];
+                const bool off = none(s), whole = s.nodes && s.half * m <= kTrNodes;
+                if (__ballot(!off && whole) != 0ull) {
+#pragma unroll
+                    for (int k = 0; k < kFN64 / 4; ++k) w[k] = Gs[h][4 * k + part];
+                    const double v = by_nodes(s, w);
+                    a += !off && whole ? v : 0.0;
+                }
+                const bool rest = !off && !whole;
+                if (__ballot(rest) == 0ull) continue;
+                for (int c = h * kTrSuper; c < min(ncl, (h + 1) * kTrSuper); ++c) {
+                    const TrCluster q = cl[c];
+                    const bool in = rest && !none(q), nodes = q.nodes && q.half * m <= kTrNodes;
+                    if (__ballot(in && nodes) != 0ull) {
+#pragma unroll
+                        for (int k = 0; k < kFN64 / 4; ++k) w[k] = Gp[k][c][part];
+                        const double v = by_nodes(q, w);
+                        a += in && nodes ? v : 0.0;
+                    }
+                    if (__ballot(in && !nodes) != 0ull) {
+                        const double *Kc = Kb + k0 + c * kTrC;
+                        double v[kTrC / 64];
+#pragma unroll
+                        for (int i = 0; i < kTrC / 64; ++i)
+                            v[i] = lane + 64 * i < q.n ? Kc[lane + 64 * i] : INFINITY;
+                        double t = 0.0;
+#pragma unroll
+                        for (int i = 0; i < kTrC / 64; ++i)
+                            for (int k = part; k < 64; k += 4) {
+                                const double kv = __shfl(v[i], k, 64);
+                                t += kv < INFINITY || !(kv == kv) ? tr_exp(kv * m) : 0.0;
+                            }
+                        a += in && !nodes ? t : 0.0;
+                    }
+                }
+            }
+            acc[g] = a;
         }
     }
+    const double nmin = nxmin ? (double)nxmin[b] : 0.0, nb = (double)Nxb;
 #pragma unroll
-    for (int q = 0; q < kTrM; ++q) s[q][tid] = a[q];
-    __syncthreads();
-    for (int h = kTrThreads / 2; h > 0; h >>= 1) {
-        if (tid < h)
-#pragma unroll
-            for (int q = 0; q < kTrM; ++q) s[q][tid] += s[q][tid + h];
-        __syncthreads();
-    }
-    if (tid < kTrM && t0 + tid < nTr) {
-        const double nmin = nxmin ? (double)nxmin[b] : 0.0;
-        const double nb = (double)Nxb;
-        Tr[(size_t)b * nTr + t0 + tid] =
-            s[tid][0] / (nb - 1.0) * (nb - nmin) / nb + exp(-kmin * m[tid]) * nmin / nb;
+    for (int g = 0; g < kTrGroups; ++g) {
+        const int ti = t0 + 16 * kTrWaves * g;
+        if (blockIdx.x * kTrPer + 16 * (wave + kTrWaves * g) >= nTr) break;
+        const double m = m_of(g);
+        double a = acc[g];
+        if (part < 3) {                     // Simpson end weights, a term per lane
+            const double w[3] = {-5.0 / 8.0, 1.0 / 6.0, -1.0 / 24.0};
+            a = fma(part == 0 ? w[0] : part == 1 ? w[1] : w[2], tr_exp(Kb[part] * m), a);
+            a = fma(part == 0 ? w[2] : part == 1 ? w[1] : w[0], tr_exp(Kb[Nxb - 1 - part] * m), a);
+        }
+        a += __shfl_xor(a, 1, 64);
+        a += __shfl_xor(a, 2, 64);
+        if (part == 0 && ti < nTr)
+            Tr[(size_t)b * nTr + ti] =
+                a / (nb - 1.0) * (nb - nmin) / nb + exp(-kmin * m) * nmin / nb;
     }
 }
 
@@ -226,7 +418,7 @@ extern "C" int hk_transmission(const double *Ksorted, int nbins, int Nxb, const 
     HK_CHECK_ARG(Nxb >= 3, "hk_transmission: %d points per bin (at least 3)", Nxb);
     HK_CHECK_ARG(nTr > 0, "hk_transmission: nTr must be > 0");
     hipStream_t s = (hipStream_t)stream;
-    dim3 g((unsigned)((nTr + kTrM - 1) / kTrM), (unsigned)nbins);
+    dim3 g((unsigned)((nTr + kTrPer - 1) / kTrPer), (unsigned)nbins);
     hipLaunchKernelGGL(transmission_kernel, g, dim3(kTrThreads), 0, s, Ksorted, Nxb, nxmin, kmin,
                        nTr, dTr, Tr);
     HK_LAUNCH_CHECK();

@@ -413,6 +413,34 @@ __device__ __forceinline__ double cheb_coef64(const double *F, const double *cos
     return (m == 0 ? 1.0 : 2.0) / (double)kFN64 * c;
 }
 
+// Adds g T_m(u), m = 0..19, to f.
+__device__ __forceinline__ void add_moments20(double g, double u, double (&f)[kFN64]) {
+    double p = g, c = g * u;
+    const double u2 = 2.0 * u;
+    f[0] += p;
+    f[1] += c;
+#pragma unroll
+    for (int m = 2; m < kFN64; ++m) {
+        const double n = fma(u2, c, -p);
+        f[m] += n;
+        p = c;
+        c = n;
+    }
+}
+
+// Node weight k from Chebyshev moments M: G_k = (M_0 + 2 sum M_m T_m(u_k)) / 20.
+__device__ __forceinline__ double node_weight(const double *M, const double *cosv, int k) {
+    double s = 0.0;
+    int j = 2 * k + 1;
+    const int step = j;
+    for (int m = 1; m < kFN64; ++m) {
+        s = fma(M[m], cosv[j], s);
+        j += step;
+        j -= j >= 4 * kFN64 ? 4 * kFN64 : 0;
+    }
+    return fma(2.0, s, M[0]) / (double)kFN64;
+}
+
 __device__ __forceinline__ double cheb_sum64(const double *c, double u) {
     double b1 = 0.0, b2 = 0.0;
     const double u2 = 2.0 * u;
