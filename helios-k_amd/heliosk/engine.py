@@ -122,7 +122,7 @@ def sort_lines(nu, S, EL, vy, n, A=None, delta=None, iso=None, iso_mass=(18.0 / 
                iso_ab=(1.0,), iso_sscale=(1.0,), name="species", form=HK_FORM_HITRAN,
                stream=None):
     """Species from an unsorted line list already on the device, ordered by
-    the library's stable radix sort (hk_lines_sort; the thrust sort and
+    the library's stable sort (hk_lines_sort; the thrust sort and
     gathers of heliosk.cu:1147-1171).  Per-line arguments are device
     tensors (float64; iso int32) or array-likes, which are uploaded."""
     dev = _dev()

@@ -175,8 +175,9 @@ int hk_line_state_init(hk_line_state *st, int64_t nlines, void *mem, size_t byte
  * iso) receive the sorted fields and must be distinct from in's, each with
  * room for in->nlines entries.  out's scalar fields (nlines, niso, form, the
  * isotopologue tables, max_abs_delta) are set from in.  At most 2^31 - 1
- * lines per call; the workspace holds two permutations and the radix-sort
- * scratch. */
+ * lines per call; the workspace holds the lines once more as 64-byte
+ * records, or, for short and for very long lists, two (centre, index) arrays;
+ * the latter's size is enough for any list, at the latter's speed. */
 size_t hk_lines_sort_workspace_bytes(int64_t nlines);
 int hk_lines_sort(const hk_lines *in, hk_lines *out, void *workspace, size_t bytes,
                   hk_stream_t stream);
