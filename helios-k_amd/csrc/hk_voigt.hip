@@ -49,6 +49,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "hk_device.h"
@@ -366,18 +367,18 @@ constexpr int kFarMinPts = 256;       // smaller (edge) tiles sum every pair
 constexpr int kFN1 = 9, kFN2 = 15, kFN3 = 19;
 constexpr double kFarRatio1 = 4.0, kFarRatio2 = 2.0, kFarRatio3 = 1.5;
 // Chebyshev-Gauss nodes cos(pi (k + 1/2) / n)
-__constant__ double kFarU1[kFN1] = {
+__device__ constexpr double kFarU1[kFN1] = {
     0.98480775301220802032, 0.86602540378443870761, 0.64278760968653936292,
     0.34202014332566882393, 0, -0.34202014332566849086,
     -0.64278760968653936292, -0.86602540378443848557, -0.98480775301220802032};
-__constant__ double kFarU2[kFN2] = {
+__device__ constexpr double kFarU2[kFN2] = {
     0.99452189536827328986, 0.95105651629515353118, 0.86602540378443870761,
     0.74314482547739424412, 0.5877852522924731371, 0.4067366430758003748,
     0.20791169081775923155, 0, -0.20791169081775934258,
     -0.40673664307580004174, -0.58778525229247302608, -0.74314482547739402207,
     -0.86602540378443870761, -0.95105651629515353118, -0.99452189536827340088};
 
-__constant__ double kFarU3[kFN3] = {
+__device__ constexpr double kFarU3[kFN3] = {
     0.99658449300666984705, 0.96940026593933037447, 0.91577332665505739584,
     0.83716647826252865716, 0.73572391067313169799, 0.61421271268966792789,
     0.47594739303707345179, 0.32469946920468356621, 0.16459459028073375464,
@@ -388,6 +389,41 @@ __constant__ double kFarU3[kFN3] = {
 template <int N>
 __device__ __forceinline__ double far_u(int k) {
     return N == kFN1 ? kFarU1[k] : (N == kFN2 ? kFarU2[k] : kFarU3[k]);
+}
+
+// Node values to Chebyshev coefficients, c_m = sum_k t[k][m] F_k with
+// t[k][m] = (2 - [m == 0]) / N T_m(u_k).  As a table: T_m(u_k) by its
+// recurrence in the loops over k cost each wave 25000 cycles a tile, a sixth
+// of a spectrum whose tiles meet few lines (24 spectra of 3e6 points with
+// 1e4 to 5e6 lines: main pass 30.9 ms, with the table 29.8).
+template <int N>
+struct FarT {
+    double t[N][N];
+};
+
+template <int N>
+constexpr FarT<N> far_table(const double (&u)[N]) {
+    FarT<N> r{};
+    for (int k = 0; k < N; ++k) {
+        double tm = 1.0, tc = u[k];
+        for (int m = 0; m < N; ++m) {
+            r.t[k][m] = (m == 0 ? 1.0 : 2.0) / N * tm;
+            const double tn = 2.0 * u[k] * tc - tm;
+            tm = tc;
+            tc = tn;
+        }
+    }
+    return r;
+}
+
+__constant__ FarT<kFN1> kFarT1 = far_table(kFarU1);
+__constant__ FarT<kFN2> kFarT2 = far_table(kFarU2);
+__constant__ FarT<kFN3> kFarT3 = far_table(kFarU3);
+template <int N>
+__device__ __forceinline__ double far_t(int k, int m) {
+    if constexpr (N == kFN1) return kFarT1.t[k][m];
+    else if constexpr (N == kFN2) return kFarT2.t[k][m];
+    else return kFarT3.t[k][m];
 }
 
 // One band's node sums (FP32, compensated: hi + lo), their totals and the
@@ -489,6 +525,47 @@ __device__ __forceinline__ float wave_total32(float v) {
     v += dpp32<0x142, 0xa>(v);    // row_bcast:15
     v += dpp32<0x143, 0xc>(v);    // row_bcast:31
     return v;
+}
+
+// Wave sums of eight values at once: lanes 0..7 return the sum of v[total_id()].
+// The tree of wave_total32 level by level (the same bits), but in its first
+// three levels two sums share a register: each lane keeps one and passes on
+// the other, 27 instructions for eight sums where single ones take 64 (the
+// FP32 main pass over 24 spectra of 3e6 points, 1e4 to 5e6 lines each: 29.8 ms
+// with single sums, 26.3 so; 1e7 lines on 3e7 points: 22.1 and 20.8).
+// Every lane must be active.
+__device__ __forceinline__ int total_id() {
+    const int l = threadIdx.x & 63, b2 = (l >> 2) & 1;
+    return 4 * (b2 ^ ((l >> 3) & 1)) + ((l & 3) ^ (3 * b2));
+}
+
+template <int CTRL>
+__device__ __forceinline__ float keep_add(bool second, float a, float b) {
+    return (second ? b : a) + dpp32<CTRL, 0xf>(second ? a : b);
+}
+
+template <int M>
+__device__ __forceinline__ float wave_totals8(const float (&v)[M], int id) {
+    static_assert(M >= 2 && M <= 8, "up to eight sums");
+    auto at = [&](int k) { return k < M ? v[k] : 0.0f; };
+    const bool s1 = id & 1, s2 = id & 2, s4 = id & 4;
+    float p[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        p[j] = 0.0f;
+        if (4 * j < M)
+            p[j] = keep_add<0x4e>(s2, keep_add<0xb1>(s1, at(4 * j), at(4 * j + 1)),
+                                  4 * j + 2 < M ? keep_add<0xb1>(s1, at(4 * j + 2), at(4 * j + 3))
+                                                : 0.0f);
+    }
+    float r = keep_add<0x141>(s4, p[0], p[1]);          // row_half_mirror
+    r += dpp32<0x140, 0xf>(r);                          // row_mirror
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(r), __float_as_uint(r), false,
+                                                    false);
+    r = __uint_as_float(h[0]) + __uint_as_float(h[1]);  // rows 0 + 1, 2 + 3
+    const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(r), __float_as_uint(r), false,
+                                                    false);
+    return __uint_as_float(w[0]) + __uint_as_float(w[1]);
 }
 
 // Maximum of v over the wave, complete in lane 63 (the DPP tree of
@@ -615,6 +692,22 @@ __device__ __forceinline__ void band_init(FarBand<N> *b, int t) {
     }
 }
 
+// Up to eight wave sums by lanes 0..7 (one sum in all lanes of its own).
+template <int M>
+__device__ __forceinline__ float wave_totals_of(const float (&v)[M], int id) {
+    if constexpr (M == 1)
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wave_total32(v[0])), 63));
+    else
+        return wave_totals8(v, id);
+}
+
+__device__ __forceinline__ void add_total(float *hi, float *lo, float v) {
+    float h = *hi, l = *lo;
+    two_sum_acc(h, l, v);
+    *hi = h;
+    *lo = l;
+}
+
 // The wave's lines of this band (mine) add their node values to the wave's
 // columns of node sums (all lanes take part in the wave sums).  A line's
 // Doppler-unit offset from the tile centre D and the tile half width h come
@@ -635,48 +728,40 @@ __device__ __forceinline__ void band_nodes(FarBand<N> *b, bool mine, int cover, 
     const bool series2 = __ballot(mine && !(fma(xn, xn, (double)fy * fy) >= (double)kRF32)) == 0ull;
     const float y2 = fy * fy, B = fB * fy * (float)(1.0 / kPi);
     const float B15 = 1.5f * B, BC = fmaxf(-2.0f * y2 * B, -1.0e37f);
-    // the wave totals are gathered into lanes (node k, or target tw and node
-    // k, in lane tw N + k) and added to the columns in one pass at the end
-    float tot = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < N; ++k) {
-        // far lines: |x| >= |D| - h >= |D| / 3, so x in FP32 from FP32 D and
-        // h keeps ~1e-7 of x
-        const float x = fmaf((float)far_u<N>(k), fh, fD);
-        float v = 0.0f;
-        if (series2) {
-            const float inv = rcp32(fmaf(x, x, y2));
-            v = mine ? inv * fmaf(fmaf(BC, inv, B15), inv, B) : 0.0f;
-        } else {
-            v = mine ? fB * far_node32(x, fy) : 0.0f;
-        }
-        if (N != kFN1 || !split) {
-            const float sw = __int_as_float(
-                __builtin_amdgcn_readlane(__float_as_int(wave_total32(v)), 63));
-            tot = lane == k ? sw : tot;
-        } else {
+    const int id = total_id();
+    auto group = [&](auto k0c) {
+        constexpr int k0 = k0c, M = N - k0 < 8 ? N - k0 : 8;
+        float v[M];
 #pragma unroll
-            for (int tw = 0; tw < kWaves; ++tw) {
-                const float sw = __int_as_float(__builtin_amdgcn_readlane(
-                    __float_as_int(wave_total32((cover >> tw) & 1 ? v : 0.0f)), 63));
-                tot = lane == tw * N + k ? sw : tot;
+        for (int j = 0; j < M; ++j) {
+            // far lines: |x| >= |D| - h >= |D| / 3, so x in FP32 from FP32 D and
+            // h keeps ~1e-7 of x
+            const float x = fmaf((float)far_u<N>(k0 + j), fh, fD);
+            if (series2) {
+                const float inv = rcp32(fmaf(x, x, y2));
+                v[j] = mine ? inv * fmaf(fmaf(BC, inv, B15), inv, B) : 0.0f;
+            } else {
+                v[j] = mine ? fB * far_node32(x, fy) : 0.0f;
             }
         }
-    }
-    if (N != kFN1 || !split) {
-        if (lane < N) {
-            float hi = b->hi[lane][wave], lo = b->lo[lane][wave];
-            two_sum_acc(hi, lo, tot);
-            b->hi[lane][wave] = hi;
-            b->lo[lane][wave] = lo;
+        if (N != kFN1 || !split) {
+            const float tot = wave_totals_of(v, id);
+            if (lane < 8 && id < M) add_total(&b->hi[k0 + id][wave], &b->lo[k0 + id][wave], tot);
+        } else if constexpr (N == kFN1) {
+#pragma unroll
+            for (int tw = 0; tw < kWaves; ++tw) {
+                float u[M];
+#pragma unroll
+                for (int j = 0; j < M; ++j) u[j] = (cover >> tw) & 1 ? v[j] : 0.0f;
+                const float tot = wave_totals_of(u, id);
+                if (lane < 8 && id < M)
+                    add_total(&b->xhi[k0 + id][tw][wave], &b->xlo[k0 + id][tw][wave], tot);
+            }
         }
-    } else if (lane < kWaves * N) {
-        const int tw = lane / N, k = lane - tw * N;
-        float hi = b->xhi[k][tw][wave], lo = b->xlo[k][tw][wave];
-        two_sum_acc(hi, lo, tot);
-        b->xhi[k][tw][wave] = hi;
-        b->xlo[k][tw][wave] = lo;
-    }
+    };
+    group(std::integral_constant<int, 0>{});
+    group(std::integral_constant<int, 8>{});
+    if constexpr (N > 16) group(std::integral_constant<int, 16>{});
 }
 
 // Node totals -> Chebyshev coefficients, per target wave, by threads t0 ..
@@ -703,22 +788,9 @@ template <int N>
 __device__ __forceinline__ void band_coeffs(FarCoef<N> *b, int t) {
     if (t >= 0 && t < N * kWaves) {
         const int tw = t / N, m = t % N;
-        // c_m = (2 - [m == 0]) / N sum_k F_k T_m(u_k), T_m by its recurrence
-        // (not unrolled: unrolled, the node constants are hoisted out of the
-        // persistent kernel's item loop and held in registers throughout)
         double c = 0.0;
-#pragma unroll 1
-        for (int k = 0; k < N; ++k) {
-            const double u = far_u<N>(k);
-            double tm = 1.0, tc = u;
-            for (int q = 2; q <= m; ++q) {
-                const double tn = fma(2.0 * u, tc, -tm);
-                tm = tc;
-                tc = tn;
-            }
-            c += b->F[tw][k] * (m == 0 ? 1.0 : tc);
-        }
-        b->c[tw][m] = (m == 0 ? 1.0 : 2.0) / (double)N * c;
+        for (int k = 0; k < N; ++k) c = fma(far_t<N>(k, m), b->F[tw][k], c);
+        b->c[tw][m] = c;
     }
 }
 
@@ -886,22 +958,22 @@ template <int N>
 __device__ __forceinline__ void wave_far_nodes(const Rec32 &q, bool mine, float cw, float hwp,
                                                float (*s)[2], int lane) {
     const float m0 = cw + (float)q.d0;
-    float tot = 0.0f;           // lane k: node k's wave total
-#pragma unroll 1
-    for (int k = 0; k < N; ++k) {
-        const float m = fmaf((float)far_u<N>(k), hwp, m0);
-        const float x = fmaf(m, q.vbh, fmaf(m, q.vbl, q.r));
-        const float v = mine ? far32(q, fmaf(x, x, q.y2)) : 0.0f;
-        const float sw = __int_as_float(
-            __builtin_amdgcn_readlane(__float_as_int(wave_total32(v)), 63));
-        tot = lane == k ? sw : tot;
-    }
-    if (lane < N) {
-        float h = s[lane][0], l = s[lane][1];
-        two_sum_acc(h, l, tot);
-        s[lane][0] = h;
-        s[lane][1] = l;
-    }
+    const int id = total_id();
+    auto group = [&](auto k0c) {
+        constexpr int k0 = k0c, M = N - k0 < 8 ? N - k0 : 8;
+        float v[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const float m = fmaf((float)far_u<N>(k0 + j), hwp, m0);
+            const float x = fmaf(m, q.vbh, fmaf(m, q.vbl, q.r));
+            v[j] = mine ? far32(q, fmaf(x, x, q.y2)) : 0.0f;
+        }
+        const float tot = wave_totals_of(v, id);
+        if (lane < 8 && id < M) add_total(&s[k0 + id][0], &s[k0 + id][1], tot);
+    };
+    group(std::integral_constant<int, 0>{});
+    group(std::integral_constant<int, 8>{});
+    if constexpr (N > 16) group(std::integral_constant<int, 16>{});
 }
 
 // Wave-level far field, coefficients of one band from the wave's node sums
@@ -910,18 +982,8 @@ template <int N>
 __device__ __forceinline__ void wave_far_coeffs(const float (*s)[2], double *c, int m) {
     if (m < 0 || m >= N) return;
     double acc = 0.0;
-#pragma unroll 1
-    for (int k = 0; k < N; ++k) {
-        const double u = far_u<N>(k);
-        double tm = 1.0, tc = u;
-        for (int q = 2; q <= m; ++q) {
-            const double tn = fma(2.0 * u, tc, -tm);
-            tm = tc;
-            tc = tn;
-        }
-        acc += ((double)s[k][0] + (double)s[k][1]) * (m == 0 ? 1.0 : tc);
-    }
-    c[m] = (m == 0 ? 1.0 : 2.0) / (double)N * acc;
+    for (int k = 0; k < N; ++k) acc = fma(far_t<N>(k, m), (double)s[k][0] + (double)s[k][1], acc);
+    c[m] = acc;
 }
 
 template <int PPT, int LM>
