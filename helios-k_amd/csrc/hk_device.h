@@ -204,8 +204,9 @@ __device__ __forceinline__ double rew_core64(double x, double y, double ey, doub
 
 // FP32 core for r2 < 25: n0 = ceil(x/a) <= 7, so every series term uses
 // n <= kNT32; dtab[n] = 1/(a^2 n^2 + y^2) is filled once per line and tile,
-// with dtab[0] = 0 so that the downward terms below n = 1 vanish without a
-// branch.
+// with dtab[-5..0] = 0 so that the downward terms below n = 1 vanish without a
+// branch or a clamp of their index (a clamp per term: 1e7 lines on 3e7 points
+// 18.6 ms, this 17.5).
 // As in the FP64 core, each series is built from two hardware exponentials by
 // the ratio recurrences (4 exponentials per pair instead of 19); the
 // recurrences add < 7 roundings per term (< 5e-7 relative).
@@ -234,7 +235,7 @@ __device__ __forceinline__ float rew_core32(float x, float y, float ey, float q1
     // s3 = sum_{n>=1} e^{-(an-x)^2} d_n, from its largest term n0 = ceil(x/a)
     // upwards (k <= kN32: exponents (ka + dl)^2, dl = a n0 - x in [0, a)) and
     // downwards (k <= kN32 + 1: exponents (ka - dl)^2 fall one step later)
-    const int n0 = (int)ceilf(x * (float)(1.0 / kA32));
+    const int n0 = max((int)ceilf(x * (float)(1.0 / kA32)), 1);
     const float dl = fmaf(a, (float)n0, -x);
     const float E0 = __expf(-dl * dl), e2 = __expf(-2.0f * a * dl);
     float s3 = 0.0f;
@@ -253,7 +254,7 @@ __device__ __forceinline__ float rew_core32(float x, float y, float ey, float q1
         for (int k = 1; k <= kN32 + 1; ++k) {
             E *= sg;
             sg *= kE2A32;
-            s3 = fmaf(E, dtab[max(n0 - k, 0)], s3);
+            s3 = fmaf(E, dtab[n0 - k], s3);
         }
     }
     const float xy = x * y;

@@ -207,11 +207,13 @@ __device__ __forceinline__ void two_sum_acc(float &hi, float &lo, float p) {
     hi = s;
 }
 
-// Per-line core table stride (entries 1..kNT32 used).  Odd, so that lanes
-// reading different lines' tables in one round of the core walk fall in
-// different LDS banks (a stride of 16 put every fourth line on one bank:
-// the c2 line-core pass 20 ms slower).
-constexpr int kDT = 17;
+// Per-line core table: kDT0 zeros, then entry n at kDT0 + n (entry 0 is zero
+// too, entries 1..kNT32 used).  The stride is odd, so that lanes reading
+// different lines' tables in one round of the core walk fall in different
+// LDS banks (a stride of 16 put every fourth line on one bank: 20 ms on the
+// line-core pass of 50 spectra).
+constexpr int kDT0 = 5, kDT = 19;
+static_assert(kDT0 + kNT32 < kDT && 1 - (kN32 + 1) >= -kDT0, "table entries of the core series");
 // Largest x^2 + y^2 over a wave for the whole-wave 8-node FP32 path: keeps
 // D12 D34 ~ r2^8 below the FP32 range.  The whole-wave series path has no
 // such limit (its coefficients are bounded by y^2 < 4096).
@@ -1262,16 +1264,17 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
         const int64_t i = base + t;
         Core32 r;
         bool valid = false;
+        const int64_t il = min(i, ti.hi - 1);
+        // all loads at once: one wait on memory, not three
+        const double nu = a.nu[il], hw = a.hw[il], y = a.y[il], ia = a.ia[il], S = a.S[il];
+        const double eyd = a.ey[il];
         if (i < ti.hi) {
-            const double nu = a.nu[i];
             int64_t wl, wh;
-            cut_window(nu, a.hw[i], a.numin, a.dnu, a.nx, wl, wh);
+            cut_window(nu, hw, a.numin, a.dnu, a.nx, wl, wh);
             const int64_t clo = max(wl, j0), chi = min(wh, j0 + W);
-            const double y = a.y[i];
             const float yf = (float)y;
             const double y2 = (double)yf * (double)yf;
             if (clo < chi && y2 < (double)kRB32) {
-                const double ia = a.ia[i];
                 const double jcd = rint((nu - a.numin) / a.dnu);
                 const double rr = (fma(jcd, a.dnu, a.numin) - nu) * ia;
                 const double vb = a.dnu * ia, d0 = (double)j0 - jcd;
@@ -1287,8 +1290,8 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
                     r.vbl = (float)(vb - (double)vbh);
                     r.y = yf;
                     r.y2 = yf * yf;
-                    r.A = (float)(ldexp(a.S[i], -ti.e) * kISqrtPi);
-                    r.ey = (float)a.ey[i];
+                    r.A = (float)(ldexp(S, -ti.e) * kISqrtPi);
+                    r.ey = (float)eyd;
                     r.q1 = core_q1_32(yf);
                     r.d0 = (int32_t)d0;
                 }
@@ -1300,10 +1303,10 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
         const int slot = compact_slot(valid, cnt, n);
         if (valid) {
             rec[slot] = r;
-            dtab[slot * kDT] = 0.0f;
+            for (int k = 0; k <= kDT0; ++k) dtab[slot * kDT + k] = 0.0f;
             for (int k = 1; k <= kNT32; ++k) {
                 const double an = kA32 * k;
-                dtab[slot * kDT + k] = (float)(1.0 / fma(an, an, (double)r.y2));
+                dtab[slot * kDT + kDT0 + k] = (float)(1.0 / fma(an, an, (double)r.y2));
             }
         }
         __syncthreads();
@@ -1360,7 +1363,7 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
             const float x = fmaf(mm, q.vbh, fmaf(mm, q.vbl, q.r));
             const float r2 = fmaf(x, x, q.y2);
             if (jr >= q.lo && jr < q.hi && r2 < kRB32)
-                part += q.A * rew_core32(x, q.y, q.ey, q.q1, dtab + l * kDT);
+                part += q.A * rew_core32(x, q.y, q.ey, q.q1, dtab + l * kDT + kDT0);
             if (++since == 32) { two_sum_acc(hi, lo, part); part = 0.0f; since = 0; }
         };
         if (4 * rounds >= 3 * nrec) {
@@ -1382,7 +1385,7 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
                 const float mm = (float)(jr + q.d0);
                 const float x = fmaf(mm, q.vbh, fmaf(mm, q.vbl, q.r));
                 const float r2 = fmaf(x, x, q.y2);
-                if (r2 < kRB32) part += q.A * rew_core32(x, q.y, q.ey, q.q1, dtab + l * kDT);
+                if (r2 < kRB32) part += q.A * rew_core32(x, q.y, q.ey, q.q1, dtab + l * kDT + kDT0);
             }
             if (++since == 32) { two_sum_acc(hi, lo, part); part = 0.0f; since = 0; }
         }
@@ -1420,7 +1423,10 @@ __global__ __launch_bounds__(256) void voigt_core_kernel(VArgs a) {
     core_f32c(a, blockIdx.x, rec, dtab, cnt);
 }
 
-// Persistent form: workgroups take (spectrum, tile) items from a queue.
+// Persistent form: workgroups take (spectrum, tile) items from a queue, `chunk`
+// of them at a time: one address takes an atomic per 12 ns from the whole chip,
+// which alone was 3.4 of the 7.9 ms of a line-core pass over 281000 tiles
+// (6.7 ms now, loads and the core table included).
 // item_start[s] = first item of spectrum s (nspec+1 entries).  PPT == 0
 // selects the line-core pass.
 // Occupancy floors (waves per SIMD): the FP32C main pass is latency-bound
@@ -1441,7 +1447,8 @@ template <int MODE, int PPT, int LM>
 __global__ __launch_bounds__(256, PPT == 0 ? (MODE == HK_VOIGT_FP32C ? 5 : 1) : main_waves(MODE, PPT, LM))
 void voigt_persistent_kernel(const VArgs *__restrict__ specs,
                                                                const int64_t *__restrict__ item_start,
-                                                               int nspec, unsigned long long *counter) {
+                                                               int nspec, unsigned long long *counter,
+                                                               int chunk) {
     constexpr size_t kBytes =
         MODE == HK_VOIGT_FP64 ? sizeof(Far64LDS)
                               : (PPT == 0 ? sizeof(Core32) : sizeof(Rec32)) * kThreads * LM;
@@ -1451,17 +1458,21 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
     __shared__ __attribute__((aligned(16))) char smem[kBytes];
     __shared__ FarLDS fl[1];
     const int64_t total = item_start[nspec];
-    for (;;) {
+    int64_t item = 0, end = 0;
+    for (;; ++item) {
         __syncthreads();
-        if (threadIdx.x == 0) s_item = (int64_t)atomicAdd(counter, 1ull);
-        __syncthreads();
-        // uniform across the workgroup: keep the item, spectrum and its
-        // arguments in scalar registers
-        const int64_t iv = s_item;
-        const int64_t item =
-            (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(iv >> 32)) << 32) |
-                      (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)iv));
-        if (item >= total) break;
+        if (item >= end) {
+            if (threadIdx.x == 0) s_item = (int64_t)atomicAdd(counter, (unsigned long long)chunk);
+            __syncthreads();
+            // uniform across the workgroup: keep the item, spectrum and its
+            // arguments in scalar registers
+            const int64_t iv = s_item;
+            item =
+                (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(iv >> 32)) << 32) |
+                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)iv));
+            if (item >= total) break;
+            end = min(item + chunk, total);
+        }
         const int s = __builtin_amdgcn_readfirstlane(item_spectrum(item_start, nspec, item));
         const VArgs a = specs[s];
         const int64_t tile = item - item_start[s];
@@ -1687,28 +1698,33 @@ void launch_tiles(int ppt, int lm, int64_t ntiles, hipStream_t s, const VArgs &a
 
 template <int MODE, int LM>
 void launch_persistent_lm(int ppt, unsigned grid, hipStream_t s, const VArgs *specs,
-                          const int64_t *item_start, int nspec, unsigned long long *counter) {
+                          const int64_t *item_start, int nspec, unsigned long long *counter,
+                          int chunk) {
     dim3 g(grid), b(kThreads);
     switch (ppt) {
-        case 1: hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, specs, item_start, nspec, counter); break;
-        case 2: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 2, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
-        case 4: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 4, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
-        case 8: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 8, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
-        default: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 16, LM>), g, b, 0, s, specs, item_start, nspec, counter); break;
+        case 1: hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
+        case 2: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 2, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
+        case 4: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 4, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
+        case 8: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 8, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
+        default: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 16, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
     }
 }
 
 // ppt == 0: the line-core pass (its stages are kThreads lines)
 template <int MODE>
 void launch_persistent(int ppt, int lm, unsigned grid, hipStream_t s, const VArgs *specs,
-                       const int64_t *item_start, int nspec, unsigned long long *counter) {
+                       const int64_t *item_start, int nspec, unsigned long long *counter,
+                       int64_t nitems) {
+    // at least 32 chunks a workgroup, so that the last ones end together (4:
+    // the line-core pass above 9.8 ms, 16: 7.1, 32: 6.8, 64: 7.2)
+    const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(64, nitems / (32 * (int64_t)grid)));
     if (MODE == HK_VOIGT_FP32C && ppt == 0)
         hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP32C, 0, 1>), dim3(grid), dim3(kThreads), 0, s,
-                           specs, item_start, nspec, counter);
+                           specs, item_start, nspec, counter, chunk);
     else if (MODE == HK_VOIGT_FP32C && lm == 2)
-        launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, grid, s, specs, item_start, nspec, counter);
+        launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, grid, s, specs, item_start, nspec, counter, chunk);
     else
-        launch_persistent_lm<MODE, 1>(ppt, grid, s, specs, item_start, nspec, counter);
+        launch_persistent_lm<MODE, 1>(ppt, grid, s, specs, item_start, nspec, counter, chunk);
 }
 
 int check_state(const hk_line_state *st, const char *fn) {
@@ -1988,7 +2004,8 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
     if (batch->items_main <= 0) return HK_OK;
     const unsigned gm = persistent_grid(batch->items_main);
     if (batch->mode == HK_VOIGT_FP64) {
-        launch_persistent<HK_VOIGT_FP64>(ppt, lm, gm, s, args, items, nspec, counter);
+        launch_persistent<HK_VOIGT_FP64>(ppt, lm, gm, s, args, items, nspec, counter,
+                                         batch->items_main);
         HK_LAUNCH_CHECK();
         return HK_OK;
     }
@@ -1999,9 +2016,10 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
                        dim3(256), 0, s, cargs, citems, nspec, kCoreW, 1);
     HK_LAUNCH_CHECK();
     const unsigned gc = persistent_grid(batch->items_core);
-    launch_persistent<HK_VOIGT_FP32C>(ppt, lm, gm, s, args, items, nspec, counter);
+    launch_persistent<HK_VOIGT_FP32C>(ppt, lm, gm, s, args, items, nspec, counter, batch->items_main);
     HK_LAUNCH_CHECK();
-    launch_persistent<HK_VOIGT_FP32C>(0, 1, gc, s, cargs, citems, nspec, counter + 1);
+    launch_persistent<HK_VOIGT_FP32C>(0, 1, gc, s, cargs, citems, nspec, counter + 1,
+                                      batch->items_core);
     HK_LAUNCH_CHECK();
     return HK_OK;
 }
