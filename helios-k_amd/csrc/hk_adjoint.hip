@@ -27,7 +27,8 @@
 //
 // What bounds it: FP64 vector instructions, about half of them the line cores.
 // One wave per line over all points of its window took 13.3 ms for 3.3e5 lines
-// on 1e6 points, cut 50 cm^-1 (3.3e9 pairs), this 2.56.
+// on 1e6 points, cut 50 cm^-1 (3.3e9 pairs), this 2.14 (with 3 workgroups a CU
+// for the registers, as the compiler chooses, 2.23).
 #include <math.h>
 
 #include "hk_device.h"
@@ -250,7 +251,7 @@ __device__ __forceinline__ void add_far(int cls, double D, double half, double i
     }
 }
 
-__global__ __launch_bounds__(kAT, 3) void adjoint_kernel(AArgs a) {
+__global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
     __shared__ AdjLDS sh;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -498,11 +499,13 @@ __global__ __launch_bounds__(1024) void sum_rows_kernel(const double *__restrict
     if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
-// Short lists split each line's tiles over several workgroups: enough that
-// ~5 workgroups per CU exist (256 lines each), at most 32.
+// Lists short of filling the chip several times over split each line's tiles
+// over several workgroups, at most 32: up to ~20 workgroups per CU (256 lines
+// each), since a workgroup's barriers leave its CU to the others.  3.3e5 lines,
+// 11 tiles a window: 1 part 2.60 ms, 2 parts 2.28, 4 parts 2.15, 8 parts 2.32.
 int adjoint_parts(int64_t nlines) {
     const int64_t nblocks = (nlines + kAT - 1) / kAT;
-    const int64_t p = nblocks > 0 ? 1280 / nblocks : 1;
+    const int64_t p = nblocks > 0 ? 5300 / nblocks : 1;
     return (int)(p < 1 ? 1 : (p > 32 ? 32 : p));
 }
 
