@@ -15,11 +15,11 @@
 //     the same kernel: Nxmin (a binary search: findCut's rules on a sorted
 //     bin), the rescale, ln(K unit_scale), the nC Chebyshev moments
 //     m_i = sum_k T_i(x_k) b_k and the first nC values b0 of b = ln K2;
-//   * a longer bin is cut into LDS-sorted runs of 16384 points (written
-//     once), a splitter kernel per bin picks value splitters from a regular
+//   * a longer bin is cut into LDS-sorted runs of 8192 or 16384 points
+//     (written once), a splitter kernel per bin picks value splitters from a regular
 //     sample of the runs (every m-th value of each run), and one workgroup
 //     per bucket [s_w, s_w+1) gathers the bucket's values from every run,
-//     sorts them in LDS and fits the output points whose rescale nodes fall
+//     merges them in LDS and fits the output points whose rescale nodes fall
 //     in the bucket's ranks; per-bucket partial moments are summed in
 //     bucket order.  With regular sampling a bucket holds at most
 //     m (g - 1 + runs) values above its lower splitter (g samples per
@@ -307,25 +307,26 @@ __global__ __launch_bounds__(kSortNT) void bin_sort_fit_kernel(const double *__r
 }
 
 // ---------------------------------------------------------------------------
-// Longer segments, step 1: LDS-sorted runs of kSortCap values.
+// Longer segments, step 1: LDS-sorted runs of NT * kIPT values.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kSortNT) void run_sort_kernel(const double *__restrict__ K,
-                                                           const Seg *__restrict__ segs,
-                                                           int64_t nseg, int nrun_max,
-                                                           double *__restrict__ runs) {
-    __shared__ double s[lds_sort_slots(kSortCap)];
+template <int NT>
+__global__ __launch_bounds__(NT) void run_sort_kernel(const double *__restrict__ K,
+                                                      const Seg *__restrict__ segs, int64_t nseg,
+                                                      int nrun_max, double *__restrict__ runs) {
+    constexpr int kCap = NT * kIPT;
+    __shared__ double s[lds_sort_slots(kCap)];
     const int64_t f = flat_block();
     if (f >= nseg * nrun_max) return;
     const Seg sg = segs[f / nrun_max];
-    const int64_t off = (int64_t)(f % nrun_max) * kSortCap;
+    const int64_t off = (int64_t)(f % nrun_max) * kCap;
     if (off >= sg.len) return;
-    const int n = (int)min((int64_t)kSortCap, sg.len - off);
+    const int n = (int)min((int64_t)kCap, sg.len - off);
     const int t = threadIdx.x;
     const double *src = K + sg.start + off;
-    for (int i = t; i < n; i += kSortNT) s[pad_index(i)] = src[i];
-    lds_sort<kSortNT, kIPT>(s, n);
+    for (int i = t; i < n; i += NT) s[pad_index(i)] = src[i];
+    lds_sort<NT, kIPT>(s, n);
     double *dst = runs + sg.start + off;
-    for (int i = t; i < n; i += kSortNT) dst[i] = s[pad_index(i)];
+    for (int i = t; i < n; i += NT) dst[i] = s[pad_index(i)];
 }
 
 // Pairwise merge of runs of length w into runs of 2w (bins of more than
@@ -447,6 +448,23 @@ __global__ __launch_bounds__(kSortNT) void splitter_kernel(const double *__restr
     }
 }
 
+// Number of values of the sorted run v[0..n) below key (upper: not above it),
+// by a quad of lanes: four probes a step.
+__device__ __forceinline__ int64_t run_bound4(const double *v, int64_t n, double key, bool upper) {
+    const int k = threadIdx.x & 3, sh = threadIdx.x & 60;
+    int64_t lo = 0, hi = n;
+    while (lo < hi) {
+        const int64_t len = hi - lo;
+        auto probe = [&](int q) { return lo + len * (q + 1) / 5; };
+        const double x = v[probe(k)];
+        const int c = __popcll((__ballot(upper ? x <= key : x < key) >> sh) & 15ull);
+        const int64_t first = c > 0 ? probe(c - 1) + 1 : lo;
+        if (c < 4) hi = probe(c);
+        lo = first;
+    }
+    return lo;
+}
+
 // ---------------------------------------------------------------------------
 // Longer segments, step 3: one workgroup per bucket [s_lo, s_hi).  Its
 // values above s_lo are gathered from every run into LDS and sorted; the
@@ -454,7 +472,10 @@ __global__ __launch_bounds__(kSortNT) void splitter_kernel(const double *__restr
 // sorted segment are then: E copies of s_lo, then the sorted values; rank
 // o1 (the next bucket's first) is the smallest run value >= s_hi.
 // Four workgroups per CU: 128 VGPRs with a few spilled, faster than three
-// per CU without spills.
+// per CU without spills.  The bounds are searched side by side, five ways a
+// step (one lane per run halving for its three bounds in turn: 39 dependent
+// loads; 300 bins of 1e5 points with 20 coefficients 646 us, so 617, and 493
+// with the runs' parts merged instead of sorted anew).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBucketNT, 4) void bucket_kernel(const double *__restrict__ runs,
                                                            const Seg *__restrict__ segs,
@@ -465,8 +486,8 @@ __global__ __launch_bounds__(kBucketNT, 4) void bucket_kernel(const double *__re
     __shared__ double red[kBucketNT / 64][kMomGroup];
     __shared__ double mom[kMaxNC];
     __shared__ int64_t r_lo[kMaxRuns], r_eq[kMaxRuns], r_hi[kMaxRuns];
-    __shared__ int s_off[kMaxRuns + 1];
-    __shared__ double s_halo;
+    __shared__ int s_off[kMaxRuns + 1], s_len[kMaxRuns];
+    __shared__ double s_halo, s_next[kMaxRuns];
     __shared__ int s_k[2];
     const int64_t f = flat_block();
     if (f >= nseg * ba.bmax) return;
@@ -492,17 +513,24 @@ __global__ __launch_bounds__(kBucketNT, 4) void bucket_kernel(const double *__re
     const int nrun = (int)((sg.len + R - 1) / R);
     const double *base = runs + sg.start;
     const bool empty = has_lo && has_hi && !(slo < shi);
-    if (t < nrun) {
-        const double *rv = base + (int64_t)t * R;
-        const int64_t len = min(R, sg.len - (int64_t)t * R);
-        int64_t lo = 0, eq = 0, hi = len;
-        if (has_lo) {
-            lo = run_lower_bound(rv, len, slo);
-            eq = run_upper_bound(rv, len, slo);
+    // four lanes per run and bound: first value >= s_lo, > s_lo, >= s_hi
+    {
+        const int c = (t >> 2) & (kMaxRuns - 1), kind = t / (4 * kMaxRuns);
+        if (kind < 3 && c < nrun) {
+            const int64_t len = min(R, sg.len - (int64_t)c * R);
+            int64_t r = kind == 2 ? len : 0;
+            if (kind == 2 ? has_hi : has_lo)
+                r = run_bound4(base + (int64_t)c * R, len, kind == 2 ? shi : slo, kind == 1);
+            if ((t & 3) == 0) (kind == 0 ? r_lo : kind == 1 ? r_eq : r_hi)[c] = r;
         }
-        if (has_hi) hi = run_lower_bound(rv, len, shi);
-        if (empty) { eq = lo; hi = lo; }
-        r_lo[t] = lo; r_eq[t] = eq; r_hi[t] = max(hi, eq);
+    }
+    __syncthreads();
+    if (t < nrun) {
+        const int64_t len = min(R, sg.len - (int64_t)t * R);
+        const int64_t eq = empty ? r_lo[t] : r_eq[t], hi = empty ? eq : max(r_hi[t], eq);
+        r_eq[t] = eq;
+        r_hi[t] = hi;
+        s_next[t] = hi < len ? base[(int64_t)t * R + hi] : INFINITY;
     }
     __syncthreads();
     if (t == 0) {
@@ -510,9 +538,10 @@ __global__ __launch_bounds__(kBucketNT, 4) void bucket_kernel(const double *__re
         double halo = INFINITY;
         for (int c = 0; c < nrun; ++c) {
             s_off[c] = off;
-            off += (int)min((int64_t)kBucketCap - off, r_hi[c] - r_eq[c]);
-            const int64_t len = min(R, sg.len - (int64_t)c * R);
-            if (r_hi[c] < len) halo = fmin(halo, base[(int64_t)c * R + r_hi[c]]);
+            const int n = (int)min((int64_t)kBucketCap - off, r_hi[c] - r_eq[c]);
+            s_len[c] = n;
+            off += (n + kIPT - 1) / kIPT * kIPT;
+            halo = fmin(halo, s_next[c]);
         }
         s_off[nrun] = off;
         s_halo = halo;
@@ -520,13 +549,18 @@ __global__ __launch_bounds__(kBucketNT, 4) void bucket_kernel(const double *__re
     __syncthreads();
     int64_t o0 = 0, E = 0;
     for (int c = 0; c < nrun; ++c) { o0 += r_lo[c]; E += r_eq[c] - r_lo[c]; }
-    const int M = s_off[nrun];
+    // each run's part, up to a multiple of kIPT with +inf, merged (the parts
+    // are in order: sorting them anew took 8 rounds instead of log2(nrun))
+    int M = 0;
     for (int c = 0; c < nrun; ++c) {
-        const int cnt = s_off[c + 1] - s_off[c];
+        const int cnt = s_len[c], np = s_off[c + 1] - s_off[c];
         const double *rv = base + (int64_t)c * R + r_eq[c];
-        for (int i = t; i < cnt; i += kBucketNT) s[pad_index(s_off[c] + i)] = rv[i];
+        for (int i = t; i < np; i += kBucketNT)
+            s[pad_index(s_off[c] + i)] = i < cnt ? rv[i] : INFINITY;
+        M += cnt;
     }
-    lds_sort<kBucketNT, kIPT>(s, M);
+    __syncthreads();
+    lds_merge_runs<kBucketNT, kIPT>(s, s_off, nrun);
     const int64_t o1 = o0 + E + M;
     const double halo = s_halo;
     auto val = [&](int64_t r) {
@@ -1121,18 +1155,30 @@ static int get_plan(int Nxb, int nC, std::vector<double> &P) {
 // ---------------------------------------------------------------------------
 struct SortPlan {
     bool chunked = false;   // some segment holds more than kSortCap values
+    int run0 = 0;           // values of an LDS-sorted run
     int nrun = 0;           // LDS-sorted runs of the longest segment
     int merges = 0;         // pairwise merge passes before the bucket pass
     int64_t runlen = 0;     // run length after the merges
     int m = 0, g = 0, bmax = 0;
 };
 
+// Values of an LDS-sorted run: 8192 while that makes at most kMaxRuns runs, else
+// kSortCap.  The shorter runs put two workgroups on a CU, so that one's
+// barriers leave it to the other, and move one merge round from the run sort to
+// the bucket pass (whole call, runs of 16384 and of 8192: 500 bins of 2e4 points
+// 504 and 416 us, 400 of 4e4 627 and 572, 300 of 1e5 1105 and 1041; runs of 4096,
+// four workgroups a CU, 446, 582 and 1062).
+static int first_run(int64_t maxlen) {
+    return maxlen <= (int64_t)kMaxRuns * (kSortCap / 2) ? kSortCap / 2 : kSortCap;
+}
+
 static int plan_sort(int64_t maxlen, SortPlan &sp) {
     sp = SortPlan();
     if (maxlen <= kSortCap) return HK_OK;
     sp.chunked = true;
-    sp.nrun = (int)((maxlen + kSortCap - 1) / kSortCap);
-    sp.runlen = kSortCap;
+    sp.run0 = first_run(maxlen);
+    sp.nrun = (int)((maxlen + sp.run0 - 1) / sp.run0);
+    sp.runlen = sp.run0;
     // sample spacing: at most kSortCap - kMaxRuns samples per segment
     sp.m = (int)std::max<int64_t>(8, (maxlen + (kSortCap - kMaxRuns) - 1) / (kSortCap - kMaxRuns));
     if (sp.m > kBucketCap / 2) {
@@ -1141,13 +1187,15 @@ static int plan_sort(int64_t maxlen, SortPlan &sp) {
         return HK_ERR_UNSUPPORTED;
     }
     int64_t k = (maxlen + sp.runlen - 1) / sp.runlen;
-    // at most kMaxRuns runs, and room for a bucket: m (g + runs) <= kBucketCap
-    while (k > kMaxRuns || sp.m * (k + 1) > kBucketCap) {
+    // at most kMaxRuns runs, and room for a bucket: m (g + runs) <= kBucketCap,
+    // each run's part rounded up to kIPT values (one run's always fits)
+    auto pad = [](int64_t runs) { return runs > 1 ? runs * kIPT : 0; };
+    while (k > kMaxRuns || sp.m * (k + 1) + pad(k) > kBucketCap) {
         sp.runlen *= 2;
         ++sp.merges;
         k = (maxlen + sp.runlen - 1) / sp.runlen;
     }
-    sp.g = kBucketCap / sp.m - (int)k;
+    sp.g = (kBucketCap - (int)pad(k)) / sp.m - (int)k;
     const int64_t nsamp = maxlen / sp.m;
     sp.bmax = (int)std::max<int64_t>(1, (nsamp + sp.g - 1) / sp.g);
     return HK_OK;
@@ -1198,14 +1246,19 @@ static int sort_fit_segments(const double *K, const Seg *segs, int64_t nseg, Seg
     }
     double *runs = (double *)(base + L.off_runs);
     double *runs2 = (double *)(base + L.off_runs2);
-    hipLaunchKernelGGL(run_sort_kernel, flat_grid(nseg * sp.nrun), dim3(kSortNT), 0, s, K, segs,
-                       nseg, sp.nrun, runs);
+    const dim3 gr = flat_grid(nseg * sp.nrun);
+    if (sp.run0 == kSortNT / 2 * kIPT)
+        hipLaunchKernelGGL(run_sort_kernel<kSortNT / 2>, gr, dim3(kSortNT / 2), 0, s, K, segs, nseg,
+                           sp.nrun, runs);
+    else
+        hipLaunchKernelGGL(run_sort_kernel<kSortNT>, gr, dim3(kSortNT), 0, s, K, segs, nseg, sp.nrun,
+                           runs);
     HK_LAUNCH_CHECK();
     // runs and K are addressed alike: run values of a segment start at its
     // own offset in the runs buffer
-    const int64_t maxlen = (int64_t)sp.nrun * kSortCap;
+    const int64_t maxlen = (int64_t)sp.nrun * sp.run0;
     const int64_t nblk = (maxlen + kMB - 1) / kMB;
-    int64_t w = kSortCap;
+    int64_t w = sp.run0;
     for (int p = 0; p < sp.merges; ++p, w *= 2) {
         hipLaunchKernelGGL(merge_lds_kernel, flat_grid(nseg * nblk), dim3(256), 0, s, runs, runs2,
                            segs, nseg, nblk, w);

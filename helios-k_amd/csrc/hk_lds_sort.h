@@ -101,6 +101,47 @@ __device__ __forceinline__ void load_window(const double *s, int i0, int m, doub
     }
 }
 
+// The IPT values from output diag on of the merge of run A (na values at a0)
+// with run B (nb values at b0).
+template <int IPT, bool FAST>
+__device__ __forceinline__ void merge_outputs(const double *s, int a0, int na, int b0, int nb,
+                                              int diag, double (&v)[IPT]) {
+    const int a = merge_path(s, a0, na, b0, nb, diag), b = diag - a;
+    if (FAST) {
+        // this thread's IPT outputs are the IPT smallest of the next
+        // IPT values of each run: the half-cleaner of a bitonic merge
+        // (A ascending against B descending) picks them, and its
+        // sorting network orders them
+        double wa[IPT], wb[IPT];
+        load_window<IPT>(s, a0 + a, na - a, wa);
+        load_window<IPT>(s, b0 + b, nb - b, wb);
+#pragma unroll
+        for (int q = 0; q < IPT; ++q) v[q] = fmin(wa[q], wb[IPT - 1 - q]);
+#pragma unroll
+        for (int j = IPT / 2; j > 0; j >>= 1) {
+#pragma unroll
+            for (int i = 0; i < IPT; ++i) {
+                if ((i & j) == 0) {
+                    const double lo = fmin(v[i], v[i + j]), hi = fmax(v[i], v[i + j]);
+                    v[i] = lo;
+                    v[i + j] = hi;
+                }
+            }
+        }
+    } else {
+        int ia = a, ib = b;
+        double va = ia < na ? s[pad_index(a0 + ia)] : INFINITY;
+        double vb = ib < nb ? s[pad_index(b0 + ib)] : INFINITY;
+#pragma unroll
+        for (int q = 0; q < IPT; ++q) {
+            const bool ta = ib >= nb || (ia < na && va <= vb);
+            v[q] = ta ? va : vb;
+            if (ta) { ++ia; va = ia < na ? s[pad_index(a0 + ia)] : INFINITY; }
+            else { ++ib; vb = ib < nb ? s[pad_index(b0 + ib)] : INFINITY; }
+        }
+    }
+}
+
 template <int NT, int IPT, bool FAST>
 __device__ __forceinline__ void lds_sort_run(double *s, int np, double (&v)[IPT], bool act,
                                              int d0, int L0) {
@@ -118,42 +159,7 @@ __device__ __forceinline__ void lds_sort_run(double *s, int np, double (&v)[IPT]
             const int ps = d0 / (2 * L) * (2 * L);
             const int na = min(L, np - ps);
             const int nb = min(L, np - ps - na);
-            const int diag = d0 - ps;
-            const int a0 = ps, b0 = ps + na;
-            const int a = merge_path(s, a0, na, b0, nb, diag), b = diag - a;
-            if (FAST) {
-                // this thread's IPT outputs are the IPT smallest of the next
-                // IPT values of each run: the half-cleaner of a bitonic merge
-                // (A ascending against B descending) picks them, and its
-                // sorting network orders them
-                double wa[IPT], wb[IPT];
-                load_window<IPT>(s, a0 + a, na - a, wa);
-                load_window<IPT>(s, b0 + b, nb - b, wb);
-#pragma unroll
-                for (int q = 0; q < IPT; ++q) v[q] = fmin(wa[q], wb[IPT - 1 - q]);
-#pragma unroll
-                for (int j = IPT / 2; j > 0; j >>= 1) {
-#pragma unroll
-                    for (int i = 0; i < IPT; ++i) {
-                        if ((i & j) == 0) {
-                            const double lo = fmin(v[i], v[i + j]), hi = fmax(v[i], v[i + j]);
-                            v[i] = lo;
-                            v[i + j] = hi;
-                        }
-                    }
-                }
-            } else {
-                int ia = a, ib = b;
-                double va = ia < na ? s[pad_index(a0 + ia)] : INFINITY;
-                double vb = ib < nb ? s[pad_index(b0 + ib)] : INFINITY;
-#pragma unroll
-                for (int q = 0; q < IPT; ++q) {
-                    const bool ta = ib >= nb || (ia < na && va <= vb);
-                    v[q] = ta ? va : vb;
-                    if (ta) { ++ia; va = ia < na ? s[pad_index(a0 + ia)] : INFINITY; }
-                    else { ++ib; vb = ib < nb ? s[pad_index(b0 + ib)] : INFINITY; }
-                }
-            }
+            merge_outputs<IPT, FAST>(s, ps, na, ps + na, nb, d0 - ps, v);
         }
         __syncthreads();
         if (act) {
@@ -161,6 +167,50 @@ __device__ __forceinline__ void lds_sort_run(double *s, int np, double (&v)[IPT]
             for (int q = 0; q < IPT; ++q) s[pad_index(d0 + q)] = v[q];
         }
     }
+}
+
+// Merges the nrun sorted runs s[pad_index(i)], off[c] <= i < off[c + 1], whose
+// bounds are multiples of IPT (so one thread's outputs stay in one pair of
+// runs); own: the run that holds this thread's first value.
+template <int IPT, bool FAST>
+__device__ __forceinline__ void lds_merge_rounds(double *s, const int *off, int nrun, int own,
+                                                 int d0, bool act, double (&v)[IPT]) {
+    for (int L = 1; L < nrun; L <<= 1) {
+        if (act) {
+            const int g = own / (2 * L) * (2 * L);
+            const int a0 = off[g], b0 = off[min(g + L, nrun)], e0 = off[min(g + 2 * L, nrun)];
+            merge_outputs<IPT, FAST>(s, a0, b0 - a0, b0, e0 - b0, d0 - a0, v);
+        }
+        __syncthreads();
+        if (act) {
+#pragma unroll
+            for (int q = 0; q < IPT; ++q) s[pad_index(d0 + q)] = v[q];
+        }
+        __syncthreads();
+    }
+}
+
+// Sorts s[pad_index(i)], i < off[nrun] <= NT*IPT, that already holds nrun sorted
+// runs with bounds off[] (multiples of IPT): log2(nrun) merge rounds.  Every
+// thread of the workgroup must call it, after a barrier behind the writes; it
+// ends with a barrier.  -0 and NaN as in lds_sort.
+template <int NT, int IPT>
+__device__ __forceinline__ void lds_merge_runs(double *s, const int *off, int nrun) {
+    const int d0 = threadIdx.x * IPT;
+    const bool act = d0 < off[nrun];
+    int odd = 0, own = 0;
+    double v[IPT];
+    if (act) {
+        for (int c = 1; c < nrun; ++c)
+            if (off[c] <= d0) own = c;
+#pragma unroll
+        for (int q = 0; q < IPT; ++q) {
+            const double x = s[pad_index(d0 + q)];
+            odd |= (x != x) | (x == 0.0 && signbit(x));
+        }
+    }
+    if (__syncthreads_or(odd)) lds_merge_rounds<IPT, false>(s, off, nrun, own, d0, act, v);
+    else lds_merge_rounds<IPT, true>(s, off, nrun, own, d0, act, v);
 }
 
 // Sorts the n values at s[pad_index(i)], i < n <= NT*IPT, in place.  Every
