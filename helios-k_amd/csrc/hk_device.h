@@ -207,7 +207,7 @@ __device__ __forceinline__ double rew_core64(double x, double y, double ey, doub
 // with dtab[-5..0] = 0 so that the downward terms below n = 1 vanish without a
 // branch or a clamp of their index (a clamp per term: 1e7 lines on 3e7 points
 // 18.6 ms, this 17.5).
-// As in the FP64 core, each series is built from two hardware exponentials by
+// As in rew_core64, each series is built from two hardware exponentials by
 // the ratio recurrences (4 exponentials per pair instead of 19); the
 // recurrences add < 7 roundings per term (< 5e-7 relative).
 constexpr int kNT32 = 13;
@@ -271,7 +271,7 @@ __device__ __noinline__ double rew916_64(double x, double y) {
     return rew_core64(x, y, erfcx(y), core_q1(y, kA64, kN64));
 }
 
-// Re w for any r2 in FP64 (used by the adjoint and by tests of the pieces).
+// Re w for any r2 in FP64 (the plinth of a line).
 __device__ __forceinline__ double rew64(double x, double y) {
     double x2 = x * x, r2 = fma(y, y, x2);
     if (r2 >= kRF64) {
@@ -283,108 +283,6 @@ __device__ __forceinline__ double rew64(double x, double y) {
     if (r2 >= kRM64) return (2.0 / kPi) * y * gh4_sum64(x2, r2);
     if (r2 >= kRB64) return (2.0 / kPi) * y * gh8_sum64(x2, r2);
     return rew916_64(x, y);
-}
-
-// --------------------------------------------------------------------------
-// Complex w in FP64 (real and imaginary part), same regions as rew64.  The
-// adjoint needs Im w for w'(z) = -2 z w(z) + 2i/sqrt(pi).
-//  asymptotic: w ~ (i/sqrt(pi)) (1/z + 1/(2 z^3) + 3/(4 z^5))
-//  Gauss-Hermite pair: Im = (2x/pi) w_k (r2 - t_k^2) / D_k
-//  Algorithm 916: Im w = -e^{-x^2} erfcx(y) sin 2xy + (2a/pi) [x e^{-x^2}
-//    sinc(2xy) + y sin(2xy) s1 + s4/2 - s5/2],  s4 = sum a n e^{-(an-x)^2}/
-//    (a^2n^2+y^2), s5 = sum a n e^{-(an+x)^2}/(a^2n^2+y^2).
-// --------------------------------------------------------------------------
-__device__ __noinline__ void w916_64(double x, double y, double &re, double &im) {
-    constexpr double a = 0.529275382982092;
-    constexpr int N1 = 13;
-    double sgn = x < 0.0 ? -1.0 : 1.0;
-    x = fabs(x);
-    if (x == 0.0) { re = erfcx(y); im = 0.0; return; }
-    double xx = x * x, yy = y * y;
-    double ex2 = exp(-xx);
-    double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0, s5 = 0.0;
-    for (int n = 1; n <= N1; ++n) {
-        double an = a * n;
-        double inv = 1.0 / (an * an + yy);
-        double e2 = exp(-(an + x) * (an + x)) * inv;
-        s1 += exp(-(an * an + xx)) * inv;
-        s2 += e2;
-        s5 += an * e2;
-    }
-    int n0 = (int)ceil(x / a);
-    for (int k = -N1; k <= N1; ++k) {
-        int n = n0 + k;
-        if (n < 1) continue;
-        double an = a * n, d = an - x;
-        double e3 = exp(-d * d) / (an * an + yy);
-        s3 += e3;
-        s4 += an * e3;
-    }
-    double xy = x * y, sxy, cxy;
-    sincos(xy, &sxy, &cxy);
-    double c2 = fma(cxy, cxy, -sxy * sxy), s2xy = 2.0 * sxy * cxy;
-    double sinc1 = xy < 1e-8 ? 1.0 : sxy / xy;
-    double sinc2 = xy < 1e-8 ? 1.0 : s2xy / (2.0 * xy);
-    constexpr double ca = 2.0 * a / kPi;
-    double ex = erfcx(y);
-    re = y == 0.0 ? ex2 : ex2 * ex * c2 + ca * (sxy * x * sinc1 * ex2 + y * (-c2 * s1 + 0.5 * (s2 + s3)));
-    im = sgn * (-ex2 * ex * s2xy + ca * (x * ex2 * sinc2 + y * s2xy * s1 + 0.5 * s4 - 0.5 * s5));
-}
-
-__device__ __forceinline__ void w64(double x, double y, double &re, double &im) {
-    double x2 = x * x, r2 = fma(y, y, x2), y2 = y * y;
-    if (r2 >= kRF64) {
-        double inv = rcp64(r2), q = inv * inv;
-        double cr = 1.0 + fma(3.0, x2, -y2) * 0.5 * q
-                  + 0.75 * fma(fma(5.0, x2, -10.0 * y2), x2, y2 * y2) * q * q;
-        double ci = 1.0 + fma(-3.0, y2, x2) * 0.5 * q
-                  + 0.75 * fma(fma(-10.0, y2, x2), x2, 5.0 * y2 * y2) * q * q;
-        re = y * kISqrtPi * inv * cr;
-        im = x * kISqrtPi * inv * ci;
-        return;
-    }
-    if (r2 >= kRB64) {
-        double sr = 0.0, si = 0.0;
-        if (r2 >= kRM64) {
-            const double t[2] = {kGH4t1, kGH4t2}, w[2] = {kGH4w1, kGH4w2};
-            for (int k = 0; k < 2; ++k) {
-                double a = t[k] * t[k], u = r2 + a;
-                double iD = rcp64(fma(u, u, -4.0 * a * x2));
-                sr = fma(w[k] * u, iD, sr);
-                si = fma(w[k] * (r2 - a), iD, si);
-            }
-        } else {
-            const double t[4] = {kGH8t1, kGH8t2, kGH8t3, kGH8t4};
-            const double w[4] = {kGH8w1, kGH8w2, kGH8w3, kGH8w4};
-            for (int k = 0; k < 4; ++k) {
-                double a = t[k] * t[k], u = r2 + a;
-                double iD = rcp64(fma(u, u, -4.0 * a * x2));
-                sr = fma(w[k] * u, iD, sr);
-                si = fma(w[k] * (r2 - a), iD, si);
-            }
-        }
-        re = (2.0 / kPi) * y * sr;
-        im = (2.0 / kPi) * x * si;
-        return;
-    }
-    w916_64(x, y, re, im);
-}
-
-// dRe w/dx = Re w'(z) and dRe w/dy = -Im w'(z) for |z|^2 >= 1e4 from the
-// asymptotic series w'(z) = -(i/sqrt(pi)) u (1 + 3/2 u + 15/4 u^2 + 105/8 u^3),
-// u = 1/z^2 (next term below 6e-15 relative).  The identity
-// w' = -2zw + 2i/sqrt(pi) cancels to ~eps |z|^2 there.
-__device__ __forceinline__ void drew_far64(double x, double y, double r2, double &ddx,
-                                           double &ddy) {
-    const double inv = rcp64(r2);
-    const double ur = (x - y) * (x + y) * inv * inv, ui = -2.0 * (x * inv) * (y * inv);
-    double pr = 13.125 * ur + 3.75, pi = 13.125 * ui;
-    double tr = pr * ur - pi * ui, ti = pr * ui + pi * ur;
-    pr = tr + 1.5; pi = ti;
-    tr = pr * ur - pi * ui; ti = pr * ui + pi * ur;
-    pr = tr + 1.0; pi = ti;
-    ddx = (ur * pi + ui * pr) * kISqrtPi;
-    ddy = (ur * pr - ui * pi) * kISqrtPi;
 }
 
 }  // namespace hk

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
 
 template <int PROFILE, bool PLINTH, bool CHI = false>
 void launch_profile(hipStream_t s, const PArgs &a) {
-    const int ppt = default_ppt64(a.nx);
+    const int ppt = default_ppt64(a.nx, false);
     const dim3 g((unsigned)((a.nx + kThreads * ppt - 1) / (kThreads * ppt))), b(kThreads);
     if (ppt == 1) hipLaunchKernelGGL((profile_tiles_kernel<1, PROFILE, PLINTH, CHI>), g, b, 0, s, a);
     else hipLaunchKernelGGL((profile_tiles_kernel<2, PROFILE, PLINTH, CHI>), g, b, 0, s, a);

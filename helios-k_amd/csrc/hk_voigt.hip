@@ -496,16 +496,8 @@ __device__ __forceinline__ float far_node32(float x, float y) {
     return -(si * zr + sr * zi) * (float)(1.0 / kPi);
 }
 
-// DPP move of a double: each lane takes the value of the lane that the
-// (compile-time) DPP control selects; rows outside row_mask keep 0.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double dpp64(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROW_MASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xf, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
+// DPP move: each lane takes the value of the lane that the (compile-time) DPP
+// control selects; rows outside row_mask keep 0.
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ float dpp32(float v) {
     return __int_as_float(
@@ -1408,7 +1400,7 @@ __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_ke
     const int64_t tile = blockIdx.x;
     if (MODE == HK_VOIGT_FP64) {
         __shared__ Far64LDS sh;
-        tile_f64<PPT, LineSum<1, false, false>>(a, tile, &sh);
+        tile_f64<PPT, LineSum<1, false, false, (PPT == 4 || PPT == 8)>>(a, tile, &sh);
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
@@ -1479,7 +1471,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
         if constexpr (PPT == 0) {
             core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
-            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false>>(a, tile, (Far64LDS *)smem);
+            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false, (PPT == 4 || PPT == 8)>>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
         }
     }
@@ -1661,7 +1653,7 @@ namespace {
 //  FP64   default_ppt64.
 int pick_ppt(int mode, const hk_tune *tune, int64_t nx) {
     if (tune && tune->tile_points > 0) return tune->tile_points / kThreads;
-    return mode == HK_VOIGT_FP64 ? default_ppt64(nx) : 4;
+    return mode == HK_VOIGT_FP64 ? default_ppt64(nx, tune && tune->exact_pairs) : 4;
 }
 
 // tile_points a caller may ask for: 512, 1024, 2048 or 4096 (256-point tiles

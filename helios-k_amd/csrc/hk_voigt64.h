@@ -55,7 +55,14 @@ constexpr double kU64[kFN64 / 2] = {0.99691733373312796, 0.97236992039767667, 0.
 // Grids of fewer than four 512-point tiles per CU take 256-point tiles: 1e4
 // points 73 against 106 us, 3e4 points under 1e5 lines 1.12 / 1.97 ms, 3e5
 // points 665 / 805 us; at 1e6 points the two are equal.
-inline int default_ppt64(int64_t nx) { return (nx + 511) / 512 < 1024 ? 1 : 2; }
+// With every pair evaluated, longer grids take 1024 or 2048 points, so that a
+// line's broadcast serves four or eight points a lane: 1e7 lines, 3e7 points 884
+// ms with 512-point tiles, 572 with 1024, 566 with 2048; 1e5 lines, 3e6 points
+// 3.6, 2.6 and 2.5 ms.  Below 1024 tiles of 2048 points the chip is not full.
+inline int default_ppt64(int64_t nx, bool exact) {
+    if ((nx + 511) / 512 < 1024) return 1;
+    return !exact ? 2 : (nx + 2047) / 2048 < 1024 ? 4 : 8;
+}
 
 // lines taken per round of the tile loop (each wave lists its own quarter)
 constexpr int kRound64 = 4096;
@@ -209,10 +216,12 @@ __device__ __forceinline__ bool chi_piece(const Chi &c, double xa, double xb, do
 // What a line contributes to a point: PROFILE 1 Voigt, 2 Lorentz, 3 Doppler,
 // 4 binned Gaussian, 0 nothing but the plinth; PLINTH subtracts the line's
 // value at its cut (args.pl) over its whole window; CHI applies args.chi.
-template <int PROFILE_, bool PLINTH_, bool CHI_>
+// WHOLE: lines that have one wing formula over all of a wave's points take
+// add_wing (worth its registers where every pair is evaluated: nearly all do).
+template <int PROFILE_, bool PLINTH_, bool CHI_, bool WHOLE_ = false>
 struct LineSum {
     static constexpr int PROFILE = PROFILE_;
-    static constexpr bool PLINTH = PLINTH_, CHI = CHI_;
+    static constexpr bool PLINTH = PLINTH_, CHI = CHI_, WHOLE = WHOLE_;
     // wings that the nodes can take, or a value that underflows to zero beyond
     // x = kDopplerEnd (e^-x^2 does at 27.3)
     static constexpr bool WINGS = PROFILE == 1 || PROFILE == 2;
@@ -602,6 +611,24 @@ __device__ __forceinline__ void add_points(const Args &a, uint32_t code, double 
     }
 }
 
+// A line that covers the wave's 64 PPT points with one wing formula (N: 2 for
+// x^2 + y^2 >= 1e4, 4 for >= 100): all of a lane's points side by side, so that
+// their reciprocals' chains overlap (every pair of 1e7 lines on 3e7 points, tiles
+// of 1024: 780 ms a segment at a time, 572 so).
+template <int N, int PPT, class Args>
+__device__ __forceinline__ void add_wing(const Args &a, double nu, double ia, double y, double G,
+                                         double jd, double (&acc)[PPT]) {
+    const double y2 = y * y;
+    const GH<N> gh;
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) {
+        const double x = (fma(jd + (double)(64 * k), a.dnu, a.numin) - nu) * ia;
+        double num, den;
+        gh_frac(gh, x * x, fma(x, x, y2), num, den);
+        acc[k] = fma(G, num * rcp64(den), acc[k]);
+    }
+}
+
 template <int PPT, class P, class Args>
 __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *sh) {
     constexpr int W = kThreads * PPT, WP = 64 * PPT;
@@ -805,7 +832,18 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 const int b = __builtin_ctzll(m);
                 m &= m - 1ull;
                 const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
-                add_points<P, PPT>(a, (uint32_t)__builtin_amdgcn_readlane((int)code, b),
+                const uint32_t scode = (uint32_t)__builtin_amdgcn_readlane((int)code, b);
+                if constexpr (P::WHOLE) {
+                    constexpr uint32_t ones = 0x55555555u & (uint32_t)((1ull << (2 * PPT)) - 1);
+                    if (slo == 0 && shi == WP && (scode == ones || scode == 2 * ones)) {
+                        const double lnu = lane_f64(nu, b), lia = lane_f64(ia, b);
+                        const double ly = lane_f64(y, b), lG = lane_f64(G, b);
+                        if (scode == ones) add_wing<2, PPT>(a, lnu, lia, ly, lG, jd, acc);
+                        else add_wing<4, PPT>(a, lnu, lia, ly, lG, jd, acc);
+                        continue;
+                    }
+                }
+                add_points<P, PPT>(a, scode,
                                    lane_f64(nu, b), lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b),
                                    P::PROFILE == 1 ? lane_f64(Apf, b) : 0.0,
                                    P::PLINTH ? lane_f64(pl, b) : 0.0, slo, shi,
