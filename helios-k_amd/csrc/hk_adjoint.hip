@@ -19,8 +19,9 @@
 // f_k at the interval's 20 Chebyshev nodes, so
 //   sum_j gK_j f(x_j) = sum_k f_k G_k,   G_k = sum_j gK_j l_k(x_j),
 // with l_k the nodes' Lagrange polynomials.  A workgroup owns 256 consecutive
-// lines, one per lane, and walks the 1024-point tiles their windows reach: it
-// forms the G_k of the tile, and of its four quarters and 16 segments where
+// lines, one per lane (64 of a short list, its waves sharing their work), and
+// walks the 1024-point tiles (256 or 512 for short lists) that their windows
+// reach: it forms the G_k of the tile, and of its four quarters and 16 segments where
 // some line is near, and each lane evaluates its line at the nodes of the
 // largest far interval; what is left (~4 segments a line) is summed point by
 // point, 64 points at a time.
@@ -239,9 +240,11 @@ __device__ __forceinline__ int far_class_adj(double D, double half, double ia, d
 
 // Adds the lane's line at the interval's nodes (class cls != 0) to its sums.
 __device__ __forceinline__ void add_far(int cls, double D, double half, double ia, double y,
-                                        const double *G, const double *u, double (&A)[4]) {
+                                        const double *G, const double *u, double (&A)[4],
+                                        int k0 = 0, int k1 = kFN64) {
     const double xc = D * ia, h = half * ia;
-    for (int k = 0; k < kFN64; ++k) {
+#pragma unroll 5
+    for (int k = k0; k < k1; ++k) {
         const double x = fma(u[k], h, xc), r2 = fma(x, x, y * y), g = G[k];
         const WD v = cls == 2 ? wd_far(x, y, r2) : wd_mid(x, y, r2);
         A[0] = fma(g, v.re, A[0]);
@@ -251,13 +254,20 @@ __device__ __forceinline__ void add_far(int cls, double D, double half, double i
     }
 }
 
+// LPB lines per workgroup: 256, one per lane of its four waves, or 64 that all
+// four waves hold, each for a quarter of the tiles' points and nodes.
+// TILE points per tile (kATile at most).
+template <int LPB, int TILE>
 __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
     __shared__ AdjLDS sh;
+    constexpr int kATile = TILE, kASub = TILE / kASubs, kASegs = TILE / kASeg;
+    static_assert(kASub % 64 == 0 && TILE % kAT == 0, "the tile's tables");
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int64_t blk = blockIdx.x;
     const int part = blockIdx.y;
-    const int64_t i = blk * kAT + t;
+    constexpr bool kShared = LPB == 64;
+    const int64_t i = kShared ? blk * LPB + lane : blk * LPB + t;
     if (t < 4 * kFN64) sh.cosv[t] = cospi((double)t / (2.0 * kFN64));
     if (t < kFN64) sh.u[t] = cospi((2.0 * t + 1.0) / (2.0 * kFN64));
     LineD r = {};
@@ -366,11 +376,14 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
                 (&sh.Gs[0][0])[e] = node_weight(sh.Ms[0] + row * kFN64, sh.cosv, k);
             }
         __syncthreads();
-        if (cls0) add_far(cls0, centre(0, Wv) - nu, half(Wv), ia, y, sh.G0, sh.u, A);
+        if (cls0)
+            add_far(cls0, centre(0, Wv) - nu, half(Wv), ia, y, sh.G0, sh.u, A,
+                    kShared ? wave * (kFN64 / kWaves) : 0,
+                    kShared ? (wave + 1) * (kFN64 / kWaves) : kFN64);
         if (!anyn) continue;
         // quarters, then segments, then points: bit s of todo = segment s left
         unsigned todo = 0;
-        for (int q = 0; q < kASubs; ++q) {
+        for (int q = kShared ? wave : 0; q < (kShared ? wave + 1 : kASubs); ++q) {
             const int f0 = q * kASub, n = valid(f0, kASub);
             const bool inq = near && wl < f0 + n && wh > f0;
             int cls = 0;
@@ -441,14 +454,30 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
             if (lane == b) { A[0] += z0; A[1] += z1; A[2] += z2; A[3] += z3; }
         }
     }
+    bool own = i < a.nl;
+    if constexpr (kShared) {
+        // the four waves' sums of each line, by wave 0
+        static_assert(kWaves == kASubs && sizeof(sh.g) >= sizeof(double) * kWaves * 4 * 64,
+                      "one quarter per wave; sums fit the tile's gradient");
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sh.g[(wave * 4 + q) * 64 + lane] = A[q];
+        __syncthreads();
+        own = own && wave == 0;
+        if (own)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                A[q] = ((sh.g[q * 64 + lane] + sh.g[(4 + q) * 64 + lane]) +
+                        sh.g[(8 + q) * 64 + lane]) + sh.g[(12 + q) * 64 + lane];
+    }
     if (a.parts > 1) {
-        if (i < a.nl)
+        if (own)
 #pragma unroll
             for (int q = 0; q < 4; ++q) a.sums[((int64_t)part * 4 + q) * a.nl + i] = A[q];
         return;
     }
     double gT = 0.0, gP = 0.0;
-    if (i < a.nl) line_grads(a, r, i, A[0], A[1], A[2], A[3], gT, gP);
+    if (own) line_grads(a, r, i, A[0], A[1], A[2], A[3], gT, gP);
     for (int off = 32; off > 0; off >>= 1) {
         gT += __shfl_xor(gT, off, 64);
         gP += __shfl_xor(gP, off, 64);
@@ -468,6 +497,7 @@ __global__ __launch_bounds__(kAT) void adjoint_combine_kernel(AArgs a) {
     double gT = 0.0, gP = 0.0;
     if (i < a.nl) {
         double A[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
         for (int p = 0; p < a.parts; ++p)
 #pragma unroll
             for (int q = 0; q < 4; ++q) A[q] += a.sums[((int64_t)p * 4 + q) * a.nl + i];
@@ -499,14 +529,31 @@ __global__ __launch_bounds__(1024) void sum_rows_kernel(const double *__restrict
     if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
+// Lines per workgroup: 64 for short lists, whose 256 neighbours spread over many
+// tiles, each near few of them, so that one wave went through all of a tile's
+// intervals for a few lanes; and narrower tiles the fewer workgroups there are.
+// Adjoint of 1000, 4000, 16000, 60000 lines with 256 lines and 1024 points 191,
+// 199, 376, 756 us; with 64 lines and 1024 points 81, 102, 227, 690, with 512
+// points 61, 83, 241, 653, with 256 points 43, 91, 272, 699.  2e5 lines: 1355 us
+// with 256 lines, which share a tile's G_k, 1880 with 64.
+constexpr int64_t kATiny = 3000;
+int adjoint_lines(int64_t nlines) { return nlines < 65536 ? 64 : kAT; }
+
 // Lists short of filling the chip several times over split each line's tiles
-// over several workgroups, at most 32: up to ~20 workgroups per CU (256 lines
-// each), since a workgroup's barriers leave its CU to the others.  3.3e5 lines,
-// 11 tiles a window: 1 part 2.60 ms, 2 parts 2.28, 4 parts 2.15, 8 parts 2.32.
+// over several workgroups, at most 32: up to ~20 workgroups per CU, since a
+// workgroup's barriers leave its CU to the others.  3.3e5 lines, 11 tiles a
+// window: 1 part 2.60 ms, 2 parts 2.28, 4 parts 2.15, 8 parts 2.32.
 int adjoint_parts(int64_t nlines) {
-    const int64_t nblocks = (nlines + kAT - 1) / kAT;
+    const int64_t nblocks = (nlines + adjoint_lines(nlines) - 1) / adjoint_lines(nlines);
     const int64_t p = nblocks > 0 ? 5300 / nblocks : 1;
     return (int)(p < 1 ? 1 : (p > 32 ? 32 : p));
+}
+
+// Workgroups whose partial dL/dT, dL/dP the last kernel adds: of the main kernel
+// or, with parts, of the combination.
+int64_t adjoint_sums(int64_t nlines) {
+    const int per = adjoint_parts(nlines) > 1 ? kAT : adjoint_lines(nlines);
+    return (nlines + per - 1) / per;
 }
 
 }  // namespace
@@ -514,8 +561,7 @@ int adjoint_parts(int64_t nlines) {
 extern "C" size_t hk_voigt_adjoint_workspace_bytes(int64_t nlines) {
     if (nlines < 0) return 0;
     const int parts = adjoint_parts(nlines);
-    const int64_t nblocks = (nlines + kAT - 1) / kAT;
-    return (size_t)(2 * nblocks + (parts > 1 ? 4 * parts * nlines : 0) + 2) * sizeof(double) + 256;
+    return (size_t)(2 * adjoint_sums(nlines) + (parts > 1 ? 4 * parts * nlines : 0) + 2) * sizeof(double) + 256;
 }
 
 extern "C" int hk_voigt_adjoint(const hk_lines *L, const hk_tp *tp, const hk_cut *cut,
@@ -545,13 +591,18 @@ extern "C" int hk_voigt_adjoint(const hk_lines *L, const hk_tp *tp, const hk_cut
     a.cut_mode = cut->cut_mode; a.cut = cut->cut == 0.0 ? 1.0e30 : cut->cut;
     a.numin = g->numin; a.dnu = g->dnu; a.nx = g->nx; a.gK = gK; a.gS = gS; a.gvy = gvy;
     a.parts = adjoint_parts(L->nlines);
-    a.nblocks = (L->nlines + kAT - 1) / kAT;
+    a.nblocks = adjoint_sums(L->nlines);
     a.part_tp = (double *)hk::align_up((size_t)ws, 256);
     a.sums = a.part_tp + 2 * a.nblocks;
     hipStream_t s = (hipStream_t)stream;
     if (a.nblocks > 0) {
-        hipLaunchKernelGGL(adjoint_kernel, dim3((unsigned)a.nblocks, (unsigned)a.parts), dim3(kAT),
-                           0, s, a);
+        const int lines = adjoint_lines(L->nlines);
+        const dim3 grid((unsigned)((L->nlines + lines - 1) / lines), (unsigned)a.parts);
+        if (lines == 64 && L->nlines < kATiny)
+            hipLaunchKernelGGL((adjoint_kernel<64, 256>), grid, dim3(kAT), 0, s, a);
+        else if (lines == 64)
+            hipLaunchKernelGGL((adjoint_kernel<64, 512>), grid, dim3(kAT), 0, s, a);
+        else hipLaunchKernelGGL((adjoint_kernel<kAT, kATile>), grid, dim3(kAT), 0, s, a);
         HK_LAUNCH_CHECK();
         if (a.parts > 1) {
             hipLaunchKernelGGL(adjoint_combine_kernel, dim3((unsigned)a.nblocks), dim3(kAT), 0, s,
