@@ -59,7 +59,7 @@ CLOCK_GHZ = 2.4
 N_CU = 256
 # Kernels are named by the prefix of their demangled name as rocprofv3 prints it.
 # One FP32C Voigt sum of the single-spectrum form at the default 1024-point tiles.
-VOIGT_KERNELS_SINGLE = ("void hk::voigt_tiles_kernel<1, 4, 1>(", "void hk::voigt_core_kernel<1>(")
+VOIGT_KERNELS_SINGLE = ("void hk::voigt_tiles_kernel<1, 4, 1>(", "hk::voigt_core_kernel(")
 # The batched form's two persistent kernels: main pass at tile 512..4096 points
 # (256 x points per thread) with 256 or 512 lines per LDS stage (256 x stages), and
 # the line-core pass.

@@ -1400,7 +1400,7 @@ __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_ke
     const int64_t tile = blockIdx.x;
     if (MODE == HK_VOIGT_FP64) {
         __shared__ Far64LDS sh;
-        tile_f64<PPT, LineSum<1, false, false, (PPT == 4 || PPT == 8)>>(a, tile, &sh);
+        tile_f64<PPT, LineSum<1, false, false, (PPT >= 4)>>(a, tile, &sh);
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
@@ -1428,11 +1428,12 @@ __global__ __launch_bounds__(256) void voigt_core_kernel(VArgs a) {
 // or per tile, outside the record loops: c2's batched sum 1070 ms at 4, 964
 // at 5, 891 at 6), 3 with 512-line stages (LDS allows 3 workgroups per CU) and
 // for 2048-point tiles (without a floor the far-field code raises the
-// register count of the persistent form enough to halve its occupancy); the
-// FP64 main pass 4; the FP32 line-core pass 5 (as its one-spectrum kernel has
+// register count of the persistent form enough to halve its occupancy), 2 for
+// 4096-point tiles (20.7 ms at two waves, 30.2 at the one that 256 registers
+// allow without a floor: 5e6 lines, 3e6 points); the FP64 main pass 4; the FP32 line-core pass 5 (as its one-spectrum kernel has
 // without a floor).
 constexpr int main_waves(int mode, int ppt, int lm) {
-    return ppt <= 4 ? (lm == 2 ? 3 : (mode == HK_VOIGT_FP32C ? 6 : 4)) : (ppt == 8 ? 3 : 1);
+    return ppt <= 4 ? (lm == 2 ? 3 : (mode == HK_VOIGT_FP32C ? 6 : 4)) : (ppt == 8 ? 3 : 2);
 }
 
 template <int MODE, int PPT, int LM>
@@ -1471,7 +1472,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
         if constexpr (PPT == 0) {
             core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
-            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false, (PPT == 4 || PPT == 8)>>(a, tile, (Far64LDS *)smem);
+            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false, (PPT >= 4)>>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
         }
     }
