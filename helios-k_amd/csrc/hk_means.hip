@@ -199,6 +199,17 @@ __device__ __forceinline__ double wave_min64(double v) {
                 fmin(hk::lane_f64(v, 32), hk::lane_f64(v, 48)));
 }
 
+// Whether nodes may stand for a cluster of this half width: 1 / half is finite
+// (subnormal spans, e.g. of tails that underflow, are summed value by value).
+__device__ __forceinline__ bool tr_half_ok(double half) { return !(half > 0.0 && half < 1.0e-290); }
+
+// Place in [-1, 1] of a value that lies d above the cluster's least.  From the
+// difference, not from a midpoint: that of two neighbouring doubles rounds onto
+// one of them, and T_19 of a place of +-2 is 4e10.
+__device__ __forceinline__ double tr_place(double d, double half, double ih) {
+    return fmin(fmax((d - half) * ih, -1.0), 1.0);
+}
+
 struct TrCluster {
     double lo, half;
     int n, nodes;            // points; whether the nodes may stand for them
@@ -275,8 +286,8 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
                 }
                 lo = wave_min64(lo);
                 hi = -wave_min64(-hi);
-                const bool nodes = __ballot(!fin) == 0ull;
-                const double half = 0.5 * (hi - lo), mid = 0.5 * (hi + lo);
+                const double half = 0.5 * (hi - lo);
+                const bool nodes = __ballot(!fin) == 0ull && tr_half_ok(half);
                 if (nodes) {
                     double f[kFN64];
 #pragma unroll
@@ -284,10 +295,11 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
                     const double ih = half > 0.0 ? 1.0 / half : 0.0;
 #pragma unroll
                     for (int q = 0; q < kTrC / 64; ++q)
-                        add_moments20(lane + 64 * q < n ? 1.0 : 0.0, (v[q] - mid) * ih, f);
+                        add_moments20(lane + 64 * q < n ? 1.0 : 0.0, tr_place(v[q] - lo, half, ih),
+                                      f);
                     add_node_totals(f, M + (c - c3) * kFN64);
                 }
-                // (a cluster with undefined or infinite values is never skipped)
+                // (without nodes -- undefined or infinite values -- never skipped)
                 if (lane == 0) cl[c] = TrCluster{nodes ? lo : -INFINITY, half, n, nodes ? 1 : 0};
             }
             wave_lds_sync();
@@ -300,14 +312,16 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
         const int nsc = (ncl + kTrSuper - 1) / kTrSuper;
         for (int h = wave; h < nsc; h += kTrWaves) {
             const int c0 = h * kTrSuper, nc = min(kTrSuper, ncl - c0);
-            double lo = INFINITY, hi = -INFINITY;
+            double lo = INFINITY, span = 0.0;
             int ok = 1;
             for (int c = c0; c < c0 + nc; ++c) {
                 lo = fmin(lo, cl[c].lo);
-                hi = fmax(hi, fma(2.0, cl[c].half, cl[c].lo));
                 ok &= cl[c].nodes;
             }
-            const double half = 0.5 * (hi - lo), mid = 0.5 * (hi + lo);
+            for (int c = c0; c < c0 + nc; ++c)
+                span = fmax(span, fma(2.0, cl[c].half, cl[c].lo - lo));
+            const double half = 0.5 * span;
+            ok &= tr_half_ok(half);
             if (ok) {
                 double f[kFN64];
 #pragma unroll
@@ -315,8 +329,9 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
                 const double ih = half > 0.0 ? 1.0 / half : 0.0;
                 for (int q = lane; q < kTrSuper * kFN64; q += 64) {
                     const int c = c0 + min(q / kFN64, nc - 1), k = q % kFN64;
-                    const double K = fma(cl[c].half, 1.0 + cosv[2 * k + 1], cl[c].lo);
-                    add_moments20(q / kFN64 < nc ? Gp[k >> 2][c][k & 3] : 0.0, (K - mid) * ih, f);
+                    const double K = fma(cl[c].half, 1.0 + cosv[2 * k + 1], cl[c].lo - lo);
+                    add_moments20(q / kFN64 < nc ? Gp[k >> 2][c][k & 3] : 0.0,
+                                  tr_place(K, half, ih), f);
                 }
                 double *M = Mw[wave];
                 wave_lds_sync();
