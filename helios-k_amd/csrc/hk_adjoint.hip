@@ -268,8 +268,8 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
     const int part = blockIdx.y;
     constexpr bool kShared = LPB == 64;
     const int64_t i = kShared ? blk * LPB + lane : blk * LPB + t;
-    if (t < 4 * kFN64) sh.cosv[t] = cospi((double)t / (2.0 * kFN64));
-    if (t < kFN64) sh.u[t] = cospi((2.0 * t + 1.0) / (2.0 * kFN64));
+    if (t < 4 * kFN64) sh.cosv[t] = cos40(t);
+    if (t < kFN64) sh.u[t] = node_u(t);
     LineD r = {};
     int64_t jlo = 0, jhi = 0;
     if (i < a.nl) {

@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     // this lane's m of group g: t0 + 16 (wave + 8 g) + lane / 4
     const int t0 = blockIdx.x * kTrPer + 16 * wave + (lane >> 2);
     auto m_of = [&](int g) { return exp((double)(t0 + 16 * kTrWaves * g - nTr / 2) * dTr); };
-    if (tid < 4 * kFN64) cosv[tid] = cospi((double)tid / (2.0 * kFN64));
+    if (tid < 4 * kFN64) cosv[tid] = cos40(tid);
     double least = INFINITY;
     for (int k = tid; k < Nxb; k += kTrThreads) least = fmin(least, Kb[k]);
     least = wave_min64(least);
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     double un[kFN64 / 4];                  // (K - lo) / half at this lane's nodes
 #pragma unroll
     for (int k = 0; k < kFN64 / 4; ++k)
-        un[k] = 1.0 + cospi((2.0 * (4 * k + part) + 1.0) / (2.0 * kFN64));
+        un[k] = 1.0 + node_u(4 * k + part);
     for (int k0 = 0; k0 < Nxb; k0 += kTrC * kTrBatch) {
         const int ncl = min(kTrBatch, (Nxb - k0 + kTrC - 1) / kTrC);
         __syncthreads();                    // the previous batch's readers are done

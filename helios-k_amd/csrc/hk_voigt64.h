@@ -16,8 +16,11 @@
 // carried to the wave's nodes), evaluated once per point in FP64.
 //
 // Truncation: the worst line (centre at the band's inner edge, zero width:
-// a double pole) interpolates to 5e-15 of its value, largest at the tile end
-// nearest the line; everything else is FP64 rounding, as in the pair sum.
+// a double pole) interpolates to 3.3e-16 of its value, largest at the tile end
+// nearest the line; everything else is FP64 rounding, as in the pair sum (one
+// line alone: 1.3e-15 of its value at most, pair by pair 9e-16; sums of 20000
+// lines 2e-15, pair by pair 1e-14).  At 3.25 half widths 5e-15 were left, for
+// 1 to 5 % less time.
 // The nodes and the points are placed relative to the tile centre, so the
 // rounding of x_j = fma(j, dnu, numin) enters the far field exactly as it
 // enters a pair.
@@ -38,15 +41,25 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 
 constexpr int kFN64 = 20;                 // Chebyshev-Gauss nodes
-constexpr double kFarRatio64 = 3.25;
+constexpr double kFarRatio64 = 3.7;
 // Largest x^2 + y^2 of a far line: keeps the products of the 8-node rule
 // (~ r2^16 for a pair of nodes) in range.
 constexpr double kFarMaxR2 = 1.0e18;
-// cos(pi (k + 1/2) / 20), k = 0..9; node 19 - k is its negative
-constexpr double kU64[kFN64 / 2] = {0.99691733373312796, 0.97236992039767667, 0.92387953251128674,
-                                    0.85264016435409218, 0.76040596560003093, 0.64944804833018377,
-                                    0.52249856471594880, 0.38268343236508984, 0.23344536385590542,
-                                    0.078459095727844999};
+// cos(j pi / 40), j = 0..20, correctly rounded: a table of cospi(j / 40.0), whose
+// argument rounds, put 3e-15 of a far line on the tile's ends
+__device__ constexpr double kCos40[kFN64 + 1] = {
+    1.0, 0.996917333733128, 0.9876883405951378, 0.9723699203976766, 0.9510565162951535,
+    0.9238795325112867, 0.8910065241883679, 0.8526401643540922, 0.8090169943749475,
+    0.7604059656000309, 0.7071067811865476, 0.6494480483301837, 0.5877852522924731,
+    0.5224985647159489, 0.4539904997395468, 0.3826834323650898, 0.30901699437494745,
+    0.23344536385590542, 0.15643446504023087, 0.07845909572784494, 0.0};
+// cos(j pi / 40), 0 <= j < 80
+__device__ __forceinline__ double cos40(int j) {
+    const int q = j > 2 * kFN64 ? 4 * kFN64 - j : j;
+    return q > kFN64 ? -kCos40[2 * kFN64 - q] : kCos40[q];
+}
+// Chebyshev-Gauss node k of 20, cos(pi (k + 1/2) / 20)
+__device__ __forceinline__ double node_u(int k) { return cos40(2 * k + 1); }
 // Points per thread of a tile (256 threads) when the caller leaves it open.
 // Halving the tile doubles the tile-level node evaluations and halves the point
 // sums; 512 points win over 1024 at 1e5 lines, 3e6 points, cut 100 (491 against
@@ -184,10 +197,11 @@ __device__ __forceinline__ double chi_exponent(const Chi &c, double d) {
     return fma(c.B1, c.s2 - c.s1, fma(c.B2, c.s3 - c.s2, c.B3 * (d - c.s3)));
 }
 
-// The factor over an interval on which it is one analytic piece:
-// exp(-(B (x - nu) + t0)) (1 + (x - nu) inv_nu); all 0 outside the range.
+// The factor over an interval on which it is one analytic piece, at u of its
+// half widths from its centre: exp(-(B (x - nu) + t0)) (c + u h), c + u h = x / nu
+// (1 + (x - nu) / nu would cancel far below the line); 1 outside the range.
 struct ChiPiece {
-    double B = 0.0, t0 = 0.0, inv_nu = 0.0;
+    double B = 0.0, t0 = 0.0, c = 1.0, h = 0.0;
 };
 
 // Finds the piece for the points xa..xb (D: the interval's centre from the
@@ -209,7 +223,9 @@ __device__ __forceinline__ bool chi_piece(const Chi &c, double xa, double xb, do
     } else return false;
     p.B = D < 0.0 ? -B : B;
     p.t0 = t0;
-    p.inv_nu = 1.0 / nu;
+    const double inv_nu = 1.0 / nu;
+    p.c = 0.5 * (xa + xb) * inv_nu;
+    p.h = half * inv_nu;
     return fabs(B) * half <= 2.0;
 }
 
@@ -327,7 +343,7 @@ __device__ __forceinline__ void add_nodes(double D, double half, double ia, doub
 #pragma unroll
     for (int k = 0; k < kFN64 / 2; ++k) {
         __builtin_amdgcn_sched_barrier(0);   // (pairs interleaved: spills)
-        const double u = local_const(kU64[k]);
+        const double u = local_const(kCos40[2 * k + 1]);
         const double xa = fma(u, h, xc), xb = fma(-u, h, xc);
         const double a2 = xa * xa, b2 = xb * xb;
         const double ra = a2 + y2, rb = b2 + y2;
@@ -350,8 +366,8 @@ __device__ __forceinline__ void add_nodes(double D, double half, double ia, doub
         }
         if (P::CHI) {
             const double ea = fma(u, half, D), eb = fma(-u, half, D);
-            va *= exp_neg(fma(chi.B, ea, chi.t0)) * fma(ea, chi.inv_nu, 1.0);
-            vb *= exp_neg(fma(chi.B, eb, chi.t0)) * fma(eb, chi.inv_nu, 1.0);
+            va *= exp_neg(fma(chi.B, ea, chi.t0)) * fma(u, chi.h, chi.c);
+            vb *= exp_neg(fma(chi.B, eb, chi.t0)) * fma(-u, chi.h, chi.c);
         }
         // (g last: strengths far below 1e-100 must not meet the products)
         f[k] = fma(g, va, f[k]);
@@ -410,16 +426,20 @@ __device__ __forceinline__ void clip_window(double nu, double hw, double numin, 
 }
 
 // Chebyshev coefficient m (lane m < 20) of the node values F: T_m(u_k) =
-// cos(m (2k + 1) pi / 40), cosv[j] = cos(j pi / 40).
+// cos(m (2k + 1) pi / 40), cosv[j] = cos(j pi / 40).  Nodes k and 19 - k share a
+// cosine up to its sign, and a middle value is taken off first: half the terms,
+// and smaller ones.
 __device__ __forceinline__ double cheb_coef64(const double *F, const double *cosv, int m) {
+    const double base = F[kFN64 / 2], sg = m & 1 ? -1.0 : 1.0;
     double c = 0.0;
     int j = m;
-    for (int k = 0; k < kFN64; ++k) {
-        c = fma(F[k], cosv[j], c);
+#pragma unroll
+    for (int k = 0; k < kFN64 / 2; ++k) {
+        c = fma(fma(sg, F[kFN64 - 1 - k] - base, F[k] - base), cosv[j], c);
         j += 2 * m;
         j -= j >= 4 * kFN64 ? 4 * kFN64 : 0;
     }
-    return (m == 0 ? 1.0 : 2.0) / (double)kFN64 * c;
+    return m == 0 ? fma(1.0 / (double)kFN64, c, base) : 2.0 / (double)kFN64 * c;
 }
 
 // Adds g T_m(u), m = 0..19, to f.
@@ -652,7 +672,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
 #pragma unroll
     for (int k = 0; k < PPT; ++k) acc[k] = 0.0;
     // line range of the tile: waves 0 and 1 search one end each
-    if (t < 4 * kFN64) sh->cosv[t] = cospi((double)t / (2.0 * kFN64));
+    if (t < 4 * kFN64) sh->cosv[t] = cos40(t);
     if (lane < kFN64) { sh->F[wave][lane] = 0.0; sh->wF[wave][lane] = 0.0; }
     if (wave < 2) {
         const double R = a.radius[0];
@@ -882,8 +902,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
             if (lane < kFN64) c[lane] = cm;
             wave_lds_sync();
             if (lane < kFN64) {
-                const double u = lane < kFN64 / 2 ? kU64[lane] : -kU64[kFN64 - 1 - lane];
-                wF[lane] += cheb_sum64(c, (fma(u, hw_w, xcw - xc)) / hW);
+                wF[lane] += cheb_sum64(c, (fma(node_u(lane), hw_w, xcw - xc)) / hW);
             }
             wave_lds_sync();
         }
