@@ -26,7 +26,7 @@
 // Voigt and Lorentz wings far from a tile or a wave through Chebyshev nodes
 // (with the sub-Lorentzian factor where it is one analytic piece there),
 // Doppler and binned-Gaussian lines only where they do not underflow to zero,
-// plinths of lines that cover a tile or a wave as one constant -- so a line
+// plinths taken off each value at nodes as at points -- so a line
 // costs a few hundred evaluations, not one per point of its window.  What bounds
 // it: FP64 vector instructions.  All arithmetic is FP64, in a fixed order.
 // Pair by pair, Voigt with chi over 2e4 lines, 1e5 points, cut 120 took 7.0 ms,

@@ -91,7 +91,7 @@ struct Far64LDS {
     double tab[kWaves][64];                     // core table of the wave's line
     double cosv[4 * kFN64];                     // cos(j pi / 40)
     uint64_t taken[kWaves][kRound64 / 64];      // lines of a chunk the wave's nodes took
-    double cst[kWaves];                         // plinths of lines that cover the tile
+    double cst[kWaves];                         // plinths alone: of lines that cover the tile
     int cnt[kWaves];
     int64_t range[2];
 };
@@ -329,10 +329,11 @@ __device__ __forceinline__ void gh_frac(const GH<4> &q, double x2, double r2, do
 
 // One line's values at the 20 nodes of an interval (centre D from the line
 // centre, half width half), added to f.  The nodes +-u_k share one
-// reciprocal.  g: line_factor (0 for a lane without a line).
+// reciprocal.  g: line_factor, pl: the plinth (0 for a lane without a line),
+// taken off here, before any sum, as from a pair.
 template <class P, int CLASS>
 __device__ __forceinline__ void add_nodes(double D, double half, double ia, double y2, double g,
-                                          const ChiPiece &chi, double (&f)[kFN64]) {
+                                          double pl, const ChiPiece &chi, double (&f)[kFN64]) {
     const double xc = D * ia, h = half * ia;
     double p2 = 0.0, p3 = 0.0, p4 = 0.0;
     if (P::PROFILE == 1 && CLASS == 1) {
@@ -370,8 +371,13 @@ __device__ __forceinline__ void add_nodes(double D, double half, double ia, doub
             vb *= exp_neg(fma(chi.B, eb, chi.t0)) * fma(-u, chi.h, chi.c);
         }
         // (g last: strengths far below 1e-100 must not meet the products)
-        f[k] = fma(g, va, f[k]);
-        f[kFN64 - 1 - k] = fma(g, vb, f[kFN64 - 1 - k]);
+        if constexpr (P::PLINTH) {
+            f[k] += fma(g, va, -pl);
+            f[kFN64 - 1 - k] += fma(g, vb, -pl);
+        } else {
+            f[k] = fma(g, va, f[k]);
+            f[kFN64 - 1 - k] = fma(g, vb, f[kFN64 - 1 - k]);
+        }
     }
 }
 
@@ -379,13 +385,13 @@ __device__ __forceinline__ void add_nodes(double D, double half, double ia, doub
 // the formula of the line nearest its interval (valid farther out too).
 template <class P>
 __device__ __forceinline__ void add_far_lines(int cls, double D, double half, double ia, double y2,
-                                              double G, const ChiPiece &chi,
+                                              double G, double pl, const ChiPiece &chi,
                                               double (&f)[kFN64]) {
     if (!P::WINGS || __ballot(cls != 0) == 0ull) return;
-    if (cls == 0) { D = 1.0; half = 0.0; ia = 1.0e4; y2 = 0.0; G = 0.0; }
-    if (P::PROFILE == 1 && __ballot(cls == 3)) add_nodes<P, 3>(D, half, ia, y2, G, chi, f);
-    else if (P::PROFILE == 1 && __ballot(cls == 2)) add_nodes<P, 2>(D, half, ia, y2, G, chi, f);
-    else add_nodes<P, 1>(D, half, ia, y2, G, chi, f);
+    if (cls == 0) { D = 1.0; half = 0.0; ia = 1.0e4; y2 = 0.0; G = 0.0; pl = 0.0; }
+    if (P::PROFILE == 1 && __ballot(cls == 3)) add_nodes<P, 3>(D, half, ia, y2, G, pl, chi, f);
+    else if (P::PROFILE == 1 && __ballot(cls == 2)) add_nodes<P, 2>(D, half, ia, y2, G, pl, chi, f);
+    else add_nodes<P, 1>(D, half, ia, y2, G, pl, chi, f);
 }
 
 // First index p of [0, n) with !(v[p] < key) (LOWER) or v[p] > key, by one
@@ -617,10 +623,10 @@ __device__ __forceinline__ void add_points(const Args &a, uint32_t code, double 
             if (xj > a.chi.lo && xj < a.chi.hi)
                 v *= exp_neg(fmin(chi_exponent(a.chi, fabs(dd)), 800.0)) * (xj / nu);
         }
+        // (plinths alone: a line that covers the wave is in the constants)
+        if (P::PLINTH && (P::PROFILE != 0 || !full)) v -= pl;
         if (!full) {
-            // (a line that covers the wave has its plinth in the constants)
             const int j = lane + 64 * k;
-            if (P::PLINTH) v -= pl;
             v = (j >= lo && j < hi) ? v : 0.0;
         }
         // one copy of the code above for all segments: acc is a register
@@ -685,7 +691,9 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     __syncthreads();
     const int64_t first = sh->range[0], last = sh->range[1];
     bool any_far = false, any_wave = false;
-    double cst = 0.0, wcst = 0.0;          // plinths of lines that cover the tile, the wave
+    // plinths alone: those of lines that cover the tile, the wave
+    constexpr bool kConst = P::PLINTH && P::PROFILE == 0;
+    double cst = 0.0, wcst = 0.0;
     for (int64_t r0 = first; r0 < last; r0 += kRound64) {
         const int nr = (int)min((int64_t)kRound64, last - r0);
         // tile level: one line per lane; near lines listed per wave
@@ -699,7 +707,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 const int e = s0 + t;
                 bool near = false;
                 int cls = 0;
-                double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0;
+                double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0, pl = 0.0;
                 ChiPiece chi;
                 if (e < nr) {
                     const int64_t i = r0 + e;
@@ -709,13 +717,14 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                     const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
                     D = xc - nu;
                     if constexpr (P::PLINTH) {
-                        if (near && full) cst -= a.pl[i];
+                        if (near) pl = a.pl[i];
                     }
-                    if (P::PROFILE == 0) {
+                    if constexpr (kConst) {
+                        if (near && full) cst -= pl;
                         near = near && !full;
                     } else if (P::COMPACT) {
                         ia = a.ia[i];
-                        if (near && !(P::PLINTH && !full) && fabs(a.S[i]) < 1.0e300)
+                        if (near && !(P::PLINTH && pl != 0.0) && fabs(a.S[i]) < 1.0e300)
                             near = (fabs(D) - hW - a.dnu) * ia <= kDopplerEnd;
                     } else if (a.far && near && full && fabs(D) >= kFarRatio64 * hW) {
                         const double y = a.y[i];
@@ -730,7 +739,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                     }
                 }
                 used |= __ballot(cls != 0) != 0ull;
-                add_far_lines<P>(cls, D, hW, ia, y2, G, chi, f);
+                add_far_lines<P>(cls, D, hW, ia, y2, G, pl, chi, f);
                 const unsigned long long m = __ballot(near);
                 if (near)
                     sh->list[wave][cnt + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)e;
@@ -763,15 +772,15 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
             const double xwl = fma((double)(jw + nw - 1), a.dnu, a.numin);
             for (int c0 = 0; c0 < total; c0 += 64) {
                 int cls = 0;
-                double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0;
+                double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0, pl = 0.0;
                 ChiPiece chi;
-                if ((a.far || P::PLINTH) && c0 + lane < total) {
+                if ((a.far || kConst) && c0 + lane < total) {
                     const int64_t i = line_at(c0 + lane);
                     const double nu = a.nu[i], hw = a.hw[i];
                     const double dl = xwf - nu, dh = xwl - nu;
                     D = xcw - nu;
                     const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
-                    if constexpr (P::PLINTH) {
+                    if constexpr (kConst) {
                         const double el = xfirst - nu, eh = xlast - nu;
                         if (full && !(el > -hw && el < hw && eh > -hw && eh < hw)) wcst -= a.pl[i];
                     }
@@ -780,6 +789,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         ia = a.ia[i];
                         y2 = y * y;
                         G = line_factor<P>(a.S[i], y);
+                        if constexpr (P::PLINTH) pl = a.pl[i];
                         cls = far_class64<P>(D, hw_w, ia, y2, G);
                         if constexpr (P::CHI) {
                             if (cls && !chi_piece(a.chi, xwf, xwl, nu, D, hw_w, chi)) cls = 0;
@@ -788,7 +798,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 }
                 unsigned long long wm = __ballot(cls != 0);
                 if (__popcll(wm) >= wave_min_lines(PPT)) {
-                    add_far_lines<P>(cls, D, hw_w, ia, y2, G, chi, f);
+                    add_far_lines<P>(cls, D, hw_w, ia, y2, G, pl, chi, f);
                     used = true;
                 } else wm = 0ull;
                 if (lane == 0) sh->taken[wave][c0 >> 6] = wm;
@@ -833,7 +843,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         // segments that the window touches; a compact profile's
                         // only where it is not zero, unless a plinth is there
                         int l = lo, h = hi;
-                        const bool part = P::PROFILE == 0 || (P::PLINTH && (lo > 0 || hi < nw));
+                        const bool part = P::PROFILE == 0 || (P::PLINTH && pl != 0.0);
                         if (P::COMPACT && !part && fabs(S) < 1.0e300) {
                             const double off = (nu - xwf) * inv_dnu;
                             const double w = kDopplerEnd / ia * inv_dnu + 2.0;
@@ -874,13 +884,13 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     }
     // node sums -> one series per wave.  any_far differs between waves: the
     // tile's totals are taken whenever any wave has some.
-    if (P::PLINTH) {
+    if (kConst) {
         const double c = wave_total64(cst);
         if (lane == 0) sh->cst[wave] = c;
     }
     const bool tile_far = __syncthreads_or(any_far) != 0;
     if (nw == 0) return;
-    if (P::PLINTH) {
+    if (kConst) {
         double c = wave_total64(wcst);
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) c += sh->cst[w];
