@@ -1224,6 +1224,23 @@ static SortLayout sort_layout(const SortPlan &sp, int64_t nvals, int64_t nseg, i
     return L;
 }
 
+// Workspace that serves every segment length up to longest (0: too long for the
+// sort).  A longer segment may need less -- its plan may have longer runs and so
+// fewer buckets -- but while run length, sample spacing and number of runs stay
+// the same the need grows with the length, so it is looked up where one of them
+// is about to change.
+static size_t sort_layout_max(int64_t longest, int64_t nvals, int64_t nseg, int64_t nfit, int nC,
+                              size_t o) {
+    SortPlan sp;
+    if (plan_sort(longest, sp)) return 0;
+    size_t need = sort_layout(sp, nvals, nseg, nfit, nC, o).total;
+    for (const int64_t step : {(int64_t)kSortCap / 2, (int64_t)kSortCap - kMaxRuns})
+        for (int64_t len = step; len < longest; len += step)
+            if (plan_sort(len, sp) == HK_OK)
+                need = std::max(need, sort_layout(sp, nvals, nseg, nfit, nC, o).total);
+    return need;
+}
+
 // Grid of n workgroups numbered by flat_block().
 static dim3 flat_grid(int64_t n) {
     const int64_t X = (int64_t)1 << 30;
@@ -1400,14 +1417,12 @@ extern "C" size_t hk_ktable_workspace_bytes(int64_t nx, int nbins, int nC, int n
     KtLayout L;
     if (kt_layout(&g, (double)nx, nbins, std::min(nC, kMaxNC), nspec, L)) return 0;
     // room for unaligned segments too (bin keys of other numin/dnu)
-    SortPlan sp;
-    if (plan_sort(nx / nbins + 1, sp)) return 0;
     const int64_t nseg = (int64_t)nspec * (nbins + 1);
     const size_t base = align_up(L.off_segs + sizeof(Seg) * (size_t)nseg, 256) +
                         align_up(sizeof(double) * (size_t)nspec * nx, 256);
-    const SortLayout sl = sort_layout(sp, (int64_t)nspec * nx, nseg, (int64_t)nspec * nbins, nC,
-                                      base);
-    return std::max(L.total, sl.total + 256);
+    const size_t sl = sort_layout_max(nx / nbins + 1, (int64_t)nspec * nx, nseg,
+                                      (int64_t)nspec * nbins, nC, base);
+    return sl ? std::max(L.total, sl + 256) : 0;
 }
 
 extern "C" int hk_ktable_prepare(const hk_grid *g, double numax, int nbins, int nC, void *ws,
@@ -1585,9 +1600,9 @@ static int sort_bins_plan(int64_t nx, const int64_t *seg, int nseg, SortPlan &sp
 extern "C" size_t hk_sort_bins_workspace_bytes(int64_t nx, int nseg) {
     if (nx <= 0 || nseg <= 0) return 0;
     // the longest possible segment is the whole spectrum
-    SortPlan sp;
-    if (plan_sort(nx, sp)) return 0;
-    return sort_layout(sp, nx, nseg, 0, 1, align_up(sizeof(Seg) * (size_t)nseg, 256)).total + 256;
+    const size_t need =
+        sort_layout_max(nx, nx, nseg, 0, 1, align_up(sizeof(Seg) * (size_t)nseg, 256));
+    return need ? need + 256 : 0;
 }
 
 extern "C" int hk_sort_bins(const double *K, int64_t nx, const int64_t *seg, int nseg,
