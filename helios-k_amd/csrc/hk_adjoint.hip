@@ -32,6 +32,8 @@
 // for the registers, as the compiler chooses, 2.23).
 #include <math.h>
 
+#include <algorithm>
+
 #include "hk_device.h"
 #include "hk_internal.h"
 #include "hk_voigt64.h"
@@ -543,25 +545,36 @@ int adjoint_lines(int64_t nlines) { return nlines < 65536 ? 64 : kAT; }
 // over several workgroups, at most 32: up to ~20 workgroups per CU, since a
 // workgroup's barriers leave its CU to the others.  3.3e5 lines, 11 tiles a
 // window: 1 part 2.60 ms, 2 parts 2.28, 4 parts 2.15, 8 parts 2.32.
+constexpr int kAPartBlocks = 5300, kAPartsMax = 32;
 int adjoint_parts(int64_t nlines) {
     const int64_t nblocks = (nlines + adjoint_lines(nlines) - 1) / adjoint_lines(nlines);
-    const int64_t p = nblocks > 0 ? 5300 / nblocks : 1;
-    return (int)(p < 1 ? 1 : (p > 32 ? 32 : p));
+    const int64_t p = nblocks > 0 ? kAPartBlocks / nblocks : 1;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kAPartsMax, p));
 }
 
 // Workgroups whose partial dL/dT, dL/dP the last kernel adds: of the main kernel
 // or, with parts, of the combination.
-int64_t adjoint_sums(int64_t nlines) {
-    const int per = adjoint_parts(nlines) > 1 ? kAT : adjoint_lines(nlines);
+int64_t adjoint_sums(int64_t nlines, int parts) {
+    const int per = parts > 1 ? kAT : adjoint_lines(nlines);
     return (nlines + per - 1) / per;
 }
+
+// Workspace [doubles] of a list summed in this many parts; parts == 1 needs no
+// more than the two numbers a line that any caller has room for.
+int64_t adjoint_doubles(int64_t nlines, int parts) {
+    return 2 * adjoint_sums(nlines, parts) + (parts > 1 ? 4 * parts * nlines : 0) + 2;
+}
+
+size_t adjoint_bytes(int64_t doubles) { return (size_t)doubles * sizeof(double) + 256; }
 
 }  // namespace
 
 extern "C" size_t hk_voigt_adjoint_workspace_bytes(int64_t nlines) {
     if (nlines < 0) return 0;
-    const int parts = adjoint_parts(nlines);
-    return (size_t)(2 * adjoint_sums(nlines) + (parts > 1 ? 4 * parts * nlines : 0) + 2) * sizeof(double) + 256;
+    // enough for this list and for every shorter one in all its parts: parts *
+    // lines is at most 32 lines and what adjoint_parts leaves of 5300 workgroups
+    const int64_t most = (int64_t)kAPartBlocks * adjoint_lines(nlines);
+    return adjoint_bytes(2 * ((nlines + 63) / 64) + 4 * std::min(kAPartsMax * nlines, most) + 2);
 }
 
 extern "C" int hk_voigt_adjoint(const hk_lines *L, const hk_tp *tp, const hk_cut *cut,
@@ -573,9 +586,12 @@ extern "C" int hk_voigt_adjoint(const hk_lines *L, const hk_tp *tp, const hk_cut
     HK_CHECK_ARG(L->form >= HK_FORM_HITRAN && L->form <= HK_FORM_SUPERLINE,
                  "hk_voigt_adjoint: form %d", L->form);
     HK_CHECK_ARG(g->nx > 0 && g->dnu > 0.0, "hk_voigt_adjoint: bad grid");
-    if (ws_bytes < hk_voigt_adjoint_workspace_bytes(L->nlines)) {
+    // in as many parts as the workspace has room for
+    int parts = adjoint_parts(L->nlines);
+    while (parts > 1 && ws_bytes < adjoint_bytes(adjoint_doubles(L->nlines, parts))) --parts;
+    if (ws_bytes < adjoint_bytes(adjoint_doubles(L->nlines, parts))) {
         hk::set_error("hk_voigt_adjoint: workspace %zu bytes, %zu needed", ws_bytes,
-                      hk_voigt_adjoint_workspace_bytes(L->nlines));
+                      adjoint_bytes(adjoint_doubles(L->nlines, parts)));
         return HK_ERR_WORKSPACE;
     }
     AArgs a;
@@ -590,8 +606,8 @@ extern "C" int hk_voigt_adjoint(const hk_lines *L, const hk_tp *tp, const hk_cut
     a.nexp = L->n; a.iso = L->iso; a.form = L->form; a.nl = L->nlines; a.T = tp->T; a.P = tp->P;
     a.cut_mode = cut->cut_mode; a.cut = cut->cut == 0.0 ? 1.0e30 : cut->cut;
     a.numin = g->numin; a.dnu = g->dnu; a.nx = g->nx; a.gK = gK; a.gS = gS; a.gvy = gvy;
-    a.parts = adjoint_parts(L->nlines);
-    a.nblocks = adjoint_sums(L->nlines);
+    a.parts = parts;
+    a.nblocks = adjoint_sums(L->nlines, parts);
     a.part_tp = (double *)hk::align_up((size_t)ws, 256);
     a.sums = a.part_tp + 2 * a.nblocks;
     hipStream_t s = (hipStream_t)stream;

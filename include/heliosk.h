@@ -401,7 +401,10 @@ int hk_transmission(const double *Ksorted, int nbins, int Nxb, const int32_t *nx
 /* Adjoint of the Voigt sum: given gK_j = dL/dK_j on the grid, writes
  * gS[i] = dL/dS_i (S = the raw S_file), gvy[i] = dL/dvy_i and
  * gTP[0..1] = dL/dT, dL/dP, holding the partition function fixed.  The
- * profile is recomputed (FP64), not stored.  gTP is device memory. */
+ * profile is recomputed (FP64), not stored.  gTP is device memory.  The
+ * workspace of one list serves every shorter one; with less than the query
+ * (16 bytes a line + 272 are always enough) the sums are taken in fewer parts,
+ * which is slower and rounds in another order. */
 size_t hk_voigt_adjoint_workspace_bytes(int64_t nlines);
 int hk_voigt_adjoint(const hk_lines *lines, const hk_tp *tp, const hk_cut *cut,
                      const hk_grid *grid, const double *gK, double *gS,

@@ -35,8 +35,8 @@ EDGES = [16384, 16385, 32736, 65536, 98304, 114688, 131072, 131073, 147312, 2621
 @pytest.mark.parametrize("nseg", [1, 100, 300, 3001])
 @pytest.mark.parametrize("extra", [0, 1, 965, 3928, 20000, 300000])
 def test_query_covers_every_plan(nseg, extra):
-    from heliosk import _lib
-    L = _lib.lib()
+    from heliosk import engine as E
+    L = E.lib()
     for edge in EDGES:
         for longest in (edge - 1, edge, edge + 1):
             nx = longest + (extra if nseg > 1 else 0)
@@ -46,8 +46,8 @@ def test_query_covers_every_plan(nseg, extra):
 
 
 def test_lists_that_were_refused():
-    from heliosk import _lib
-    L = _lib.lib()
+    from heliosk import engine as E
+    L = E.lib()
     for nx, nseg, longest in ((132037, 100, 131072), (135000, 300, 131072), (524855, 300, 523855)):
         need = _needed(L, nx, _segments(nx, nseg, longest, 0))
         assert need <= L.hk_sort_bins_workspace_bytes(nx, nseg), (nx, nseg, longest)
@@ -55,8 +55,8 @@ def test_lists_that_were_refused():
 
 def test_query_stays_close_to_the_longest_plan():
     """The maximum is no more than a few tables above one plan's size."""
-    from heliosk import _lib
-    L = _lib.lib()
+    from heliosk import engine as E
+    L = E.lib()
     for nx in (1000, 16385, 131073, 3000000, 30000000):
         one = _needed(L, nx, [0, nx])
         assert one <= L.hk_sort_bins_workspace_bytes(nx, 1) <= one + 8 * nx + 65536
