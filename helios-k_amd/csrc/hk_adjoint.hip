@@ -24,7 +24,9 @@
 // reach: it forms the G_k of the tile, and of its four quarters and 16 segments where
 // some line is near, and each lane evaluates its line at the nodes of the
 // largest far interval; what is left (~4 segments a line) is summed point by
-// point, 64 points at a time.
+// point, 64 points at a time.  Tiles between two windows are passed over, and the
+// windows of a short list that are few and short against their tiles are summed
+// point by point throughout.
 //
 // What bounds it: FP64 vector instructions, about half of them the line cores.
 // One wave per line over all points of its window took 13.3 ms for 3.3e5 lines
@@ -48,6 +50,13 @@ constexpr double kFarRatioAdj = 3.5;
 constexpr int kAT = 256;                  // lines per workgroup
 constexpr int kATile = 1024, kASub = 256, kASeg = 64;
 constexpr int kASubs = kATile / kASub, kASegs = kATile / kASeg;
+
+// Short lists: a line is summed by itself, 64 points of its window a step, where
+// that takes at most this many steps per tile that a workgroup would walk.  With
+// 0, 20, 40 and 80 (1e6 points): 500 lines of 1000 points 137, 31, 31, 31 us,
+// 3000 of 5000 points 178, 175, 82, 82, 10000 of 5000 269, 271, 272, 210, 50000 of
+// 5000 625, 628, 625, 750; on 1e5 points 10000 of 5000 166, 167, 167, 205.
+constexpr int kDirectSteps = 40;
 
 struct IsoTabA {
     double mass[HK_MAX_ISO], ab[HK_MAX_ISO], ss[HK_MAX_ISO], Q[HK_MAX_ISO];
@@ -220,6 +229,59 @@ __device__ __forceinline__ WD wd_core(double x, double y, double pf, const doubl
     return wd_identity(x, y, re, x < 0.0 ? -im : im);
 }
 
+// 1/(s^2 + y^2) and that times s = (n0 - m + 1/2) h, for wd_core.
+__device__ __forceinline__ void wd_table(double *tab, double y2) {
+    const int lane = threadIdx.x & 63;
+    const double s = ((double)(lane - kCHi) + 0.5) * kHC;
+    wave_lds_sync();
+    if (lane < kCTab) {
+        const double dd = rcp64(fma(s, s, y2));
+        tab[lane] = dd;
+        tab[64 + lane] = s * dd;
+    }
+    wave_lds_sync();
+}
+
+// One line at one point per lane (on: it lies in the window), added to the
+// lane's sums.  have_tab: whether tab holds this line's table yet.
+__device__ __forceinline__ void add_point(bool on, double x, double y, double pf, double g,
+                                          double *tab, bool &have_tab, double (&s)[4]) {
+    const double y2 = y * y, r2 = fma(x, x, y2);
+    WD v = {0.0, 0.0, 0.0};
+    if (__ballot(on && r2 < kRB64)) {
+        if (!have_tab) wd_table(tab, y2);
+        have_tab = true;
+        v = wd_core(x, y, pf, tab);
+    }
+    if (on && r2 >= kRB64) v = r2 >= kRM64 ? wd_far(x, y, r2) : wd_mid(x, y, r2);
+    if (on && !(r2 >= kRB64) && !(r2 < kRB64)) v.re = v.dx = v.dy = r2;   // undefined
+    if (on) {
+        s[0] = fma(g, v.re, s[0]);
+        s[1] = fma(g, v.dy, s[1]);
+        s[2] = fma(g, v.dx, s[2]);
+        s[3] = fma(g * x, v.dx, s[3]);
+    }
+}
+
+// The wave's totals of s, added to lane b's sums.
+__device__ __forceinline__ void add_line_totals(const double (&s)[4], int b, double (&A)[4]) {
+    // rows of 16 lanes end up with s0, s2, s1, s3
+    double z = swap_add16(swap_add32(s[0], s[1]), swap_add32(s[2], s[3]));
+    z += row_dpp64<0xb1>(z);
+    z += row_dpp64<0x4e>(z);
+    z += row_dpp64<0x141>(z);
+    z += row_dpp64<0x140>(z);
+    const double z0 = lane_f64(z, 0), z2 = lane_f64(z, 16), z1 = lane_f64(z, 32),
+                 z3 = lane_f64(z, 48);
+    if ((threadIdx.x & 63) == b) { A[0] += z0; A[1] += z1; A[2] += z2; A[3] += z3; }
+}
+
+__device__ __forceinline__ int64_t lane_i64(int64_t v, int b) {
+    const unsigned lo = __builtin_amdgcn_readlane((int)v, b);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(v >> 32), b);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 struct AdjLDS {
     double g[kATile];
     double M0[kWaves][kFN64];                 // tile moments, one row per wave
@@ -297,6 +359,32 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
     const double nu = r.nu, ia = r.ia, y = r.y;
     const double pf = core_pole(y);
     double A[4] = {0.0, 0.0, 0.0, 0.0};          // sums of g times re, dy, dx, x dx
+    if constexpr (kShared) {
+        // windows short against the tiles they spread over: a line at a time per
+        // wave, all its points, as many lines at once as the parts have waves
+        int64_t most = jhi - jlo;
+        for (int off = 32; off > 0; off >>= 1)
+            most = max(most, (int64_t)__shfl_xor((long long)most, off, 64));
+        const int64_t rounds = (LPB + kWaves * a.parts - 1) / (kWaves * a.parts);
+        const int64_t tiles = ((hi - lo) / kATile + a.parts) / a.parts;
+        if (lo < hi && rounds * (most / 64 + 1) <= kDirectSteps * tiles) {
+            for (int b = part * kWaves + wave; b < LPB; b += kWaves * a.parts) {
+                const int64_t l = lane_i64(jlo, b), h = lane_i64(jhi, b);
+                const double lnu = lane_f64(nu, b), lia = lane_f64(ia, b), ly = lane_f64(y, b);
+                const double lpf = lane_f64(pf, b);
+                bool have_tab = false;
+                double sums[4] = {0.0, 0.0, 0.0, 0.0};
+                for (int64_t j0 = l; j0 < h; j0 += 64) {
+                    const int64_t j = j0 + lane;
+                    const bool on = j < h;
+                    add_point(on, (fma((double)j, a.dnu, a.numin) - lnu) * lia, ly, lpf,
+                              on ? a.gK[j] : 0.0, sh.tab[wave], have_tab, sums);
+                }
+                add_line_totals(sums, b, A);
+            }
+            hi = lo;                             // no tiles left
+        }
+    }
     for (int64_t tile = lo / kATile + part; lo < hi && tile <= (hi - 1) / kATile;
          tile += a.parts) {
         const int64_t j0 = tile * kATile;
@@ -305,7 +393,11 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
         auto valid = [&](int first, int len) { return max(0, min(len, Wv - first)); };
         auto half = [&](int n) { return fmax(0.5 * (double)(n - 1), 0.5) * a.dnu; };
         auto centre = [&](int first, int n) { return xat((double)first + 0.5 * (double)max(n - 1, 0)); };
-        __syncthreads();                         // the previous tile's readers are done
+        const int wl = (int)min(max(jlo - j0, (int64_t)0), (int64_t)Wv);
+        const int wh = (int)min(max(jhi - j0, (int64_t)0), (int64_t)Wv);
+        const bool in = wl < wh;
+        // (also the barrier behind the previous tile's readers)
+        if (!__syncthreads_or(in)) continue;     // between two windows
         bool ok = true;
 #pragma unroll
         for (int q = 0; q < kATile / kAT; ++q) {
@@ -318,9 +410,6 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
         // (a tile with an infinite or undefined gradient is taken point by
         // point: each line meets it at the points of its own window)
         const bool fin = __syncthreads_and(ok) != 0;
-        const int wl = (int)min(max(jlo - j0, (int64_t)0), (int64_t)Wv);
-        const int wh = (int)min(max(jhi - j0, (int64_t)0), (int64_t)Wv);
-        const bool in = wl < wh;
         int cls0 = 0;
         if (in && fin && wl == 0 && wh == Wv) cls0 = far_class_adj(centre(0, Wv) - nu, half(Wv), ia, y);
         const bool near = in && cls0 == 0;
@@ -411,49 +500,16 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
             unsigned segs = __builtin_amdgcn_readlane((int)todo, b);
             const int l = __builtin_amdgcn_readlane(wl, b), h = __builtin_amdgcn_readlane(wh, b);
             const double lnu = lane_f64(nu, b), lia = lane_f64(ia, b), ly = lane_f64(y, b);
-            const double lpf = lane_f64(pf, b), ly2 = ly * ly;
+            const double lpf = lane_f64(pf, b);
             bool have_tab = false;
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+            double sums[4] = {0.0, 0.0, 0.0, 0.0};
             while (segs) {
                 const int j = (__builtin_ctz(segs)) * kASeg + lane;
                 segs &= segs - 1u;
-                const bool on = j >= l && j < h;
-                const double x = (xat((double)j) - lnu) * lia, r2 = fma(x, x, ly2);
-                WD v = {0.0, 0.0, 0.0};
-                if (__ballot(on && r2 < kRB64)) {
-                    if (!have_tab) {
-                        // 1/(s^2 + y^2) and that times s = (n0 - m + 1/2) h
-                        const double s = ((double)(lane - kCHi) + 0.5) * kHC;
-                        wave_lds_sync();
-                        if (lane < kCTab) {
-                            const double dd = rcp64(fma(s, s, ly2));
-                            tab[lane] = dd;
-                            tab[64 + lane] = s * dd;
-                        }
-                        wave_lds_sync();
-                        have_tab = true;
-                    }
-                    v = wd_core(x, ly, lpf, tab);
-                }
-                if (on && r2 >= kRB64) v = r2 >= kRM64 ? wd_far(x, ly, r2) : wd_mid(x, ly, r2);
-                if (on && !(r2 >= kRB64) && !(r2 < kRB64)) v.re = v.dx = v.dy = r2;   // undefined
-                if (on) {
-                    const double g = sh.g[j];
-                    s0 = fma(g, v.re, s0);
-                    s1 = fma(g, v.dy, s1);
-                    s2 = fma(g, v.dx, s2);
-                    s3 = fma(g * x, v.dx, s3);
-                }
+                add_point(j >= l && j < h, (xat((double)j) - lnu) * lia, ly, lpf, sh.g[j], tab,
+                          have_tab, sums);
             }
-            // wave totals: rows of 16 lanes end up with s0, s2, s1, s3
-            double z = swap_add16(swap_add32(s0, s1), swap_add32(s2, s3));
-            z += row_dpp64<0xb1>(z);
-            z += row_dpp64<0x4e>(z);
-            z += row_dpp64<0x141>(z);
-            z += row_dpp64<0x140>(z);
-            const double z0 = lane_f64(z, 0), z2 = lane_f64(z, 16), z1 = lane_f64(z, 32),
-                         z3 = lane_f64(z, 48);
-            if (lane == b) { A[0] += z0; A[1] += z1; A[2] += z2; A[3] += z3; }
+            add_line_totals(sums, b, A);
         }
     }
     bool own = i < a.nl;
