@@ -29,6 +29,7 @@ constexpr int kRun = kNT * kIPT;          // pairs per LDS-sorted run (8192)
 constexpr int kMergeE = 8;                // outputs per thread in a merge pass
 constexpr int kMB = 256 * kMergeE;        // outputs per merge workgroup (2048)
 constexpr int64_t kMaxSortLines = 0x7fffffff;
+constexpr int64_t kWideSplitLines = (int64_t)1 << 20;
 
 // (key, index) order: by key, then by index.
 __device__ __forceinline__ bool pless(double ka, int32_t ia, double kb, int32_t ib) {
@@ -165,12 +166,22 @@ __global__ __launch_bounds__(kNT) void pair_block_sort_kernel(const double *__re
 }
 
 // First a in [max(0, diag-nb), min(diag, na)] with A[a] after B[diag-a-1], by
-// a wave: 64 probes a round, so a range of 2.5e5 takes three rounds of loads
-// (one thread halving it: 18; a merge pass over it 17 us, this 13 us).
+// a wave (WIDE: 64 probes a round, so a range of 2.5e5 takes three rounds of
+// loads; halving it 18, a merge pass over it 17 us against 13) or by one lane:
+// long lists are bound by memory, and 64 probes a round move as much as the merge
+// itself (2.2e7 lines: 354 us a pass, halving 338).
+template <bool WIDE>
 __device__ __forceinline__ int64_t pair_split(const double *Ak, const int32_t *Ai, int64_t na,
                                               const double *Bk, const int32_t *Bi, int64_t nb,
                                               int64_t diag) {
     int64_t lo = std::max<int64_t>(0, diag - nb), hi = std::min<int64_t>(diag, na);
+    if (!WIDE) {
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1, bm = diag - mid - 1;
+            if (!pless(Bk[bm], Bi[bm], Ak[mid], Ai[mid])) lo = mid + 1; else hi = mid;
+        }
+        return lo;
+    }
     while (lo < hi) {
         const int64_t step = (hi - lo + 63) >> 6;
         const int64_t mid = lo + (threadIdx.x & 63) * step;
@@ -184,6 +195,7 @@ __device__ __forceinline__ int64_t pair_split(const double *Ak, const int32_t *A
     return lo;
 }
 
+template <bool WIDE>
 __global__ __launch_bounds__(256) void pair_merge_kernel(const double *__restrict__ ik,
                                                          const int32_t *__restrict__ ii,
                                                          double *__restrict__ ok,
@@ -200,9 +212,14 @@ __global__ __launch_bounds__(256) void pair_merge_kernel(const double *__restric
     const double *Ak = ik + ps, *Bk = Ak + na;
     const int32_t *Ai = ii + ps, *Bi = Ai + na;
     const int64_t d0 = o0 - ps, d1 = std::min(d0 + kMB, na + nb);
-    if (t < 128) {
-        const int64_t a = pair_split(Ak, Ai, na, Bk, Bi, nb, t < 64 ? d0 : d1);
-        if ((t & 63) == 0) sp[t >> 6] = a;
+    if (WIDE) {
+        if (t < 128) {
+            const int64_t a = pair_split<WIDE>(Ak, Ai, na, Bk, Bi, nb, t < 64 ? d0 : d1);
+            if ((t & 63) == 0) sp[t >> 6] = a;
+        }
+    } else {                                    // (scalar loads: the diagonals are uniform)
+        if (t == 0) sp[0] = pair_split<WIDE>(Ak, Ai, na, Bk, Bi, nb, d0);
+        if (t == 64) sp[1] = pair_split<WIDE>(Ak, Ai, na, Bk, Bi, nb, d1);
     }
     __syncthreads();
     const int64_t a0 = sp[0], a1 = sp[1], b0 = d0 - a0, b1 = d1 - a1;
@@ -576,7 +593,12 @@ int sort_pairs(const double *key, int64_t n, double *k0, int32_t *i0, double *k1
     which = 0;
     const unsigned nblk = (unsigned)((n + kMB - 1) / kMB);
     for (int64_t wl = kRun; wl < n; wl *= 2) {
-        hipLaunchKernelGGL(pair_merge_kernel, dim3(nblk), dim3(256), 0, s, ck, ci, nk, ni, n, wl);
+        if (n <= kWideSplitLines)
+            hipLaunchKernelGGL(pair_merge_kernel<true>, dim3(nblk), dim3(256), 0, s, ck, ci, nk, ni, n,
+                               wl);
+        else
+            hipLaunchKernelGGL(pair_merge_kernel<false>, dim3(nblk), dim3(256), 0, s, ck, ci, nk, ni,
+                               n, wl);
         HK_LAUNCH_CHECK();
         std::swap(ck, nk);
         std::swap(ci, ni);
