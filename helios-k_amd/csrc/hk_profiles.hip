@@ -71,7 +71,7 @@ struct PArgs {
     double numin, dnu;
     int64_t nx;
     double kmin;
-    int accumulate, far;
+    int accumulate;
     double *K;
     Chi chi;
     // sub-Lorentzian range and the points a pass writes: 0 all, 1 those inside
@@ -182,7 +182,7 @@ extern "C" int hk_profile_accumulate(const hk_line_state *st, const hk_grid *gri
     a.nu = st->nu; a.S = st->S; a.ia = st->ialphaD; a.y = st->y; a.hw = st->hw; a.pl = pl;
     a.key = st->key; a.radius = st->radius;
     a.nl = n; a.numin = grid->numin; a.dnu = grid->dnu; a.nx = grid->nx;
-    a.kmin = kmin; a.accumulate = accumulate || voigt_sum; a.far = 1; a.K = K;
+    a.kmin = kmin; a.accumulate = accumulate || voigt_sum; a.K = K;
     a.chi = Chi{0, 0, 0, 0, 0, 0, 0, 0};
     a.lo = a.hi = 0.0;
     a.side = 0;

@@ -1395,12 +1395,21 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
 // line-core pass.
 constexpr int main_waves(int mode, int ppt, int lm);
 
+// Kernels' MODE beside the public forms: FP64 with every pair evaluated.
+constexpr int kFP64Pairs = 3;
+
+// The FP64 forms' line sum.  Whole-wave lines are
+// worth their registers there, where nearly all lines are, and on tiles that a
+// caller makes so wide that few lines are far.
+template <int MODE, int PPT>
+using Sum64 = LineSum<1, false, false, MODE == kFP64Pairs || (PPT >= 4), MODE == kFP64Pairs>;
+
 template <int MODE, int PPT, int LM>
 __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_kernel(VArgs a) {
     const int64_t tile = blockIdx.x;
-    if (MODE == HK_VOIGT_FP64) {
+    if constexpr (MODE != HK_VOIGT_FP32C) {
         __shared__ Far64LDS sh;
-        tile_f64<PPT, LineSum<1, false, false, (PPT >= 4)>>(a, tile, &sh);
+        tile_f64<PPT, Sum64<MODE, PPT>>(a, tile, &sh);
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
@@ -1443,7 +1452,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
                                                                int nspec, unsigned long long *counter,
                                                                int chunk) {
     constexpr size_t kBytes =
-        MODE == HK_VOIGT_FP64 ? sizeof(Far64LDS)
+        MODE != HK_VOIGT_FP32C ? sizeof(Far64LDS)
                               : (PPT == 0 ? sizeof(Core32) : sizeof(Rec32)) * kThreads * LM;
     __shared__ int64_t s_item;
     __shared__ int cnt[kThreads / 64];
@@ -1472,7 +1481,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
         if constexpr (PPT == 0) {
             core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
-            if constexpr (MODE == HK_VOIGT_FP64) tile_f64<PPT, LineSum<1, false, false, (PPT >= 4)>>(a, tile, (Far64LDS *)smem);
+            if constexpr (MODE != HK_VOIGT_FP32C) tile_f64<PPT, Sum64<MODE, PPT>>(a, tile, (Far64LDS *)smem);
             else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
         }
     }
@@ -1648,20 +1657,24 @@ using namespace hk;
 
 namespace {
 
-// Points per thread of the main pass's tiles: the caller's choice, or
+// tile_points a caller may ask for: 512, 1024, 2048 or 4096 (256-point tiles
+// are FP64's own choice for short grids).
+bool tile_points_ok(const hk_tune *tune) {
+    if (!(tune && tune->tile_points > 0)) return true;
+    const int ppt = tune->tile_points / kThreads;
+    return ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16;
+}
+
+// Points per thread of the main pass's tiles: the caller's choice (FP64:
+// asked_ppt64), or
 //  FP32C  1024-point tiles (smaller ones trade direct pairs for node
 //         evaluations; 1024 was fastest at 1e7 lines x 3e7 points);
 //  FP64   default_ppt64.
 int pick_ppt(int mode, const hk_tune *tune, int64_t nx) {
-    if (tune && tune->tile_points > 0) return tune->tile_points / kThreads;
-    return mode == HK_VOIGT_FP64 ? default_ppt64(nx, tune && tune->exact_pairs) : 4;
-}
-
-// tile_points a caller may ask for: 512, 1024, 2048 or 4096 (256-point tiles
-// are FP64's own choice for short grids).
-bool tile_points_ok(int mode, const hk_tune *tune, int ppt) {
-    if (!(tune && tune->tile_points > 0)) return true;
-    return (ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16);
+    const bool exact = tune && tune->exact_pairs;
+    const int asked = tune && tune->tile_points > 0 ? tune->tile_points / kThreads : 0;
+    if (mode != HK_VOIGT_FP64) return asked ? asked : 4;
+    return asked ? asked_ppt64(asked, nx, exact) : default_ppt64(nx, exact);
 }
 
 // Lines per LDS stage of the main pass: 256 (default) or 512; returns the
@@ -1671,53 +1684,69 @@ int pick_lm(const hk_tune *tune) {
     return sl == kThreads ? 1 : (sl == 2 * kThreads ? 2 : 0);
 }
 
+// MODE of the kernels for a public form and its exact_pairs (FP32C's kernels see
+// that in their arguments).
+int kernel_mode(int mode, bool exact) {
+    return mode == HK_VOIGT_FP64 && exact ? kFP64Pairs : mode;
+}
+
+// (tiles of 256 points are FP64's only, those of 4096 FP32C's, and FP64 has no
+// stages)
 template <int MODE, int LM>
 void launch_tiles_lm(int ppt, int64_t ntiles, hipStream_t s, const VArgs &a) {
     dim3 g((unsigned)ntiles), b(kThreads);
     switch (ppt) {
-        case 1: hipLaunchKernelGGL((voigt_tiles_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((voigt_tiles_kernel<MODE == HK_VOIGT_FP32C ? HK_VOIGT_FP64 : MODE, 1, 1>), g, b, 0, s, a); break;
         case 2: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 2, LM>), g, b, 0, s, a); break;
         case 4: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 4, LM>), g, b, 0, s, a); break;
         case 8: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 8, LM>), g, b, 0, s, a); break;
-        default: hipLaunchKernelGGL((voigt_tiles_kernel<MODE, 16, LM>), g, b, 0, s, a); break;
+        default: hipLaunchKernelGGL((voigt_tiles_kernel<HK_VOIGT_FP32C, 16, LM>), g, b, 0, s, a); break;
     }
 }
 
-template <int MODE>
-void launch_tiles(int ppt, int lm, int64_t ntiles, hipStream_t s, const VArgs &a) {
-    if (MODE == HK_VOIGT_FP32C && lm == 2) launch_tiles_lm<HK_VOIGT_FP32C, 2>(ppt, ntiles, s, a);
-    else launch_tiles_lm<MODE, 1>(ppt, ntiles, s, a);
+void launch_tiles(int kmode, int ppt, int lm, int64_t ntiles, hipStream_t s, const VArgs &a) {
+    if (kmode == kFP64Pairs) launch_tiles_lm<kFP64Pairs, 1>(ppt, ntiles, s, a);
+    else if (kmode == HK_VOIGT_FP64) launch_tiles_lm<HK_VOIGT_FP64, 1>(ppt, ntiles, s, a);
+    else if (lm == 2) launch_tiles_lm<HK_VOIGT_FP32C, 2>(ppt, ntiles, s, a);
+    else launch_tiles_lm<HK_VOIGT_FP32C, 1>(ppt, ntiles, s, a);
+}
+
+struct Queue {
+    unsigned grid;
+    const VArgs *specs;
+    const int64_t *item_start;
+    int nspec;
+    unsigned long long *counter;
+    int chunk;
+};
+
+template <int MODE, int PPT, int LM>
+void launch_queue(hipStream_t s, const Queue &q) {
+    hipLaunchKernelGGL((voigt_persistent_kernel<MODE, PPT, LM>), dim3(q.grid), dim3(kThreads), 0, s,
+                       q.specs, q.item_start, q.nspec, q.counter, q.chunk);
 }
 
 template <int MODE, int LM>
-void launch_persistent_lm(int ppt, unsigned grid, hipStream_t s, const VArgs *specs,
-                          const int64_t *item_start, int nspec, unsigned long long *counter,
-                          int chunk) {
-    dim3 g(grid), b(kThreads);
+void launch_persistent_lm(int ppt, hipStream_t s, const Queue &q) {
     switch (ppt) {
-        case 1: hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP64, 1, 1>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
-        case 2: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 2, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
-        case 4: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 4, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
-        case 8: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 8, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
-        default: hipLaunchKernelGGL((voigt_persistent_kernel<MODE, 16, LM>), g, b, 0, s, specs, item_start, nspec, counter, chunk); break;
+        case 1: launch_queue<MODE == HK_VOIGT_FP32C ? HK_VOIGT_FP64 : MODE, 1, 1>(s, q); break;
+        case 2: launch_queue<MODE, 2, LM>(s, q); break;
+        case 4: launch_queue<MODE, 4, LM>(s, q); break;
+        case 8: launch_queue<MODE, 8, LM>(s, q); break;
+        default: launch_queue<HK_VOIGT_FP32C, 16, LM>(s, q); break;
     }
 }
 
-// ppt == 0: the line-core pass (its stages are kThreads lines)
-template <int MODE>
-void launch_persistent(int ppt, int lm, unsigned grid, hipStream_t s, const VArgs *specs,
-                       const int64_t *item_start, int nspec, unsigned long long *counter,
-                       int64_t nitems) {
+// ppt == 0: FP32C's line-core pass (its stages are kThreads lines)
+void launch_persistent(int kmode, int ppt, int lm, hipStream_t s, Queue q, int64_t nitems) {
     // at least 32 chunks a workgroup, so that the last ones end together (4:
     // the line-core pass above 9.8 ms, 16: 7.1, 32: 6.8, 64: 7.2)
-    const int chunk = (int)std::max<int64_t>(1, std::min<int64_t>(64, nitems / (32 * (int64_t)grid)));
-    if (MODE == HK_VOIGT_FP32C && ppt == 0)
-        hipLaunchKernelGGL((voigt_persistent_kernel<HK_VOIGT_FP32C, 0, 1>), dim3(grid), dim3(kThreads), 0, s,
-                           specs, item_start, nspec, counter, chunk);
-    else if (MODE == HK_VOIGT_FP32C && lm == 2)
-        launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, grid, s, specs, item_start, nspec, counter, chunk);
-    else
-        launch_persistent_lm<MODE, 1>(ppt, grid, s, specs, item_start, nspec, counter, chunk);
+    q.chunk = (int)std::max<int64_t>(1, std::min<int64_t>(64, nitems / (32 * (int64_t)q.grid)));
+    if (kmode == kFP64Pairs) launch_persistent_lm<kFP64Pairs, 1>(ppt, s, q);
+    else if (kmode == HK_VOIGT_FP64) launch_persistent_lm<HK_VOIGT_FP64, 1>(ppt, s, q);
+    else if (ppt == 0) launch_queue<HK_VOIGT_FP32C, 0, 1>(s, q);
+    else if (lm == 2) launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, s, q);
+    else launch_persistent_lm<HK_VOIGT_FP32C, 1>(ppt, s, q);
 }
 
 int check_state(const hk_line_state *st, const char *fn) {
@@ -1754,7 +1783,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     if (int e = check_state(st, "hk_voigt_accumulate")) return e;
     if (int e = check_grid(grid, "hk_voigt_accumulate")) return e;
     const int ppt = pick_ppt(mode, tune, grid->nx);
-    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_accumulate: tile_points must be 512, 1024, 2048 or 4096");
+    HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_accumulate: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_accumulate: stage_lines must be 256 or 512");
     if (ws_bytes < hk_voigt_workspace_bytes(grid, tune)) {
@@ -1777,7 +1806,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     a.kmin = kmin; a.accumulate = accumulate; a.K = K;
     a.far = tune && tune->exact_pairs ? 0 : 1;
     if (mode == HK_VOIGT_FP64) {            // one pass; its tiles search their own line ranges
-        launch_tiles<HK_VOIGT_FP64>(ppt, lm, ntiles, s, a);
+        launch_tiles(kernel_mode(mode, a.far == 0), ppt, lm, ntiles, s, a);
         HK_LAUNCH_CHECK();
         return HK_OK;
     }
@@ -1789,7 +1818,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
                        st->key, st->nlines, st->radius + 1, st->blk_max, grid->numin, grid->dnu,
                        grid->nx, kCoreW, ncore, 1, ctiles);
     HK_LAUNCH_CHECK();
-    launch_tiles<HK_VOIGT_FP32C>(ppt, lm, ntiles, s, a);
+    launch_tiles(mode, ppt, lm, ntiles, s, a);
     HK_LAUNCH_CHECK();
     a.tiles = ctiles;
     hipLaunchKernelGGL(voigt_core_kernel, dim3((unsigned)ncore), dim3(kThreads), 0, s, a);
@@ -1908,7 +1937,7 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
     int64_t longest = 0;
     for (int i = 0; i < nspec; ++i) longest = std::max(longest, spec[i].grid.nx);
     const int ppt = pick_ppt(mode, tune, longest);
-    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_batched_prepare: tile_points must be 512, 1024, 2048 or 4096");
+    HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_batched_prepare: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_batched_prepare: stage_lines must be 256 or 512");
     for (int i = 0; i < nspec; ++i) {
@@ -1968,7 +1997,8 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
     batch->tile_points = W;
     batch->stage_lines = kThreads * lm;
     batch->items_main = items[nspec];
-    batch->items_core = citems[nspec];
+    // (FP64 has no line-core pass; none at all marks every pair evaluated)
+    batch->items_core = mode == HK_VOIGT_FP64 && tune && tune->exact_pairs ? 0 : citems[nspec];
     batch->off_args = L.off_args; batch->off_cargs = L.off_cargs;
     batch->off_items = L.off_items; batch->off_citems = L.off_citems;
     batch->off_counter = L.off_counter;
@@ -1980,8 +2010,8 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
                  "hk_voigt_batched_launch: batch not prepared");
     const int ppt = batch->tile_points / kThreads;
     const int lm = batch->stage_lines / kThreads;
-    HK_CHECK_ARG((ppt == 2 || ppt == 4 || ppt == 8 || ppt == 16 ||
-                  (ppt == 1 && batch->mode == HK_VOIGT_FP64)) && (lm == 1 || lm == 2) &&
+    HK_CHECK_ARG((ppt == 2 || ppt == 4 || ppt == 8 ||
+                  ppt == (batch->mode == HK_VOIGT_FP64 ? 1 : 16)) && (lm == 1 || lm == 2) &&
                      (batch->mode == HK_VOIGT_FP64 || batch->mode == HK_VOIGT_FP32C),
                  "hk_voigt_batched_launch: batch not prepared");
     char *base = (char *)batch->workspace;
@@ -1997,8 +2027,8 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
     if (batch->items_main <= 0) return HK_OK;
     const unsigned gm = persistent_grid(batch->items_main);
     if (batch->mode == HK_VOIGT_FP64) {
-        launch_persistent<HK_VOIGT_FP64>(ppt, lm, gm, s, args, items, nspec, counter,
-                                         batch->items_main);
+        launch_persistent(kernel_mode(batch->mode, batch->items_core == 0), ppt, lm, s,
+                          Queue{gm, args, items, nspec, counter, 1}, batch->items_main);
         HK_LAUNCH_CHECK();
         return HK_OK;
     }
@@ -2009,10 +2039,11 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
                        dim3(256), 0, s, cargs, citems, nspec, kCoreW, 1);
     HK_LAUNCH_CHECK();
     const unsigned gc = persistent_grid(batch->items_core);
-    launch_persistent<HK_VOIGT_FP32C>(ppt, lm, gm, s, args, items, nspec, counter, batch->items_main);
+    launch_persistent(batch->mode, ppt, lm, s, Queue{gm, args, items, nspec, counter, 1},
+                      batch->items_main);
     HK_LAUNCH_CHECK();
-    launch_persistent<HK_VOIGT_FP32C>(0, 1, gc, s, cargs, citems, nspec, counter + 1,
-                                      batch->items_core);
+    launch_persistent(batch->mode, 0, 1, s, Queue{gc, cargs, citems, nspec, counter + 1, 1},
+                      batch->items_core);
     HK_LAUNCH_CHECK();
     return HK_OK;
 }
@@ -2140,7 +2171,7 @@ extern "C" int hk_voigt_work_count(const hk_line_state *st, const hk_grid *grid,
     if (int e = check_state(st, "hk_voigt_work_count")) return e;
     if (int e = check_grid(grid, "hk_voigt_work_count")) return e;
     const int ppt = pick_ppt(HK_VOIGT_FP32C, tune, grid->nx);
-    HK_CHECK_ARG(tile_points_ok(mode, tune, ppt), "hk_voigt_work_count: tile_points must be 512, 1024, 2048 or 4096");
+    HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_work_count: tile_points must be 512, 1024, 2048 or 4096");
     const int far = (mode == HK_VOIGT_FP32C && !(tune && tune->exact_pairs)) ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(zero12_kernel, dim3(1), dim3(64), 0, s, counts);

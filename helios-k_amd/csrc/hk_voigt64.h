@@ -32,6 +32,8 @@
 // pass) that spectrum took 2217 us, now 533; 2.35e6 lines on 7e6 points at
 // 10 bar, cut 25: 132 ms, now 15.3.
 #pragma once
+#include <type_traits>
+
 #include "hk_device.h"
 #include "hk_tiles.h"
 
@@ -69,12 +71,24 @@ __device__ __forceinline__ double node_u(int k) { return cos40(2 * k + 1); }
 // points 73 against 106 us, 3e4 points under 1e5 lines 1.12 / 1.97 ms, 3e5
 // points 665 / 805 us; at 1e6 points the two are equal.
 // With every pair evaluated, longer grids take 1024 or 2048 points, so that a
-// line's broadcast serves four or eight points a lane: 1e7 lines, 3e7 points 884
-// ms with 512-point tiles, 572 with 1024, 566 with 2048; 1e5 lines, 3e6 points
-// 3.6, 2.6 and 2.5 ms.  Below 1024 tiles of 2048 points the chip is not full.
+// line's broadcast serves four or eight points a lane (tiles of 512, 1024 and 2048
+// points: 24 spectra of 3e6 points, 1e4 to 5e6 lines, 684, 559 and 535 ms; 1e5
+// lines, 3e6 points 2.12, 2.01 and 1.92 ms; 2.35e6 lines at 10 bar, 7e6 points 128,
+// 115 and 126 ms).  Below 1024 tiles of 2048 points the chip is not full.
+inline int64_t tiles64(int64_t nx, int ppt) { return (nx + kThreads * ppt - 1) / (kThreads * ppt); }
 inline int default_ppt64(int64_t nx, bool exact) {
-    if ((nx + 511) / 512 < 1024) return 1;
-    return !exact ? 2 : (nx + 2047) / 2048 < 1024 ? 4 : 8;
+    if (tiles64(nx, 2) < 1024) return 1;
+    return !exact ? 2 : tiles64(nx, 8) < 1024 ? 4 : 8;
+}
+// The width a caller asks for is kept where it can be of use: 4096 points are
+// taken as 2048 (16 sums a lane leave two waves a SIMD: 1e5 lines, 3e6 points 1.97
+// and 0.81 ms, every pair 3.31 and 1.92), more than 1024 need a tile for each CU
+// (1e4 points, 2000 lines, every pair: 1024 points 428 us, 2048 1086), and with
+// every pair evaluated 512 are taken as 1024 where those fill the chip (above).
+inline int asked_ppt64(int ppt, int64_t nx, bool exact) {
+    if (exact && ppt == 2 && tiles64(nx, 4) >= 1024) return 4;
+    if (ppt > 8) ppt = 8;
+    return ppt == 8 && tiles64(nx, 8) < 256 ? 4 : ppt;
 }
 
 // lines taken per round of the tile loop (each wave lists its own quarter)
@@ -233,11 +247,11 @@ __device__ __forceinline__ bool chi_piece(const Chi &c, double xa, double xb, do
 // 4 binned Gaussian, 0 nothing but the plinth; PLINTH subtracts the line's
 // value at its cut (args.pl) over its whole window; CHI applies args.chi.
 // WHOLE: lines that have one wing formula over all of a wave's points take
-// add_wing (worth its registers where every pair is evaluated: nearly all do).
-template <int PROFILE_, bool PLINTH_, bool CHI_, bool WHOLE_ = false>
+// add_wing.  EXACT: every pair is evaluated, nothing goes through nodes.
+template <int PROFILE_, bool PLINTH_, bool CHI_, bool WHOLE_ = false, bool EXACT_ = false>
 struct LineSum {
     static constexpr int PROFILE = PROFILE_;
-    static constexpr bool PLINTH = PLINTH_, CHI = CHI_, WHOLE = WHOLE_;
+    static constexpr bool PLINTH = PLINTH_, CHI = CHI_, WHOLE = WHOLE_, EXACT = EXACT_;
     // wings that the nodes can take, or a value that underflows to zero beyond
     // x = kDopplerEnd (e^-x^2 does at 27.3)
     static constexpr bool WINGS = PROFILE == 1 || PROFILE == 2;
@@ -573,9 +587,6 @@ __device__ __forceinline__ double core_value(double x, double y, double G, doubl
     return v;
 }
 
-// Point-by-point part of one line on the wave's points: per 64-point segment
-// 2 bits of code, 1: x^2 + y^2 >= 1e4 at all its points (4 nodes), 2: >= 100
-// (8 nodes), 3: some points lie in the line core.
 // Binned Gaussian cell average of exp(-t^2)/sqrt(pi) times vb:
 // (erf(x + h) - erf(x - h)) / 2 with h = vb/2, from the side away from the
 // centre.
@@ -583,6 +594,9 @@ __device__ __forceinline__ double binned_gauss(double x, double h) {
     return x >= 0.0 ? 0.5 * (erfc(x - h) - erfc(x + h)) : 0.5 * (erfc(-x - h) - erfc(-x + h));
 }
 
+// Point-by-point part of one line on the wave's points: per 64-point segment
+// 2 bits of code, 1: x^2 + y^2 >= 1e4 at all its points (4 nodes), 2: >= 100
+// (8 nodes), 3: some points lie in the line core.
 template <class P, int PPT, class Args>
 __device__ __forceinline__ void add_points(const Args &a, uint32_t code, double nu, double ia,
                                            double y, double G, double Apf, double pl, int lo,
@@ -637,27 +651,37 @@ __device__ __forceinline__ void add_points(const Args &a, uint32_t code, double 
     }
 }
 
-// A line that covers the wave's 64 PPT points with one wing formula (N: 2 for
-// x^2 + y^2 >= 1e4, 4 for >= 100): all of a lane's points side by side, so that
-// their reciprocals' chains overlap (every pair of 1e7 lines on 3e7 points, tiles
-// of 1024: 780 ms a segment at a time, 572 so).
-template <int N, int PPT, class Args>
-__device__ __forceinline__ void add_wing(const Args &a, double nu, double ia, double y, double G,
-                                         double jd, double (&acc)[PPT]) {
+// A line that covers the wave's 64 PPT points with one wing formula (N: 1, the
+// asymptotic series, for x^2 + y^2 >= 1e6, 2 for >= 1e4, 4 for >= 100): a lane's
+// points side by side, so that their reciprocals' chains overlap.
+template <int N, int PPT, class XAt>
+__device__ __forceinline__ void add_wing(const XAt &x_at, double nu, double ia, double y, double G,
+                                         double (&acc)[PPT]) {
     const double y2 = y * y;
-    const GH<N> gh;
+    const GH<N == 4 ? 4 : 2> gh;
+    // (series: G is S y / pi, as in add_nodes)
+    if (N == 1) G *= 0.5 * kPi * kISqrtPi;
+    const double p2 = fma(-2.0, y2, 3.75), p3 = -15.0 * y2, p4 = 12.0 * y2 * y2;
 #pragma unroll
     for (int k = 0; k < PPT; ++k) {
-        const double x = (fma(jd + (double)(64 * k), a.dnu, a.numin) - nu) * ia;
-        double num, den;
-        gh_frac(gh, x * x, fma(x, x, y2), num, den);
-        acc[k] = fma(G, num * rcp64(den), acc[k]);
+        if (k > 0 && k % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // (16 at once: spills)
+        const double x = (x_at(k) - nu) * ia;
+        const double r2 = fma(x, x, y2);
+        if (N == 1) {
+            const double q = rcp64(r2);
+            acc[k] = fma(G * q, fma(fma(fma(fma(p4, q, p3), q, p2), q, 1.5), q, 1.0), acc[k]);
+        } else {
+            double num, den;
+            gh_frac(gh, x * x, r2, num, den);
+            acc[k] = fma(G, num * rcp64(den), acc[k]);
+        }
     }
 }
 
 template <int PPT, class P, class Args>
 __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *sh) {
     constexpr int W = kThreads * PPT, WP = 64 * PPT;
+    constexpr bool kNodes = P::WINGS && !P::EXACT;
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -677,6 +701,14 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     double acc[PPT];
 #pragma unroll
     for (int k = 0; k < PPT; ++k) acc[k] = 0.0;
+    // this lane's points, kept where most of the work is theirs
+    double xj[P::EXACT ? PPT : 1];
+    auto x_of = [&](int k) { return fma(jd + (double)(64 * k), a.dnu, a.numin); };
+    auto x_at = [&](int k) { return P::EXACT ? xj[P::EXACT ? k : 0] : x_of(k); };
+    if constexpr (P::EXACT) {
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) xj[k] = x_of(k);
+    }
     // line range of the tile: waves 0 and 1 search one end each
     if (t < 4 * kFN64) sh->cosv[t] = cos40(t);
     if (lane < kFN64) { sh->F[wave][lane] = 0.0; sh->wF[wave][lane] = 0.0; }
@@ -726,7 +758,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         ia = a.ia[i];
                         if (near && !(P::PLINTH && pl != 0.0) && fabs(a.S[i]) < 1.0e300)
                             near = (fabs(D) - hW - a.dnu) * ia <= kDopplerEnd;
-                    } else if (a.far && near && full && fabs(D) >= kFarRatio64 * hW) {
+                    } else if (kNodes && near && full && fabs(D) >= kFarRatio64 * hW) {
                         const double y = a.y[i];
                         ia = a.ia[i];
                         y2 = y * y;
@@ -738,8 +770,10 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         near = cls == 0;
                     }
                 }
-                used |= __ballot(cls != 0) != 0ull;
-                add_far_lines<P>(cls, D, hW, ia, y2, G, pl, chi, f);
+                if constexpr (kNodes) {
+                    used |= __ballot(cls != 0) != 0ull;
+                    add_far_lines<P>(cls, D, hW, ia, y2, G, pl, chi, f);
+                }
                 const unsigned long long m = __ballot(near);
                 if (near)
                     sh->list[wave][cnt + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)e;
@@ -764,7 +798,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         };
         // wave level (a loop of its own: its node sums and the point loop's
         // values do not fit the registers together)
-        {
+        if constexpr (kNodes || kConst) {
             double f[kFN64];
 #pragma unroll
             for (int k = 0; k < kFN64; ++k) f[k] = 0.0;
@@ -774,7 +808,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 int cls = 0;
                 double D = 1.0, ia = 1.0, y2 = 1.0, G = 0.0, pl = 0.0;
                 ChiPiece chi;
-                if ((a.far || kConst) && c0 + lane < total) {
+                if (c0 + lane < total) {
                     const int64_t i = line_at(c0 + lane);
                     const double nu = a.nu[i], hw = a.hw[i];
                     const double dl = xwf - nu, dh = xwl - nu;
@@ -784,7 +818,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         const double el = xfirst - nu, eh = xlast - nu;
                         if (full && !(el > -hw && el < hw && eh > -hw && eh < hw)) wcst -= a.pl[i];
                     }
-                    if (P::WINGS && a.far && full && fabs(D) >= kFarRatio64 * hw_w) {
+                    if (kNodes && full && fabs(D) >= kFarRatio64 * hw_w) {
                         const double y = a.y[i];
                         ia = a.ia[i];
                         y2 = y * y;
@@ -812,7 +846,8 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
             uint32_t code = 0;
             int lo = 0, hi = 0;
             double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0, pl = 0.0;
-            if (e < total && !((sh->taken[wave][c0 >> 6] >> lane) & 1ull)) {
+            bool far = false;                    // x^2 + y^2 >= 1e6 at all points
+            if (e < total && !((kNodes || kConst) && (sh->taken[wave][c0 >> 6] >> lane) & 1ull)) {
                 const int64_t i = line_at(e);
                 nu = a.nu[i];
                 clip_window(nu, a.hw[i], a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
@@ -830,6 +865,11 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
                         const float mg = 2.0f + 1.0e-5f * fabsf(cen);
                         const bool in1 = fy2 < 1.0002e2f, in2 = fy2 < 1.0002e4f;
+                        if constexpr (P::WHOLE) {
+                            const float r3 = sqrtf(fmaxf(1.0002e6f - fy2, 0.0f)) / vb;
+                            far = !(fy2 < 1.0002e6f && cen - r3 - mg <= (float)(WP - 1) &&
+                                    cen + r3 + mg >= 0.0f) && fy2 < 1.0e12f;
+                        }
 #pragma unroll
                         for (int k = 0; k < PPT; ++k) {
                             const int s0 = 64 * k, s1 = s0 + 63;
@@ -858,21 +898,30 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 }
             }
             unsigned long long m = __ballot(code != 0);
+            if constexpr (P::WHOLE) {
+                // lines of one formula over the wave, in a loop of its own each:
+                // merged, every line copies the sums between its paths
+                constexpr uint32_t ones = 0x55555555u & (uint32_t)((1ull << (2 * PPT)) - 1);
+                const bool whole = lo == 0 && hi == WP;
+                auto wings = [&](auto formula, bool mine) {
+                    unsigned long long w = __ballot(mine);
+                    m &= ~w;
+                    while (w) {
+                        const int b = __builtin_ctzll(w);
+                        w &= w - 1ull;
+                        add_wing<formula, PPT>(x_at, lane_f64(nu, b), lane_f64(ia, b),
+                                               lane_f64(y, b), lane_f64(G, b), acc);
+                    }
+                };
+                wings(std::integral_constant<int, 1>{}, whole && code == ones && far);
+                wings(std::integral_constant<int, 2>{}, whole && code == ones && !far);
+                wings(std::integral_constant<int, 4>{}, whole && code == 2 * ones);
+            }
             while (m) {
                 const int b = __builtin_ctzll(m);
                 m &= m - 1ull;
                 const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
                 const uint32_t scode = (uint32_t)__builtin_amdgcn_readlane((int)code, b);
-                if constexpr (P::WHOLE) {
-                    constexpr uint32_t ones = 0x55555555u & (uint32_t)((1ull << (2 * PPT)) - 1);
-                    if (slo == 0 && shi == WP && (scode == ones || scode == 2 * ones)) {
-                        const double lnu = lane_f64(nu, b), lia = lane_f64(ia, b);
-                        const double ly = lane_f64(y, b), lG = lane_f64(G, b);
-                        if (scode == ones) add_wing<2, PPT>(a, lnu, lia, ly, lG, jd, acc);
-                        else add_wing<4, PPT>(a, lnu, lia, ly, lG, jd, acc);
-                        continue;
-                    }
-                }
                 add_points<P, PPT>(a, scode,
                                    lane_f64(nu, b), lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b),
                                    P::PROFILE == 1 ? lane_f64(Apf, b) : 0.0,

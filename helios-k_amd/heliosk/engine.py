@@ -207,7 +207,7 @@ def _tune(tile_points=0, exact_pairs=False, stage_lines=0):
 def voigt(state, grid, kmin=0.0, mode=HK_VOIGT_FP32C, tile_points=0, K=None, accumulate=False,
           stream=None, workspace=None, exact_pairs=False, stage_lines=0):
     """K_j = kmin + sum_i S_i Re w / sqrt(pi) on the grid (or K += sum).
-    exact_pairs: FP32C evaluates every pair instead of interpolating the far
+    exact_pairs: every pair is evaluated, instead of interpolating the far
     field of distant lines; stage_lines: lines per LDS stage (256 or 512)."""
     tune = _tune(tile_points, exact_pairs, stage_lines)
     if K is None:
