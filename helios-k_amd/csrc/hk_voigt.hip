@@ -2130,25 +2130,33 @@ extern "C" int hk_voigt_autotune(const hk_line_state *st, const hk_grid *grid, i
     hipEvent_t e0, e1;
     HK_HIP(hipEventCreate(&e0));
     HK_HIP(hipEventCreate(&e1));
-    float bestms = 0.0f;
+    float bestms = -1.0f;
     int bestw = 0, bests = 0, rc = HK_OK;
-    for (int c = 0; c < 8 && rc == HK_OK; ++c) {
-        hk_tune t = {kCand[c % 4], exact, kStageCand[c / 4]};
-        rc = hk_voigt_accumulate(st, grid, 0.0, 0, mode, &t, K, ws, ws_bytes, stream);
-        if (rc != HK_OK) break;
-        if (hipEventRecord(e0, s) != hipSuccess) { rc = HK_ERR_HIP; break; }
-        rc = hk_voigt_accumulate(st, grid, 0.0, 0, mode, &t, K, ws, ws_bytes, stream);
-        if (rc != HK_OK) break;
-        float dt = 0.0f;
+    auto run = [&](const hk_tune &t, float &dt) {
+        int e = hk_voigt_accumulate(st, grid, 0.0, 0, mode, &t, K, ws, ws_bytes, stream);
+        if (e != HK_OK) return e;
+        if (hipEventRecord(e0, s) != hipSuccess) return (int)HK_ERR_HIP;
+        e = hk_voigt_accumulate(st, grid, 0.0, 0, mode, &t, K, ws, ws_bytes, stream);
+        if (e != HK_OK) return e;
         if (hipEventRecord(e1, s) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
             hipEventElapsedTime(&dt, e0, e1) != hipSuccess) {
             set_error("hk_voigt_autotune: event timing failed");
-            rc = HK_ERR_HIP;
-            break;
+            return (int)HK_ERR_HIP;
         }
-        if (ms) ms[c] = dt;
-        if (bestw == 0 || dt < bestms) { bestms = dt; bestw = t.tile_points; bests = t.stage_lines; }
+        if (bestms < 0.0f || dt < bestms) { bestms = dt; bestw = t.tile_points; bests = t.stage_lines; }
+        return (int)HK_OK;
+    };
+    float dts[8] = {};
+    for (int c = 0; c < 8 && rc == HK_OK; ++c) {
+        // FP64 has no stages: its widths are timed once
+        if (mode == HK_VOIGT_FP64 && c >= 4) dts[c] = dts[c - 4];
+        else rc = run(hk_tune{kCand[c % 4], exact, kStageCand[c / 4]}, dts[c]);
+        if (ms && rc == HK_OK) ms[c] = dts[c];
     }
+    // its own choice for a short grid is narrower than any width to ask for
+    float own = 0.0f;
+    if (rc == HK_OK && mode == HK_VOIGT_FP64 && default_ppt64(grid->nx, exact != 0) == 1)
+        rc = run(hk_tune{0, exact, kStageCand[0]}, own);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc == HK_OK) {

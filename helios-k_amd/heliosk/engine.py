@@ -276,7 +276,8 @@ def autotune(state, grid, mode=HK_VOIGT_FP32C, stream=None, exact_pairs=False):
     """Fastest (tile width, lines per LDS stage) of the main pass for this
     input (hk_voigt_autotune; the library keeps the choice per problem
     signature for the process).  Returns (tile_points, stage_lines,
-    {(tile, stage): ms}) -- ms 0 for a cached choice."""
+    {(tile, stage): ms}) -- ms 0 for a cached choice, tile_points 0 where the
+    FP64 form's own narrower width for short grids is the fastest."""
     K = torch.empty(grid.nx, dtype=torch.float64, device=_dev())
     tune = _tune(0)
     nbytes = lib().hk_voigt_workspace_bytes(ctypes.byref(grid), ctypes.byref(tune))

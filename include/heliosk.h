@@ -248,7 +248,9 @@ int hk_voigt_work_count(const hk_line_state *st, const hk_grid *grid, int mode,
  * {512, 1024, 2048, 4096} points and each stage of {256, 512} lines (one
  * untimed and one timed launch each, device events) and writes the fastest
  * pair into *best; ms[8] (may be NULL) receives the timings, tile-major
- * within each stage size (ms[4 * (stage == 512) + tile index]).  K is overwritten; the workspace must be sized
+ * within each stage size (ms[4 * (stage == 512) + tile index]).  HK_VOIGT_FP64
+ * has no stages (its widths are timed once) and for short grids a width of its
+ * own, which is timed too: tile_points 0 if that is the fastest.  K is overwritten; the workspace must be sized
  * for the smallest tile (hk_voigt_workspace_bytes covers every size).
  * Waits for the stream.  Results of different tile sizes agree to
  * rounding, not bit for bit, so the choice is cached for the process per
