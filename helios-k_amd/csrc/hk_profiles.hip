@@ -82,7 +82,7 @@ struct PArgs {
 
 // PROFILE 1..4: profile sums (minus plinths when PLINTH); PROFILE 0: the
 // plinth subtraction alone (after an FP32C or compat Voigt sum).
-template <int PPT, int PROFILE, bool PLINTH, bool CHI>
+template <int PPT, int PROFILE, bool PLINTH, bool CHI, bool SPARSE>
 __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
     __shared__ Far64LDS sh;
     if constexpr (CHI) {
@@ -101,19 +101,25 @@ __global__ __launch_bounds__(kThreads, 4) void profile_tiles_kernel(PArgs a) {
                 a.chi.hi = -a.chi.lo;
                 __syncthreads();
             }
-            tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
+            tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI, SPARSE && PROFILE <= 2 && !CHI, false, SPARSE>>(a, (int64_t)blockIdx.x, &sh);
         }
     } else {
-        tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI>>(a, (int64_t)blockIdx.x, &sh);
+        tile_f64<PPT, LineSum<PROFILE, PLINTH, CHI, SPARSE && PROFILE <= 2 && !CHI, false, SPARSE>>(a, (int64_t)blockIdx.x, &sh);
     }
 }
 
 template <int PROFILE, bool PLINTH, bool CHI = false>
 void launch_profile(hipStream_t s, const PArgs &a) {
-    const int ppt = default_ppt64(a.nx, false);
-    const dim3 g((unsigned)((a.nx + kThreads * ppt - 1) / (kThreads * ppt))), b(kThreads);
-    if (ppt == 1) hipLaunchKernelGGL((profile_tiles_kernel<1, PROFILE, PLINTH, CHI>), g, b, 0, s, a);
-    else hipLaunchKernelGGL((profile_tiles_kernel<2, PROFILE, PLINTH, CHI>), g, b, 0, s, a);
+    constexpr bool kSparse = PROFILE != 0;      // (plinths alone are constants)
+    const bool sparse = kSparse && sparse64(a.nx, a.nl);
+    const int ppt = default_ppt64(a.nx, a.nl, false);
+    const dim3 g((unsigned)tiles64(a.nx, ppt)), b(kThreads);
+    if (sparse) {
+        hipLaunchKernelGGL((profile_tiles_kernel<2, PROFILE, PLINTH, CHI, kSparse>), g, b, 0, s, a);
+        return;
+    }
+    if (ppt == 1) hipLaunchKernelGGL((profile_tiles_kernel<1, PROFILE, PLINTH, CHI, false>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((profile_tiles_kernel<2, PROFILE, PLINTH, CHI, false>), g, b, 0, s, a);
 }
 
 template <int PROFILE>

@@ -1395,14 +1395,16 @@ __device__ __forceinline__ void core_f32c(const VArgs &a, int64_t tile, Core32 *
 // line-core pass.
 constexpr int main_waves(int mode, int ppt, int lm);
 
-// Kernels' MODE beside the public forms: FP64 with every pair evaluated.
-constexpr int kFP64Pairs = 3;
+// Kernels' MODE beside the public forms: FP64 with every pair evaluated, FP64 for
+// sparse lists.
+constexpr int kFP64Pairs = 3, kFP64Sparse = 4;
 
-// The FP64 forms' line sum.  Whole-wave lines are
-// worth their registers there, where nearly all lines are, and on tiles that a
-// caller makes so wide that few lines are far.
+// The FP64 forms' line sum.  Whole-wave lines are worth their registers where
+// nearly all lines are (every pair, tiles of few lines) and on tiles that a caller
+// makes so wide that few lines are far.
 template <int MODE, int PPT>
-using Sum64 = LineSum<1, false, false, MODE == kFP64Pairs || (PPT >= 4), MODE == kFP64Pairs>;
+using Sum64 = LineSum<1, false, false, MODE == kFP64Pairs || MODE == kFP64Sparse || (PPT >= 4), MODE == kFP64Pairs,
+                      MODE == kFP64Sparse>;
 
 template <int MODE, int PPT, int LM>
 __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_kernel(VArgs a) {
@@ -1670,11 +1672,11 @@ bool tile_points_ok(const hk_tune *tune) {
 //  FP32C  1024-point tiles (smaller ones trade direct pairs for node
 //         evaluations; 1024 was fastest at 1e7 lines x 3e7 points);
 //  FP64   default_ppt64.
-int pick_ppt(int mode, const hk_tune *tune, int64_t nx) {
+int pick_ppt(int mode, const hk_tune *tune, int64_t nx, int64_t nl) {
     const bool exact = tune && tune->exact_pairs;
     const int asked = tune && tune->tile_points > 0 ? tune->tile_points / kThreads : 0;
     if (mode != HK_VOIGT_FP64) return asked ? asked : 4;
-    return asked ? asked_ppt64(asked, nx, exact) : default_ppt64(nx, exact);
+    return asked ? asked_ppt64(asked, nx, exact) : default_ppt64(nx, nl, exact);
 }
 
 // Lines per LDS stage of the main pass: 256 (default) or 512; returns the
@@ -1684,10 +1686,12 @@ int pick_lm(const hk_tune *tune) {
     return sl == kThreads ? 1 : (sl == 2 * kThreads ? 2 : 0);
 }
 
-// MODE of the kernels for a public form and its exact_pairs (FP32C's kernels see
-// that in their arguments).
-int kernel_mode(int mode, bool exact) {
-    return mode == HK_VOIGT_FP64 && exact ? kFP64Pairs : mode;
+// MODE of the kernels for a public form, its exact_pairs (FP32C's kernels see that
+// in their arguments) and, for FP64, tiles of 256 ppt points on nx points under nl
+// lines.
+int kernel_mode(int mode, bool exact, int ppt, int64_t nx, int64_t nl) {
+    if (mode != HK_VOIGT_FP64) return mode;
+    return exact ? kFP64Pairs : ppt == 2 && sparse64(nx, nl) ? kFP64Sparse : mode;
 }
 
 // (tiles of 256 points are FP64's only, those of 4096 FP32C's, and FP64 has no
@@ -1705,7 +1709,9 @@ void launch_tiles_lm(int ppt, int64_t ntiles, hipStream_t s, const VArgs &a) {
 }
 
 void launch_tiles(int kmode, int ppt, int lm, int64_t ntiles, hipStream_t s, const VArgs &a) {
-    if (kmode == kFP64Pairs) launch_tiles_lm<kFP64Pairs, 1>(ppt, ntiles, s, a);
+    if (kmode == kFP64Sparse)
+        hipLaunchKernelGGL((voigt_tiles_kernel<kFP64Sparse, 2, 1>), dim3((unsigned)ntiles), dim3(kThreads), 0, s, a);
+    else if (kmode == kFP64Pairs) launch_tiles_lm<kFP64Pairs, 1>(ppt, ntiles, s, a);
     else if (kmode == HK_VOIGT_FP64) launch_tiles_lm<HK_VOIGT_FP64, 1>(ppt, ntiles, s, a);
     else if (lm == 2) launch_tiles_lm<HK_VOIGT_FP32C, 2>(ppt, ntiles, s, a);
     else launch_tiles_lm<HK_VOIGT_FP32C, 1>(ppt, ntiles, s, a);
@@ -1742,7 +1748,8 @@ void launch_persistent(int kmode, int ppt, int lm, hipStream_t s, Queue q, int64
     // at least 32 chunks a workgroup, so that the last ones end together (4:
     // the line-core pass above 9.8 ms, 16: 7.1, 32: 6.8, 64: 7.2)
     q.chunk = (int)std::max<int64_t>(1, std::min<int64_t>(64, nitems / (32 * (int64_t)q.grid)));
-    if (kmode == kFP64Pairs) launch_persistent_lm<kFP64Pairs, 1>(ppt, s, q);
+    if (kmode == kFP64Sparse) launch_queue<kFP64Sparse, 2, 1>(s, q);
+    else if (kmode == kFP64Pairs) launch_persistent_lm<kFP64Pairs, 1>(ppt, s, q);
     else if (kmode == HK_VOIGT_FP64) launch_persistent_lm<HK_VOIGT_FP64, 1>(ppt, s, q);
     else if (ppt == 0) launch_queue<HK_VOIGT_FP32C, 0, 1>(s, q);
     else if (lm == 2) launch_persistent_lm<HK_VOIGT_FP32C, 2>(ppt, s, q);
@@ -1782,7 +1789,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
                  "hk_voigt_accumulate: mode %d", mode);
     if (int e = check_state(st, "hk_voigt_accumulate")) return e;
     if (int e = check_grid(grid, "hk_voigt_accumulate")) return e;
-    const int ppt = pick_ppt(mode, tune, grid->nx);
+    const int ppt = pick_ppt(mode, tune, grid->nx, st->nlines);
     HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_accumulate: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_accumulate: stage_lines must be 256 or 512");
@@ -1806,7 +1813,7 @@ extern "C" int hk_voigt_accumulate(const hk_line_state *st, const hk_grid *grid,
     a.kmin = kmin; a.accumulate = accumulate; a.K = K;
     a.far = tune && tune->exact_pairs ? 0 : 1;
     if (mode == HK_VOIGT_FP64) {            // one pass; its tiles search their own line ranges
-        launch_tiles(kernel_mode(mode, a.far == 0), ppt, lm, ntiles, s, a);
+        launch_tiles(kernel_mode(mode, a.far == 0, ppt, grid->nx, st->nlines), ppt, lm, ntiles, s, a);
         HK_LAUNCH_CHECK();
         return HK_OK;
     }
@@ -1933,10 +1940,15 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
     HK_CHECK_ARG(nspec > 0 && spec && ws && batch, "hk_voigt_batched_prepare: bad arguments");
     HK_CHECK_ARG(mode == HK_VOIGT_FP64 || mode == HK_VOIGT_FP32C,
                  "hk_voigt_batched_prepare: mode %d", mode);
-    // one tile width for the batch: that of its longest grid
-    int64_t longest = 0;
-    for (int i = 0; i < nspec; ++i) longest = std::max(longest, spec[i].grid.nx);
-    const int ppt = pick_ppt(mode, tune, longest);
+    // one tile width for the batch: that of all its points and lines together,
+    // since its tiles share the chip (100 spectra of 1e5 points under 500 lines by
+    // the width for one of them 1.18 ms, so 0.66)
+    int64_t points = 0, lines = 0;
+    for (int i = 0; i < nspec; ++i) {
+        points += std::max<int64_t>(spec[i].grid.nx, 0);
+        lines += std::max<int64_t>(spec[i].st.nlines, 0);
+    }
+    const int ppt = pick_ppt(mode, tune, points, lines);
     HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_batched_prepare: tile_points must be 512, 1024, 2048 or 4096");
     const int lm = pick_lm(tune);
     HK_CHECK_ARG(lm > 0, "hk_voigt_batched_prepare: stage_lines must be 256 or 512");
@@ -1997,8 +2009,11 @@ extern "C" int hk_voigt_batched_prepare(int nspec, const hk_spectrum *spec, int 
     batch->tile_points = W;
     batch->stage_lines = kThreads * lm;
     batch->items_main = items[nspec];
-    // (FP64 has no line-core pass; none at all marks every pair evaluated)
-    batch->items_core = mode == HK_VOIGT_FP64 && tune && tune->exact_pairs ? 0 : citems[nspec];
+    // (FP64 has no line-core pass: 0 marks every pair evaluated, -1 sparse lists)
+    batch->items_core = citems[nspec];
+    const int kmode = kernel_mode(mode, tune && tune->exact_pairs, ppt, points, lines);
+    if (kmode == kFP64Pairs) batch->items_core = 0;
+    if (kmode == kFP64Sparse) batch->items_core = -1;
     batch->off_args = L.off_args; batch->off_cargs = L.off_cargs;
     batch->off_items = L.off_items; batch->off_citems = L.off_citems;
     batch->off_counter = L.off_counter;
@@ -2027,7 +2042,9 @@ extern "C" int hk_voigt_batched_launch(const hk_voigt_batch *batch, hk_stream_t 
     if (batch->items_main <= 0) return HK_OK;
     const unsigned gm = persistent_grid(batch->items_main);
     if (batch->mode == HK_VOIGT_FP64) {
-        launch_persistent(kernel_mode(batch->mode, batch->items_core == 0), ppt, lm, s,
+        const int kmode = batch->items_core == 0 ? kFP64Pairs
+                          : batch->items_core < 0 && ppt == 2 ? kFP64Sparse : batch->mode;
+        launch_persistent(kmode, ppt, lm, s,
                           Queue{gm, args, items, nspec, counter, 1}, batch->items_main);
         HK_LAUNCH_CHECK();
         return HK_OK;
@@ -2155,7 +2172,7 @@ extern "C" int hk_voigt_autotune(const hk_line_state *st, const hk_grid *grid, i
     }
     // its own choice for a short grid is narrower than any width to ask for
     float own = 0.0f;
-    if (rc == HK_OK && mode == HK_VOIGT_FP64 && default_ppt64(grid->nx, exact != 0) == 1)
+    if (rc == HK_OK && mode == HK_VOIGT_FP64 && default_ppt64(grid->nx, st->nlines, exact != 0) == 1)
         rc = run(hk_tune{0, exact, kStageCand[0]}, own);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -2178,7 +2195,7 @@ extern "C" int hk_voigt_work_count(const hk_line_state *st, const hk_grid *grid,
                  mode);
     if (int e = check_state(st, "hk_voigt_work_count")) return e;
     if (int e = check_grid(grid, "hk_voigt_work_count")) return e;
-    const int ppt = pick_ppt(HK_VOIGT_FP32C, tune, grid->nx);
+    const int ppt = pick_ppt(HK_VOIGT_FP32C, tune, grid->nx, 0);
     HK_CHECK_ARG(tile_points_ok(tune), "hk_voigt_work_count: tile_points must be 512, 1024, 2048 or 4096");
     const int far = (mode == HK_VOIGT_FP32C && !(tune && tune->exact_pairs)) ? 1 : 0;
     hipStream_t s = (hipStream_t)stream;

@@ -76,7 +76,17 @@ __device__ __forceinline__ double node_u(int k) { return cos40(2 * k + 1); }
 // lines, 3e6 points 2.12, 2.01 and 1.92 ms; 2.35e6 lines at 10 bar, 7e6 points 128,
 // 115 and 126 ms).  Below 1024 tiles of 2048 points the chip is not full.
 inline int64_t tiles64(int64_t nx, int ppt) { return (nx + kThreads * ppt - 1) / (kThreads * ppt); }
-inline int default_ppt64(int64_t nx, bool exact) {
+// Sparse lists, at most two lines per 512 points on average, have kernels of their
+// own that take a tile of few lines point by point: its nodes, of which a line or
+// two fill one lane each, their series and the registers spilled around them took
+// most of the time (500 lines, 3e6 points, cut 25: 78 us, 34 without; 5000 lines
+// 147 and 90).  In the kernel for all lists the second path costs dense ones 2 to
+// 9 %.
+inline bool sparse64(int64_t nx, int64_t nl) {
+    return nl <= 2 * tiles64(nx, 2) && tiles64(nx, 2) >= 512;
+}
+inline int default_ppt64(int64_t nx, int64_t nl, bool exact) {
+    if (!exact && sparse64(nx, nl)) return 2;
     if (tiles64(nx, 2) < 1024) return 1;
     return !exact ? 2 : tiles64(nx, 8) < 1024 ? 4 : 8;
 }
@@ -90,6 +100,9 @@ inline int asked_ppt64(int ppt, int64_t nx, bool exact) {
     if (ppt > 8) ppt = 8;
     return ppt == 8 && tiles64(nx, 8) < 256 ? 4 : ppt;
 }
+
+// Tiles of a sparse list that at most this many lines can reach.
+constexpr int kFewLines = 32;
 
 // lines taken per round of the tile loop (each wave lists its own quarter)
 constexpr int kRound64 = 4096;
@@ -248,10 +261,13 @@ __device__ __forceinline__ bool chi_piece(const Chi &c, double xa, double xb, do
 // value at its cut (args.pl) over its whole window; CHI applies args.chi.
 // WHOLE: lines that have one wing formula over all of a wave's points take
 // add_wing.  EXACT: every pair is evaluated, nothing goes through nodes.
-template <int PROFILE_, bool PLINTH_, bool CHI_, bool WHOLE_ = false, bool EXACT_ = false>
+// SPARSE: tiles of few lines take them point by point, each wave by itself.
+template <int PROFILE_, bool PLINTH_, bool CHI_, bool WHOLE_ = false, bool EXACT_ = false,
+          bool SPARSE_ = false>
 struct LineSum {
     static constexpr int PROFILE = PROFILE_;
     static constexpr bool PLINTH = PLINTH_, CHI = CHI_, WHOLE = WHOLE_, EXACT = EXACT_;
+    static constexpr bool SPARSE = SPARSE_;
     // wings that the nodes can take, or a value that underflows to zero beyond
     // x = kDopplerEnd (e^-x^2 does at 27.3)
     static constexpr bool WINGS = PROFILE == 1 || PROFILE == 2;
@@ -651,12 +667,12 @@ __device__ __forceinline__ void add_points(const Args &a, uint32_t code, double 
     }
 }
 
-// A line that covers the wave's 64 PPT points with one wing formula (N: 1, the
-// asymptotic series, for x^2 + y^2 >= 1e6, 2 for >= 1e4, 4 for >= 100): a lane's
+// A line that covers the wave's 64 PPT points with one wing formula (N: 0, Lorentz
+// less the plinth, 1, the asymptotic series, for x^2 + y^2 >= 1e6, 2 for >= 1e4, 4 for >= 100): a lane's
 // points side by side, so that their reciprocals' chains overlap.
 template <int N, int PPT, class XAt>
 __device__ __forceinline__ void add_wing(const XAt &x_at, double nu, double ia, double y, double G,
-                                         double (&acc)[PPT]) {
+                                         double pl, double (&acc)[PPT]) {
     const double y2 = y * y;
     const GH<N == 4 ? 4 : 2> gh;
     // (series: G is S y / pi, as in add_nodes)
@@ -667,14 +683,138 @@ __device__ __forceinline__ void add_wing(const XAt &x_at, double nu, double ia, 
         if (k > 0 && k % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // (16 at once: spills)
         const double x = (x_at(k) - nu) * ia;
         const double r2 = fma(x, x, y2);
-        if (N == 1) {
+        if (N == 0) {
+            acc[k] += G / r2 - pl;
+        } else if (N == 1) {
             const double q = rcp64(r2);
-            acc[k] = fma(G * q, fma(fma(fma(fma(p4, q, p3), q, p2), q, 1.5), q, 1.0), acc[k]);
+            acc[k] += fma(G * q, fma(fma(fma(fma(p4, q, p3), q, p2), q, 1.5), q, 1.0), -pl);
         } else {
             double num, den;
             gh_frac(gh, x * x, r2, num, den);
-            acc[k] = fma(G, num * rcp64(den), acc[k]);
+            acc[k] += fma(G, num * rcp64(den), -pl);
         }
+    }
+}
+
+// The wave's part of a tile.
+struct WavePoints {
+    int64_t jw;                 // first point
+    int nw;                     // points
+    double xwf, jd, inv_dnu;    // centre of the first, this lane's index, 1/dnu
+};
+
+// Up to 64 lines point by point: one line per lane (i: its index, -1: none) finds
+// its window and formulas on the wave's points, then the wave takes them in turn.
+template <int PPT, class P, class Args, class XAt>
+__device__ __forceinline__ void add_lines(const Args &a, int64_t i, const WavePoints &w,
+                                          const XAt &x_at, double (&acc)[PPT], double *tab) {
+    constexpr int WP = 64 * PPT;
+    const int64_t jw = w.jw;
+    const int nw = w.nw;
+    const double xwf = w.xwf, jd = w.jd, inv_dnu = w.inv_dnu;
+    uint32_t code = 0;
+    int lo = 0, hi = 0;
+    double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0, pl = 0.0;
+    bool far = false;                            // x^2 + y^2 >= 1e6 at all points
+    if (i >= 0) {
+        nu = a.nu[i];
+        const double hw = a.hw[i], S = a.S[i];
+        y = a.y[i];
+        ia = a.ia[i];
+        clip_window(nu, hw, a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
+        if (lo < hi) {
+            G = line_factor<P>(S, y);
+            if constexpr (P::PLINTH) pl = a.pl[i];
+            if constexpr (P::PROFILE == 1) {
+                // conservative point intervals with x^2 + y^2 < 100, 1e4
+                const float vb = (float)(a.dnu * ia), fy2 = (float)(y * y);
+                const float cen = (float)((nu - xwf) * inv_dnu);
+                const float r1 = sqrtf(fmaxf(1.0002e2f - fy2, 0.0f)) / vb;
+                const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
+                const float mg = 2.0f + 1.0e-5f * fabsf(cen);
+                const bool in1 = fy2 < 1.0002e2f, in2 = fy2 < 1.0002e4f;
+                if constexpr (P::WHOLE) {
+                    const float r3 = sqrtf(fmaxf(1.0002e6f - fy2, 0.0f)) / vb;
+                    far = !(fy2 < 1.0002e6f && cen - r3 - mg <= (float)(WP - 1) &&
+                            cen + r3 + mg >= 0.0f) && fy2 < 1.0e12f;
+                }
+#pragma unroll
+                for (int k = 0; k < PPT; ++k) {
+                    const int s0 = 64 * k, s1 = s0 + 63;
+                    if (lo > s1 || hi <= s0) continue;
+                    const bool c3 = in1 && cen - r1 - mg <= (float)s1 && cen + r1 + mg >= (float)s0;
+                    const bool c2 = in2 && cen - r2 - mg <= (float)s1 && cen + r2 + mg >= (float)s0;
+                    code |= (c3 ? 3u : c2 ? 2u : 1u) << (2 * k);
+                }
+                if (code & (code >> 1) & 0x55555555u) Apf = S * kISqrtPi * core_pole(y);
+            } else {
+                // segments that the window touches; a compact profile's
+                // only where it is not zero, unless a plinth is there
+                int l = lo, h = hi;
+                const bool part = P::PROFILE == 0 || (P::PLINTH && pl != 0.0);
+                if (P::COMPACT && !part && fabs(S) < 1.0e300) {
+                    const double off = (nu - xwf) * inv_dnu;
+                    const double w = kDopplerEnd / ia * inv_dnu + 2.0;
+                    l = max(lo, (int)fmin(fmax(off - w, 0.0), (double)nw));
+                    h = min(hi, (int)fmin(fmax(off + w, 0.0), (double)nw));
+                }
+                if (P::PROFILE != 0 || part)
+#pragma unroll
+                    for (int k = 0; k < PPT; ++k)
+                        if (l < 64 * k + 64 && h > 64 * k && l < h) code |= 1u << (2 * k);
+            }
+        }
+    }
+    unsigned long long m = __ballot(code != 0);
+    if constexpr (P::WHOLE) {
+        // lines of one formula over the wave, in a loop of its own each:
+        // merged, every line copies the sums between its paths
+        constexpr uint32_t ones = 0x55555555u & (uint32_t)((1ull << (2 * PPT)) - 1);
+        const bool whole = lo == 0 && hi == WP;
+        auto wings = [&](auto formula, bool these) {
+            unsigned long long q = __ballot(these);
+            m &= ~q;
+            while (q) {
+                const int b = __builtin_ctzll(q);
+                q &= q - 1ull;
+                add_wing<formula, PPT>(x_at, lane_f64(nu, b), lane_f64(ia, b),
+                                       lane_f64(y, b), lane_f64(G, b),
+                                       P::PLINTH ? lane_f64(pl, b) : 0.0, acc);
+            }
+        };
+        if constexpr (P::PROFILE == 2) {
+            wings(std::integral_constant<int, 0>{}, whole && code == ones);
+        } else {
+            wings(std::integral_constant<int, 1>{}, whole && code == ones && far);
+            wings(std::integral_constant<int, 2>{}, whole && code == ones && !far);
+            wings(std::integral_constant<int, 4>{}, whole && code == 2 * ones);
+        }
+    }
+    while (m) {
+        const int b = __builtin_ctzll(m);
+        m &= m - 1ull;
+        const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
+        const uint32_t scode = (uint32_t)__builtin_amdgcn_readlane((int)code, b);
+        add_points<P, PPT>(a, scode,
+                           lane_f64(nu, b), lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b),
+                           P::PROFILE == 1 ? lane_f64(Apf, b) : 0.0,
+                           P::PLINTH ? lane_f64(pl, b) : 0.0, slo, shi,
+                           slo == 0 && shi == nw, jd, acc, tab);
+    }
+}
+
+// Writes the wave's sums.
+template <int PPT, class P, class Args, class XAt>
+__device__ __forceinline__ void store_points(const Args &a, const WavePoints &w, const XAt &x_at,
+                                             const double (&acc)[PPT]) {
+#pragma unroll
+    for (int k = 0; k < PPT; ++k) {
+        const int64_t j = w.jw + (threadIdx.x & 63) + 64 * k;
+        if constexpr (P::CHI) {
+            const double x = x_at(k);
+            if (a.side != 0 && (x > a.lo && x < a.hi) != (a.side > 0)) continue;
+        }
+        if (j < a.nx) a.K[j] = a.accumulate ? a.K[j] + acc[k] : a.kmin + acc[k];
     }
 }
 
@@ -710,8 +850,11 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         for (int k = 0; k < PPT; ++k) xj[k] = x_of(k);
     }
     // line range of the tile: waves 0 and 1 search one end each
-    if (t < 4 * kFN64) sh->cosv[t] = cos40(t);
-    if (lane < kFN64) { sh->F[wave][lane] = 0.0; sh->wF[wave][lane] = 0.0; }
+    auto clear = [&]() {
+        if (t < 4 * kFN64) sh->cosv[t] = cos40(t);
+        if (lane < kFN64) { sh->F[wave][lane] = 0.0; sh->wF[wave][lane] = 0.0; }
+    };
+    if constexpr (!P::SPARSE) clear();
     if (wave < 2) {
         const double R = a.radius[0];
         int64_t b = 0;
@@ -722,6 +865,18 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
     }
     __syncthreads();
     const int64_t first = sh->range[0], last = sh->range[1];
+    const WavePoints w = {jw, nw, xwf, jd, inv_dnu};
+    if constexpr (P::SPARSE) {
+        if (last - first <= kFewLines) {
+            if (nw == 0) return;
+            if (first < last)
+                add_lines<PPT, P>(a, lane < last - first ? first + lane : -1, w, x_at, acc,
+                                  sh->tab[wave]);
+            store_points<PPT, P>(a, w, x_at, acc);
+            return;
+        }
+        clear();                                 // (barriers follow before its readers)
+    }
     bool any_far = false, any_wave = false;
     // plinths alone: those of lines that cover the tile, the wave
     constexpr bool kConst = P::PLINTH && P::PROFILE == 0;
@@ -743,7 +898,11 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 ChiPiece chi;
                 if (e < nr) {
                     const int64_t i = r0 + e;
+                    // (all loads at once: one wait on memory, not three)
                     const double nu = a.nu[i], hw = a.hw[i];
+                    double y = 0.0, S = 0.0;
+                    if constexpr (kNodes || P::COMPACT) { ia = a.ia[i]; S = a.S[i]; }
+                    if constexpr (kNodes) y = a.y[i];
                     const double dl = xfirst - nu, dh = xlast - nu;
                     near = hw > 0.0 && dl < hw && dh > -hw;
                     const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
@@ -755,14 +914,11 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         if (near && full) cst -= pl;
                         near = near && !full;
                     } else if (P::COMPACT) {
-                        ia = a.ia[i];
-                        if (near && !(P::PLINTH && pl != 0.0) && fabs(a.S[i]) < 1.0e300)
+                        if (near && !(P::PLINTH && pl != 0.0) && fabs(S) < 1.0e300)
                             near = (fabs(D) - hW - a.dnu) * ia <= kDopplerEnd;
                     } else if (kNodes && near && full && fabs(D) >= kFarRatio64 * hW) {
-                        const double y = a.y[i];
-                        ia = a.ia[i];
                         y2 = y * y;
-                        G = line_factor<P>(a.S[i], y);
+                        G = line_factor<P>(S, y);
                         cls = far_class64<P>(D, hW, ia, y2, G);
                         if constexpr (P::CHI) {
                             if (cls && !chi_piece(a.chi, xfirst, xlast, nu, D, hW, chi)) cls = 0;
@@ -811,6 +967,8 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                 if (c0 + lane < total) {
                     const int64_t i = line_at(c0 + lane);
                     const double nu = a.nu[i], hw = a.hw[i];
+                    double y = 0.0, S = 0.0;
+                    if constexpr (kNodes) { ia = a.ia[i]; S = a.S[i]; y = a.y[i]; }
                     const double dl = xwf - nu, dh = xwl - nu;
                     D = xcw - nu;
                     const bool full = dl > -hw && dl < hw && dh > -hw && dh < hw;
@@ -819,10 +977,8 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
                         if (full && !(el > -hw && el < hw && eh > -hw && eh < hw)) wcst -= a.pl[i];
                     }
                     if (kNodes && full && fabs(D) >= kFarRatio64 * hw_w) {
-                        const double y = a.y[i];
-                        ia = a.ia[i];
                         y2 = y * y;
-                        G = line_factor<P>(a.S[i], y);
+                        G = line_factor<P>(S, y);
                         if constexpr (P::PLINTH) pl = a.pl[i];
                         cls = far_class64<P>(D, hw_w, ia, y2, G);
                         if constexpr (P::CHI) {
@@ -843,91 +999,9 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         // the rest point by point
         for (int c0 = 0; c0 < total; c0 += 64) {
             const int e = c0 + lane;
-            uint32_t code = 0;
-            int lo = 0, hi = 0;
-            double nu = 0.0, ia = 1.0, y = 1.0, G = 0.0, Apf = 0.0, pl = 0.0;
-            bool far = false;                    // x^2 + y^2 >= 1e6 at all points
-            if (e < total && !((kNodes || kConst) && (sh->taken[wave][c0 >> 6] >> lane) & 1ull)) {
-                const int64_t i = line_at(e);
-                nu = a.nu[i];
-                clip_window(nu, a.hw[i], a.numin, a.dnu, inv_dnu, jw, nw, lo, hi);
-                if (lo < hi) {
-                    const double S = a.S[i];
-                    y = a.y[i];
-                    ia = a.ia[i];
-                    G = line_factor<P>(S, y);
-                    if constexpr (P::PLINTH) pl = a.pl[i];
-                    if constexpr (P::PROFILE == 1) {
-                        // conservative point intervals with x^2 + y^2 < 100, 1e4
-                        const float vb = (float)(a.dnu * ia), fy2 = (float)(y * y);
-                        const float cen = (float)((nu - xwf) * inv_dnu);
-                        const float r1 = sqrtf(fmaxf(1.0002e2f - fy2, 0.0f)) / vb;
-                        const float r2 = sqrtf(fmaxf(1.0002e4f - fy2, 0.0f)) / vb;
-                        const float mg = 2.0f + 1.0e-5f * fabsf(cen);
-                        const bool in1 = fy2 < 1.0002e2f, in2 = fy2 < 1.0002e4f;
-                        if constexpr (P::WHOLE) {
-                            const float r3 = sqrtf(fmaxf(1.0002e6f - fy2, 0.0f)) / vb;
-                            far = !(fy2 < 1.0002e6f && cen - r3 - mg <= (float)(WP - 1) &&
-                                    cen + r3 + mg >= 0.0f) && fy2 < 1.0e12f;
-                        }
-#pragma unroll
-                        for (int k = 0; k < PPT; ++k) {
-                            const int s0 = 64 * k, s1 = s0 + 63;
-                            if (lo > s1 || hi <= s0) continue;
-                            const bool c3 = in1 && cen - r1 - mg <= (float)s1 && cen + r1 + mg >= (float)s0;
-                            const bool c2 = in2 && cen - r2 - mg <= (float)s1 && cen + r2 + mg >= (float)s0;
-                            code |= (c3 ? 3u : c2 ? 2u : 1u) << (2 * k);
-                        }
-                        if (code & (code >> 1) & 0x55555555u) Apf = S * kISqrtPi * core_pole(y);
-                    } else {
-                        // segments that the window touches; a compact profile's
-                        // only where it is not zero, unless a plinth is there
-                        int l = lo, h = hi;
-                        const bool part = P::PROFILE == 0 || (P::PLINTH && pl != 0.0);
-                        if (P::COMPACT && !part && fabs(S) < 1.0e300) {
-                            const double off = (nu - xwf) * inv_dnu;
-                            const double w = kDopplerEnd / ia * inv_dnu + 2.0;
-                            l = max(lo, (int)fmin(fmax(off - w, 0.0), (double)nw));
-                            h = min(hi, (int)fmin(fmax(off + w, 0.0), (double)nw));
-                        }
-                        if (P::PROFILE != 0 || part)
-#pragma unroll
-                            for (int k = 0; k < PPT; ++k)
-                                if (l < 64 * k + 64 && h > 64 * k && l < h) code |= 1u << (2 * k);
-                    }
-                }
-            }
-            unsigned long long m = __ballot(code != 0);
-            if constexpr (P::WHOLE) {
-                // lines of one formula over the wave, in a loop of its own each:
-                // merged, every line copies the sums between its paths
-                constexpr uint32_t ones = 0x55555555u & (uint32_t)((1ull << (2 * PPT)) - 1);
-                const bool whole = lo == 0 && hi == WP;
-                auto wings = [&](auto formula, bool mine) {
-                    unsigned long long w = __ballot(mine);
-                    m &= ~w;
-                    while (w) {
-                        const int b = __builtin_ctzll(w);
-                        w &= w - 1ull;
-                        add_wing<formula, PPT>(x_at, lane_f64(nu, b), lane_f64(ia, b),
-                                               lane_f64(y, b), lane_f64(G, b), acc);
-                    }
-                };
-                wings(std::integral_constant<int, 1>{}, whole && code == ones && far);
-                wings(std::integral_constant<int, 2>{}, whole && code == ones && !far);
-                wings(std::integral_constant<int, 4>{}, whole && code == 2 * ones);
-            }
-            while (m) {
-                const int b = __builtin_ctzll(m);
-                m &= m - 1ull;
-                const int slo = __builtin_amdgcn_readlane(lo, b), shi = __builtin_amdgcn_readlane(hi, b);
-                const uint32_t scode = (uint32_t)__builtin_amdgcn_readlane((int)code, b);
-                add_points<P, PPT>(a, scode,
-                                   lane_f64(nu, b), lane_f64(ia, b), lane_f64(y, b), lane_f64(G, b),
-                                   P::PROFILE == 1 ? lane_f64(Apf, b) : 0.0,
-                                   P::PLINTH ? lane_f64(pl, b) : 0.0, slo, shi,
-                                   slo == 0 && shi == nw, jd, acc, sh->tab[wave]);
-            }
+            const bool mine =
+                e < total && !((kNodes || kConst) && (sh->taken[wave][c0 >> 6] >> lane) & 1ull);
+            add_lines<PPT, P>(a, mine ? line_at(e) : -1, w, x_at, acc, sh->tab[wave]);
         }
         __syncthreads();      // the lists are free for the next round
     }
@@ -973,15 +1047,7 @@ __device__ __forceinline__ void tile_f64(const Args &a, int64_t tile, Far64LDS *
         for (int k = 0; k < PPT; ++k)
             acc[k] += cheb_sum64(c, (fma(jd + (double)(64 * k), a.dnu, a.numin) - xcw) / hw_w);
     }
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        const int64_t j = jw + lane + 64 * k;
-        if constexpr (P::CHI) {
-            const double x = fma(jd + (double)(64 * k), a.dnu, a.numin);
-            if (a.side != 0 && (x > a.lo && x < a.hi) != (a.side > 0)) continue;
-        }
-        if (j < a.nx) a.K[j] = a.accumulate ? a.K[j] + acc[k] : a.kmin + acc[k];
-    }
+    store_points<PPT, P>(a, w, x_at, acc);
 }
 
 }  // namespace hk

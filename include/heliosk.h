@@ -144,10 +144,10 @@ typedef struct {
 typedef struct {
     int tile_points;    /* grid points per workgroup tile: 512, 1024,
                            2048 or 4096; 0: 1024.  HK_VOIGT_FP64: 0 chooses
-                           by the length of the grid (in a batch, of its
-                           longest), and a width that cannot fill the chip
-                           or its registers is taken one or two steps
-                           narrower, or wider with every pair evaluated */
+                           by the points and lines (of the whole batch),
+                           and a width that cannot fill the chip or its
+                           registers is taken one or two steps narrower,
+                           or wider with every pair evaluated */
     int exact_pairs;    /* 1 evaluates every (line, point) pair; 0
                            (default) sums lines far from a tile, or from a
                            wave's quarter of it, through Chebyshev far
