@@ -169,8 +169,7 @@ __global__ __launch_bounds__(kTrDThreads) void transmission_direct_kernel(
 
 constexpr int kTrThreads = 512;
 constexpr int kTrWaves = kTrThreads / 64;
-constexpr int kTrGroups = 1;                 // groups of 16 m values per wave
-constexpr int kTrPer = kTrWaves * kTrGroups * 16;   // m values per workgroup
+constexpr int kTrPer = kTrWaves * 16;        // m values per workgroup, 16 a wave
 constexpr int kTrC = 128;                    // points per cluster
 constexpr int kTrBatch = 128;                // clusters in LDS at a time
 constexpr int kTrSuper = 16;                 // clusters per super-cluster
@@ -241,9 +240,10 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     const int tid = threadIdx.x, lane = tid & 63, part = tid & 3;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const double *Kb = Ks + (size_t)b * Nxb;
-    // this lane's m of group g: t0 + 16 (wave + 8 g) + lane / 4
-    const int t0 = blockIdx.x * kTrPer + 16 * wave + (lane >> 2);
-    auto m_of = [&](int g) { return exp((double)(t0 + 16 * kTrWaves * g - nTr / 2) * dTr); };
+    // four lanes per m; a wave past the last has none
+    const int ti = blockIdx.x * kTrPer + 16 * wave + (lane >> 2);
+    const bool any_m = blockIdx.x * kTrPer + 16 * wave < nTr;
+    const double m = exp((double)(ti - nTr / 2) * dTr);
     if (tid < 4 * kFN64) cosv[tid] = cos40(tid);
     double least = INFINITY;
     for (int k = tid; k < Nxb; k += kTrThreads) least = fmin(least, Kb[k]);
@@ -252,9 +252,7 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kTrWaves; ++w) least = fmin(least, red[w]);
-    double acc[kTrGroups];
-#pragma unroll
-    for (int g = 0; g < kTrGroups; ++g) acc[g] = 0.0;
+    double a = 0.0;
     double un[kFN64 / 4];                  // (K - lo) / half at this lane's nodes
 #pragma unroll
     for (int k = 0; k < kFN64 / 4; ++k)
@@ -344,11 +342,7 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
             if (lane == 0) sc[h] = TrCluster{lo, half, 0, ok};
         }
         __syncthreads();
-#pragma unroll
-        for (int g = 0; g < kTrGroups; ++g) {
-            if (blockIdx.x * kTrPer + 16 * (wave + kTrWaves * g) >= nTr) break;
-            const double m = m_of(g);
-            double a = acc[g];
+        if (any_m) {
             // e^{-lo m} (the product's rounding, eps lo m of the value, put
             // back) times the nodes' e^{-(K - lo) m}, argument <= 6
             auto by_nodes = [&](const TrCluster &q, const double (&w)[kFN64 / 4]) {
@@ -400,27 +394,20 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
                     }
                 }
             }
-            acc[g] = a;
         }
     }
+    if (!any_m) return;
     const double nmin = nxmin ? (double)nxmin[b] : 0.0, nb = (double)Nxb;
-#pragma unroll
-    for (int g = 0; g < kTrGroups; ++g) {
-        const int ti = t0 + 16 * kTrWaves * g;
-        if (blockIdx.x * kTrPer + 16 * (wave + kTrWaves * g) >= nTr) break;
-        const double m = m_of(g);
-        double a = acc[g];
-        if (part < 3) {                     // Simpson end weights, a term per lane
-            const double w[3] = {-5.0 / 8.0, 1.0 / 6.0, -1.0 / 24.0};
-            a = fma(part == 0 ? w[0] : part == 1 ? w[1] : w[2], tr_exp(Kb[part] * m), a);
-            a = fma(part == 0 ? w[2] : part == 1 ? w[1] : w[0], tr_exp(Kb[Nxb - 1 - part] * m), a);
-        }
-        a += __shfl_xor(a, 1, 64);
-        a += __shfl_xor(a, 2, 64);
-        if (part == 0 && ti < nTr)
-            Tr[(size_t)b * nTr + ti] =
-                a / (nb - 1.0) * (nb - nmin) / nb + exp(-kmin * m) * nmin / nb;
+    if (part < 3) {                         // Simpson end weights, a term per lane
+        const double w[3] = {-5.0 / 8.0, 1.0 / 6.0, -1.0 / 24.0};
+        a = fma(part == 0 ? w[0] : part == 1 ? w[1] : w[2], tr_exp(Kb[part] * m), a);
+        a = fma(part == 0 ? w[2] : part == 1 ? w[1] : w[0], tr_exp(Kb[Nxb - 1 - part] * m), a);
     }
+    a += __shfl_xor(a, 1, 64);
+    a += __shfl_xor(a, 2, 64);
+    if (part == 0 && ti < nTr)
+        Tr[(size_t)b * nTr + ti] =
+            a / (nb - 1.0) * (nb - nmin) / nb + exp(-kmin * m) * nmin / nb;
 }
 
 // Whether the clusters take a transmission, else every value is exponentiated.
