@@ -220,12 +220,12 @@ struct TrCluster {
 // 20 Chebyshev nodes with the values' Lagrange weights, whatever m; a cluster
 // too wide for an m is summed value by value, and one with nothing left to add
 // is skipped.  Sixteen clusters make a super-cluster, whose nodes stand for them
-// where they are narrow enough for the m.  The waves make the clusters of a batch together, then each takes
-// its m values, 16 at a time and four lanes each, without waiting for the
-// others.  A cluster's range is its values' own, so bins that are not sorted
+// where they are narrow enough for the m.  The waves make the clusters of a batch
+// together, then each takes its 16 m values, four lanes each, without waiting for
+// the others.  A cluster's range is its values' own, so bins that are not sorted
 // are summed too, more slowly.
 // Bound by FP64 vector instructions (300 bins of 1e4 points, 300 m: one
-// exponential per point and m took 724 us, this 273).
+// exponential per point and m takes 633 us, this 256).
 __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
     const double *__restrict__ Ks, int Nxb, const int32_t *__restrict__ nxmin, double kmin,
     int nTr, double dTr, double *__restrict__ Tr) {
@@ -411,15 +411,16 @@ __global__ __launch_bounds__(kTrThreads, 4) void transmission_kernel(
 }
 
 // Whether the clusters take a transmission, else every value is exponentiated.
-// Measured: the direct kernel adds 1.24e6 terms per us once it fills the chip;
-// a workgroup of the clusters, 512 of which run at once, takes 60 us and 5.5 us
-// per 1000 points, little of which others can hide.  300 bins of 1e4 points,
-// 300 m: 724 us direct, 273 clusters; 300 of 1714: 125 and 134; 10 of 9059: 25
-// and 110.
+// Measured: the direct kernel adds 1.24e6 to 1.42e6 terms per us, by the values,
+// once it fills the chip; a workgroup of the clusters, 512 of which run at once,
+// takes 60 us and 5.5 us per 1000 points, little of which others can hide; they
+// have to be a fifth faster by this.  300 bins of 1e4 points, 300 m: 633 us direct,
+// 256 clusters; 80 bins 178 and 126; 300 of 1714: 136 and 141; 10 of 9059: 37 and
+// 110.
 bool transmission_by_clusters(int nbins, int Nxb, int nTr) {
     const double direct = (double)nbins * Nxb * nTr / 1.24e6;
     const double blocks = (double)nbins * ((nTr + kTrPer - 1) / kTrPer);
-    return direct > (60.0 + 0.0055 * Nxb) * fmax(1.0, blocks / 512.0);
+    return direct > 1.2 * (60.0 + 0.0055 * Nxb) * fmax(1.0, blocks / 512.0);
 }
 
 }  // namespace
