@@ -981,9 +981,9 @@ __device__ __forceinline__ void wave_far_coeffs(const float (*s)[2], double *c, 
 }
 
 template <int PPT, int LM>
-__device__ __forceinline__ void tile_f32c(const VArgs &a, int64_t tile, Rec32 *rec, FarLDS *fl) {
+__device__ __forceinline__ void tile_f32c(const VArgs &a, int64_t tile, Rec32 *rec, FarLDS *fl,
+                                          const int t) {
     constexpr int W = kThreads * PPT;
-    const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wlo = wave * 64 * PPT;
@@ -1415,7 +1415,13 @@ __global__ __launch_bounds__(256, main_waves(MODE, PPT, LM)) void voigt_tiles_ke
     } else {
         __shared__ Rec32 rec[kThreads * LM];
         __shared__ FarLDS fl;
-        tile_f32c<PPT, LM>(a, tile, rec, &fl);
+        // (tiles of 1024 points and more: the thread index, kept, is spilled before
+        // the first branch, and empty tiles pay for it: 500 lines on 3e7 points 242
+        // us, with the lane counted anew 226)
+        const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        tile_f32c<PPT, LM>(a, tile, rec, &fl,
+                           PPT >= 4 ? 64 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + lane
+                                    : (int)threadIdx.x);
     }
 }
 
@@ -1484,7 +1490,7 @@ void voigt_persistent_kernel(const VArgs *__restrict__ specs,
             core_f32c(a, tile, (Core32 *)smem, dtab, cnt);
         } else {
             if constexpr (MODE != HK_VOIGT_FP32C) tile_f64<PPT, Sum64<MODE, PPT>>(a, tile, (Far64LDS *)smem);
-            else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl);
+            else tile_f32c<PPT, LM>(a, tile, (Rec32 *)smem, fl, threadIdx.x);
         }
     }
 }
