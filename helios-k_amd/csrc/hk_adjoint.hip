@@ -56,7 +56,12 @@ constexpr int kASubs = kATile / kASub, kASegs = kATile / kASeg;
 // 0, 20, 40 and 80 (1e6 points): 500 lines of 1000 points 137, 31, 31, 31 us,
 // 3000 of 5000 points 178, 175, 82, 82, 10000 of 5000 269, 271, 272, 210, 50000 of
 // 5000 625, 628, 625, 750; on 1e5 points 10000 of 5000 166, 167, 167, 205.
-constexpr int kDirectSteps = 40;
+// What counts is the average window, and the wave with the longest one may not end
+// far behind the others: half of those steps, and kDirectWave for what the tiles cost
+// at the least.  With 40 steps a tile for the longest instead: windows of 1 to 1e4
+// points 5000 lines 164 -> 100 us, 60000 622 -> 375; one of 1e4 points in 64, 50000
+// lines 460 -> 325; one of 1e5 points in 16, a line at a time 2119, by tiles 1607.
+constexpr int kDirectSteps = 40, kDirectWave = 200;
 
 struct IsoTabA {
     double mass[HK_MAX_ISO], ab[HK_MAX_ISO], ss[HK_MAX_ISO], Q[HK_MAX_ISO];
@@ -362,12 +367,16 @@ __global__ __launch_bounds__(kAT, 4) void adjoint_kernel(AArgs a) {
     if constexpr (kShared) {
         // windows short against the tiles they spread over: a line at a time per
         // wave, all its points, as many lines at once as the parts have waves
-        int64_t most = jhi - jlo;
-        for (int off = 32; off > 0; off >>= 1)
-            most = max(most, (int64_t)__shfl_xor((long long)most, off, 64));
+        double steps = (double)(jhi - jlo) * (1.0 / 64) + 1.0, most = steps;
+        for (int off = 32; off > 0; off >>= 1) {
+            steps += __shfl_xor(steps, off, 64);
+            most = fmax(most, __shfl_xor(most, off, 64));
+        }
         const int64_t rounds = (LPB + kWaves * a.parts - 1) / (kWaves * a.parts);
         const int64_t tiles = ((hi - lo) / kATile + a.parts) / a.parts;
-        if (lo < hi && rounds * (most / 64 + 1) <= kDirectSteps * tiles) {
+        const double allowed = (double)(kDirectSteps * tiles);
+        if (lo < hi && (double)rounds * steps <= 64.0 * allowed
+            && most <= 0.5 * allowed + kDirectWave) {
             for (int b = part * kWaves + wave; b < LPB; b += kWaves * a.parts) {
                 const int64_t l = lane_i64(jlo, b), h = lane_i64(jhi, b);
                 const double lnu = lane_f64(nu, b), lia = lane_f64(ia, b), ly = lane_f64(y, b);

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 # nx 20011: 78 tiles of 256 points in 32 parts are 3 rounds of 40 steps of 64
-# points, so a window of up to 7679 points is taken a line at a time, if the
+# points, so a window of up to 7616 points is taken a line at a time, if the
 # lines spread over the whole grid
 @pytest.mark.parametrize("nx", [20011, 8191])
 @pytest.mark.parametrize("n", [1, 65, 257])
