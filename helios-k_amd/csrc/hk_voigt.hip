@@ -29,8 +29,9 @@
 // Forms:
 //   HK_VOIGT_FP64  x = (x_j - nu)/alpha_D in FP64, FP64 profile (midpoint
 //                  rule with the pole's residue in the core, 8- and 4-node
-//                  Gauss-Hermite, 3-term asymptotic) and FP64 accumulation; lines far from a tile through 20
-//                  Chebyshev nodes, exact to FP64 rounding (hk_voigt64.h).
+//                  Gauss-Hermite, 3-term asymptotic) and FP64 accumulation;
+//                  lines far from a tile through 20 Chebyshev nodes, exact to
+//                  FP64 rounding (hk_voigt64.h).
 //   HK_VOIGT_FP32C the line offset is formed in FP64 once per line and tile
 //                  (nearest grid point jc, remainder r), then
 //                  x = (j - jc) vb + r in FP32 with vb split hi+lo; FP32

@@ -29,8 +29,8 @@
 // 100 cm^-1 a line has 2e4 pairs in its window; it takes 20 node values in
 // each of ~17 tiles, 20 in ~9 waves and ~13 segments of 64 points -- 30 times
 // fewer evaluations than pairs.  Pair by pair (with a separate line-core
-// pass) that spectrum took 2217 us, now 533; 2.35e6 lines on 7e6 points at
-// 10 bar, cut 25: 132 ms, now 15.3.
+// pass) that spectrum took 2217 us, now 497; 2.35e6 lines on 7e6 points at
+// 10 bar, cut 25: 132 ms, now 15.8.
 #pragma once
 #include <type_traits>
 
@@ -64,12 +64,12 @@ __device__ __forceinline__ double cos40(int j) {
 __device__ __forceinline__ double node_u(int k) { return cos40(2 * k + 1); }
 // Points per thread of a tile (256 threads) when the caller leaves it open.
 // Halving the tile doubles the tile-level node evaluations and halves the point
-// sums; 512 points win over 1024 at 1e5 lines, 3e6 points, cut 100 (491 against
-// 520 us), 5e6 lines (15.2 / 20.4 ms) and 3.3e5 lines, 1e6 points (0.98 / 1.34
-// ms), and cost 3 % at 2.35e6 lines, 7e6 points, cut 25 on a 0.001 cm^-1 grid.
+// sums; 512 points win over 1024 at 1e5 lines, 3e6 points, cut 100 (492 against
+// 542 us), 5e6 lines (16.4 / 20.4 ms), 3.3e5 lines, 1e6 points (1.06 / 1.40 ms) and
+// 2.35e6 lines, 7e6 points, cut 25 on a 0.001 cm^-1 grid (15.9 / 16.4 ms).
 // Grids of fewer than four 512-point tiles per CU take 256-point tiles: 1e4
-// points 73 against 106 us, 3e4 points under 1e5 lines 1.12 / 1.97 ms, 3e5
-// points 665 / 805 us; at 1e6 points the two are equal.
+// points 67 against 110 us, 1e5 lines of cut 100 on 3e4 points 1.13 / 2.34 ms, on
+// 3e5 points 430 / 468 us; at 1e6 points the two are equal.
 // With every pair evaluated, longer grids take 1024 or 2048 points, so that a
 // line's broadcast serves four or eight points a lane (tiles of 512, 1024 and 2048
 // points: 24 spectra of 3e6 points, 1e4 to 5e6 lines, 684, 559 and 535 ms; 1e5
@@ -536,7 +536,7 @@ __device__ __forceinline__ double cheb_sum64(const double *c, double u) {
 // One exponential, one cosine and 24 table reads replace the 40 reciprocals
 // and 4 exponentials of the Algorithm 916 series that a separate pass took
 // (2.35e6 lines, 7e6 points at 10 bar: that pass 31 ms, the whole sum 39.9 ms,
-// now 15.3; 1e5 lines, 3e6 points: 900 -> 533 us).
+// now 15.8; 1e5 lines, 3e6 points: 900 -> 497 us).
 // ---------------------------------------------------------------------------
 constexpr double kHC = 0.5178;
 constexpr int kCLo = 11, kCHi = 12;               // m = -kCLo .. kCHi
